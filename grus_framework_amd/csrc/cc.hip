@@ -5,14 +5,15 @@
 // frontier).  Its fixed point on a symmetric graph is the minimum vertex id
 // of each component; both methods below reach exactly that labelling.
 //
-// method 0 (default) -- hooking + pointer jumping with neighbour sampling
-//   (Sutton et al., IPDPS'18 "Afforest"): link every vertex to its first two
-//   neighbours, compress, find the most frequent root by sampling, then
-//   link the remaining edges only for vertices outside that component.  A
-//   link always hooks the larger root under the smaller one with a CAS, so
-//   parent[x] <= x holds throughout and every root is the minimum of its
-//   tree.  The giant component's edges (most of an RMAT graph) are never
-//   read after the first two per vertex.
+// method 0 (default) -- hooking + pointer jumping (after Sutton et al.,
+//   IPDPS'18 "Afforest"): hook every vertex under its first neighbour where
+//   that is smaller (one store, no atomic), compress, find the most frequent
+//   root by sampling, then link every edge of the vertices outside that
+//   component.  A link hooks the larger root under the smaller one with a
+//   CAS, so parent[x] <= x holds throughout and every root is the minimum of
+//   its tree.  Rows of generated graphs ascend, so the first neighbour is the
+//   lowest: on RMAT s20 the hooks alone put 93% of the vertices with edges
+//   into the giant component, and the rest hold 0.3% of the edges.
 // method 1 -- the reference's min-label propagation through the push
 //   operator (advance.hpp), frontier deduplicated by round stamps.
 #include <algorithm>
@@ -27,7 +28,7 @@
 namespace mgg {
 
 struct CcWork {
-  Buf q[2], stamp, sample;
+  Buf q[2], stamp, giant;
   PushWork push;
   uint64_t cap_v = 0;
   uint32_t stamp_id = 0;
@@ -42,7 +43,7 @@ __global__ void k_init(uint32_t *label, uint64_t V) {
 }
 
 __device__ __forceinline__ uint32_t ld(const uint32_t *p) {
-  return __atomic_load_n(p, __ATOMIC_RELAXED);
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // hook the larger root under the smaller (CAS); parent[x] <= x is invariant
@@ -58,46 +59,108 @@ __device__ __forceinline__ void link(uint32_t u, uint32_t v, uint32_t *parent) {
   }
 }
 
-// link neighbour number r (0-based) of every vertex that has one
-__global__ void k_link_round(CsrView g, uint32_t r, uint32_t *parent) {
+// parent[u] = u's first neighbour where that is smaller, else u.  Bound by
+// the gather of one cache line per row.
+__global__ __launch_bounds__(BLOCK) void k_hook_first(CsrView g, uint32_t *parent) {
   uint64_t u = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
   uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (; u < g.V; u += stride) {
-    uint64_t e = g.off[u] + r;
-    if (e < g.off[u + 1]) link((uint32_t)u, edge_col(g, e), parent);
+    const uint64_t e = g.off[u];
+    uint32_t p = (uint32_t)u;
+    if (e < g.off[u + 1]) p = min(p, edge_col(g, e));
+    parent[u] = p;
   }
 }
 
-__global__ void k_compress(uint32_t *parent, uint64_t V) {
+// v's root, or `stop` if it lies on the way, climbing at most `hops` steps
+// past v's parent.  v takes every ancestor it reaches as its parent, so that
+// the vertices below it skip what it has climbed: on a grid, whose hooks form
+// chains as long as its side, storing only the root made each vertex climb
+// its whole chain.  (A vertex that is not a root never becomes one, and only
+// its own thread stores its parent, so the stores race with no CAS.)
+__device__ __forceinline__ uint32_t climb(uint32_t v, uint32_t *parent, uint32_t stop,
+                                          uint32_t hops) {
+  uint32_t p = parent[v];  // cached: a stale parent is an older ancestor
+  uint32_t pp = p == stop ? p : ld(&parent[p]);
+  for (uint32_t i = 0; p != pp && i < hops; i++) {
+    __hip_atomic_store(&parent[v], pp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    p = pp;
+    pp = p == stop ? p : ld(&parent[p]);
+  }
+  return p;
+}
+
+// A full climb by every vertex at once is slow on long chains (each starts
+// before those above it have shortened theirs), so the first pass stops
+// after FIRST_HOPS and k_link_rest climbs the rest: 4096 x 4096 grid 1.19 ->
+// 0.44 ms in all; RMAT s22, where FIRST_HOPS reach every root, 0.13 either way.
+constexpr uint32_t FIRST_HOPS = 8;
+__global__ __launch_bounds__(BLOCK) void k_compress(uint32_t *parent, uint64_t V, uint32_t hops) {
   uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
   uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (; v < V; v += stride) {
-    uint32_t p = ld(&parent[v]);
-    uint32_t pp = ld(&parent[p]);
-    while (p != pp) {
-      p = pp;
-      pp = ld(&parent[p]);
-    }
-    parent[v] = p;
+  for (; v < V; v += stride) climb((uint32_t)v, parent, GRUS_NO_VERTEX, hops);
+}
+
+// The most frequent root among kSample pseudo-random vertices (ties: the
+// smaller root) to *giant, in one workgroup with a vertex per thread: each
+// thread counts the samples equal to its own, so the mode needs no sort and
+// no trip to the host.
+constexpr uint32_t kSample = 1024;
+__global__ __launch_bounds__(kSample) void k_sample_mode(uint32_t *parent, uint64_t V,
+                                                         uint64_t seed, uint32_t *giant) {
+  __shared__ uint4 s_root[kSample / 4];
+  __shared__ unsigned long long s_best[kSample / WAVE];
+  const uint32_t t = threadIdx.x;
+  const uint32_t mine =
+      climb((uint32_t)(mix64(seed + t) % V), parent, GRUS_NO_VERTEX, 0xFFFFFFFFu);
+  reinterpret_cast<uint32_t *>(s_root)[t] = mine;
+  __syncthreads();
+  uint32_t n = 0;
+  for (uint32_t i = 0; i < kSample / 4; i++) {
+    const uint4 x = s_root[i];
+    n += (x.x == mine) + (x.y == mine) + (x.z == mine) + (x.w == mine);
+  }
+  unsigned long long best = ((unsigned long long)n << 32) | (0xFFFFFFFFu - mine);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const unsigned long long y = __shfl_xor(best, o);
+    best = y > best ? y : best;
+  }
+  if (lane_id() == 0) s_best[t / WAVE] = best;
+  __syncthreads();
+  if (t == 0) {
+    for (uint32_t w = 1; w < kSample / WAVE; w++) best = s_best[w] > best ? s_best[w] : best;
+    *giant = 0xFFFFFFFFu - (uint32_t)best;
   }
 }
 
-__global__ void k_sample(const uint32_t *parent, uint64_t V, uint32_t n, uint64_t seed,
-                         uint32_t *out) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = parent[mix64(seed + i) % V];
-}
-
-// wave per vertex outside the giant component: link edges from number `from` on
-__global__ __launch_bounds__(BLOCK) void k_link_rest(CsrView g, uint32_t from, uint32_t giant,
+// Every edge of the vertices outside the giant component.  A lane tests one
+// vertex and links its row itself up to REST_LANE edges; the wave shares
+// longer rows.  Nearly every vertex fails the test, so this costs one
+// coalesced read of the parents: RMAT s22 spent 325 of 503 us here with a
+// wave per vertex; the whole call now takes 126 us on the device.
+constexpr uint64_t REST_LANE = 16;
+__global__ __launch_bounds__(BLOCK) void k_link_rest(CsrView g, const uint32_t *giant_p,
                                                      uint32_t *parent) {
-  uint64_t wave = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) / WAVE;
-  uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
-  for (uint64_t u = wave; u < g.V; u += nwaves) {
-    if (ld(&parent[u]) == giant) continue;
-    uint64_t end = g.off[u + 1];
-    for (uint64_t e = g.off[u] + from + lane_id(); e < end; e += WAVE)
-      link((uint32_t)u, edge_col(g, e), parent);
+  const uint32_t giant = *giant_p;
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  const uint64_t first = blockIdx.x * (uint64_t)blockDim.x + (threadIdx.x & ~(uint32_t)(WAVE - 1));
+  for (uint64_t base = first; base < g.V; base += stride) {  // wave-uniform
+    const uint64_t u = base + lane_id();
+    uint64_t beg = 0, end = 0;
+    if (u < g.V && climb((uint32_t)u, parent, giant, 0xFFFFFFFFu) != giant) {
+      beg = g.off[u];
+      end = g.off[u + 1];
+    }
+    const bool shared_row = end - beg > REST_LANE;
+    if (!shared_row)
+      for (uint64_t e = beg; e < end; e++) link((uint32_t)u, edge_col(g, e), parent);
+    for (uint64_t m = __ballot(shared_row); m; m &= m - 1) {
+      const int l = __ffsll((unsigned long long)m) - 1;
+      const uint64_t b = __shfl(beg, l), x = __shfl(end, l);
+      for (uint64_t e = b + lane_id(); e < x; e += WAVE)
+        link((uint32_t)(base + l), edge_col(g, e), parent);
+    }
   }
 }
 
@@ -135,7 +198,7 @@ struct job_t {
 
 // The device buffers of one CC run beyond the graph and the labels.
 struct CcSpace {
-  uint32_t *sample = nullptr;           // method 0: kSample roots
+  uint32_t *giant = nullptr;            // method 0: root of the giant component
   uint32_t *q[2] = {nullptr, nullptr};  // method 1: frontier queues, V + 1 each
   uint32_t *stamp = nullptr;            // method 1: round stamps, V + 1
   uint32_t *stamp_id = nullptr;         // method 1: last stamp handed out (host)
@@ -143,8 +206,7 @@ struct CcSpace {
 };
 
 namespace {
-constexpr uint32_t kSample = 1024;  // roots sampled to find the giant component
-static_assert(kSample * 4 <= 4096, "the sample is read back through the pinned control block");
+constexpr uint64_t kGiantBytes = 256;
 
 void cc_core(Graph &g, int method, uint32_t *label, CcSpace &sp, grus_stats *st) {
   Context &ctx = *g.ctx;
@@ -153,46 +215,29 @@ void cc_core(Graph &g, int method, uint32_t *label, CcSpace &sp, grus_stats *st)
   uint64_t launches = 0;
   uint32_t iterations = 0;
   GRUS_HIP(hipEventRecord(ctx.ev0, ctx.stream));
-  cc::k_init<<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(label, V);
-  GRUS_LAUNCH_CHECK();
-  launches++;
   if (method == 0) {
-    const uint32_t kRounds = 2;
-    for (uint32_t r = 0; r < kRounds; r++) {
-      cc::k_link_round<<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(gr, r, label);
+    const unsigned grid = grid_cap(ctx, V, BLOCK);
+    if (V) {
+      cc::k_hook_first<<<grid, BLOCK, 0, ctx.stream>>>(gr, label);
       GRUS_LAUNCH_CHECK();
-      cc::k_compress<<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(label, V);
+      cc::k_compress<<<grid, BLOCK, 0, ctx.stream>>>(label, V, cc::FIRST_HOPS);
       GRUS_LAUNCH_CHECK();
-      launches += 2;
+      cc::k_sample_mode<<<1, cc::kSample, 0, ctx.stream>>>(label, V, 0x5EEDull, sp.giant);
+      GRUS_LAUNCH_CHECK();
+      cc::k_link_rest<<<grid, BLOCK, 0, ctx.stream>>>(gr, sp.giant, label);
+      GRUS_LAUNCH_CHECK();
+      cc::k_compress<<<grid, BLOCK, 0, ctx.stream>>>(label, V, 0xFFFFFFFFu);
+      GRUS_LAUNCH_CHECK();
+      launches += 5;
     }
-    // most frequent root among kSample pseudo-random vertices (ties: the
-    // smaller root), read back through the pinned control block
-    cc::k_sample<<<div_up(kSample, BLOCK), BLOCK, 0, ctx.stream>>>(label, V, kSample, 0x5EEDull,
-                                                                  sp.sample);
-    GRUS_LAUNCH_CHECK();
-    GRUS_HIP(hipMemcpyAsync(ctx.h_ctl, sp.sample, kSample * 4, hipMemcpyDeviceToHost, ctx.stream));
-    ctx.sync();
-    uint32_t hs[kSample];
-    memcpy(hs, ctx.h_ctl, sizeof hs);
-    std::sort(hs, hs + kSample);
-    uint32_t giant = hs[0], best = 0;
-    for (uint32_t i = 0; i < kSample;) {
-      uint32_t j = i;
-      while (j < kSample && hs[j] == hs[i]) j++;
-      if (j - i > best) best = j - i, giant = hs[i];  // ascending: ties keep the smaller
-      i = j;
-    }
-    cc::k_link_rest<<<grid_cap(ctx, V * WAVE, BLOCK, 8), BLOCK, 0, ctx.stream>>>(gr, kRounds,
-                                                                               giant, label);
-    GRUS_LAUNCH_CHECK();
-    cc::k_compress<<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(label, V);
-    GRUS_LAUNCH_CHECK();
-    launches += 3;
-    iterations = kRounds + 1;
+    iterations = 2;  // the hooks, then the rest
   } else {
     auto *cnt = reinterpret_cast<StepCounters *>(ctx.d_ctl.p);
     const StepCounters *hc = reinterpret_cast<const StepCounters *>(ctx.h_ctl);
     uint32_t &stamp_id = *sp.stamp_id;
+    cc::k_init<<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(label, V);
+    GRUS_LAUNCH_CHECK();
+    launches++;
     cc::k_iota<<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(sp.q[0], V);
     GRUS_LAUNCH_CHECK();
     uint64_t nf = V, mf = g.E;
@@ -247,8 +292,8 @@ void run_cc(Graph &g, int method, grus_stats *st) {
   g.result.ensure(V * 4);
   CcSpace sp;
   if (method == 0) {
-    w.sample.ensure(kSample * 4);
-    sp.sample = w.sample.as<uint32_t>();
+    w.giant.ensure(kGiantBytes);
+    sp.giant = w.giant.as<uint32_t>();
   } else {
     if (w.cap_v < V) {
       w.q[0].alloc((V + 1) * 4);
@@ -269,7 +314,7 @@ void run_cc(Graph &g, int method, grus_stats *st) {
 }
 
 uint64_t cc_scratch_bytes(Context &ctx, uint64_t V, int method) {
-  if (method == 0) return kSample * 4;
+  if (method == 0) return kGiantBytes;
   // queues and stamps (3 x (V + 1) u32), degree and scan (2 x (V + 2) u64),
   // the scan's temporaries, each start aligned to 256 bytes
   auto up = [](uint64_t x) { return (x + 255) & ~255ull; };
@@ -293,7 +338,7 @@ void run_cc_in(Graph &g, int method, uint32_t *label, void *scratch, uint64_t sc
   PushWork push;  // borrowed buffers only: its own Bufs stay empty
   uint32_t stamp_id = 0;
   if (method == 0) {
-    sp.sample = reinterpret_cast<uint32_t *>(base);
+    sp.giant = reinterpret_cast<uint32_t *>(base);
   } else {
     uint64_t at = 0;
     auto take = [&](uint64_t bytes) {
