@@ -13,7 +13,8 @@
 // graphs).  Dangling mass is dropped, as in the reference.
 //
 // Layouts (grus_tuning::pr_layout): the binned push (4, automatic on HBM
-// graphs that fit it), the plain pull (2, everything else), propagation
+// graphs that fit it, but for the smallest, which pull into the same exact
+// sums), the plain pull (2, everything else), propagation
 // blocking over the pull (3) and a degree-sorted relabelled pull (1).
 //
 // Binned push (pr_layout = 4; build_binned, k_bp_scatter, k_bp_accum):
@@ -25,6 +26,11 @@
 // the ranks are bit-identical run to run and whatever the bin width or task
 // split, and closer to the FP64 oracle than an FP32 sum.  Every global
 // access is a sequential stream; the random accesses hit LDS.
+//
+// Exact pull (HBM graphs of at most PX_MAX_V vertices and PX_MAX_E edges when
+// the layout is automatic; k_pull_exact): the plain pull's windows with the
+// binned layout's fixed-point sums, one launch per iteration and nothing to
+// build beyond the window table.
 //
 // Plain pull (SpMV over the in-edge CSR): the edge array is cut into windows of
 // WIN edges, one per workgroup, WIN_EPT consecutive edges per thread.
@@ -62,6 +68,14 @@
 namespace mgg {
 
 constexpr int PB_BITS = 14;   // blocked layout: 16K destinations per bin
+// Exact pull: edges per thread (4 measured 7.3 us an iteration on RMAT s12, 8
+// measured 9.2), and the largest graphs that take it.  It gathers contrib
+// per edge, so it wants contrib in an XCD's 4 MB L2 (V <= 2^20), and its time
+// grows with E where the binned layout's starts at 20-70 us (us per iteration
+// exact / binned, the latter with 2^14-vertex bins: RMAT s12 7 / 25, s16 15 /
+// 65, s18 (7.6 M edges) 41 / 69, s19 79 / 80, s20 156 / 82).
+constexpr int PX_EPT = 4;
+constexpr uint64_t PX_MAX_V = 1ull << 20, PX_MAX_E = 1ull << 23;
 
 struct PrWork {
   Buf contrib[2], win_row, head_sum, tail_sum;
@@ -101,22 +115,28 @@ struct PrWork {
   int bp_w2_bytes = 4;  // 1, 2 or 4: the narrowest that holds the largest weight
   const void *bp_w2_for = nullptr;
   const void *bp_unusable_for = nullptr;  // offsets a failed build was tried on
+  // exact pull: window table, the sums and arrival counts of the rows that
+  // span windows (zero between iterations), and the two contrib arrays
+  Buf px_win_row, px_sums, px_arrived, px_contrib[2];
+  uint64_t px_nwin = 0;
+  const void *px_for = nullptr;  // in-edge offsets they were built on
 };
 
-__global__ void k_window_rows(const uint64_t *off, uint64_t V, uint64_t nwin, uint32_t *win_row) {
+__global__ void k_window_rows(const uint64_t *off, uint64_t V, uint64_t nwin, uint32_t *win_row,
+                              uint32_t win) {
   uint64_t r = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
   uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (; r <= V; r += stride) {
     // rows are owned by the window of their start offset; row V is a sentinel
-    int64_t kprev = (r == 0) ? -1 : (int64_t)(off[r - 1] / WIN);
-    int64_t kcur = (r == V) ? (int64_t)nwin : (int64_t)(off[r] / WIN);
+    int64_t kprev = (r == 0) ? -1 : (int64_t)(off[r - 1] / win);
+    int64_t kcur = (r == V) ? (int64_t)nwin : (int64_t)(off[r] / win);
     for (int64_t k = kprev + 1; k <= kcur; k++) win_row[k] = (uint32_t)r;
   }
 }
 
 void build_window_rows(Context &ctx, const uint64_t *off, uint64_t V, uint64_t nwin,
-                       uint32_t *win_row) {
-  k_window_rows<<<grid_cap(ctx, V + 1, BLOCK), BLOCK, 0, ctx.stream>>>(off, V, nwin, win_row);
+                       uint32_t *win_row, uint32_t win) {
+  k_window_rows<<<grid_cap(ctx, V + 1, BLOCK), BLOCK, 0, ctx.stream>>>(off, V, nwin, win_row, win);
   GRUS_LAUNCH_CHECK();
 }
 
@@ -1023,7 +1043,7 @@ template <bool kLast>
 __global__ __launch_bounds__(BLOCK) void k_pull_window(CsrView in, const uint32_t *win_row,
                                                        PrOp<kLast> op, uint64_t nwin,
                                                        bool xcd_order) {
-  __shared__ WindowShared sh;
+  __shared__ WindowShared<> sh;
   // blocked layout: consecutive windows gather from the same bin, so they
   // are kept on one XCD (its L2); the plain pull gathers from anywhere and
   // runs slightly faster in dispatch order
@@ -1037,6 +1057,63 @@ __global__ void k_fixup(CsrView in, const uint32_t *win_row, PrOp<kLast> op, uin
   uint64_t k = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
   if (k >= nwin) return;
   window_fixup(in, win_row, k, op);
+}
+
+// The exact pull of small graphs: a window reduction whose partial sums are
+// the binned layout's 64-bit fixed point, so the ranks are bit for bit those
+// of the binned layout, in one launch per iteration.  Bound by the latency of
+// that launch (columns, contributions, the row scan, the division) up to
+// about 10^5 edges, then by the gathers.  A row that spans
+// windows adds its pieces to sums[row]; the piece that arrives last takes
+// the total (leaving zeros for the next iteration) and finishes the row.
+// What crosses workgroups there moves in device-scope atomics only, each
+// waited for before the next (s_waitcnt), so no fence is needed.
+template <bool kLast>
+struct PrExactOp {
+  using T = unsigned long long;
+  const uint64_t *in_off;
+  const uint32_t *win_row;
+  const float *contrib;
+  float *next;
+  const uint64_t *out_off;
+  float base, alpha;
+  unsigned long long *sums;
+  uint32_t *arrived;
+  static constexpr uint64_t W = PX_EPT * BLOCK;
+  __device__ T identity() const { return 0ull; }
+  __device__ T combine(T a, T b) const { return a + b; }
+  __device__ T value(uint64_t, uint32_t c) const { return to_fixed(contrib[c]); }
+  __device__ void finish(uint32_t r, T s) const {
+    pr::finish<kLast>(r, from_fixed(s), out_off, next, base, alpha);
+  }
+  __device__ void empty(uint32_t r) const { finish(r, 0ull); }
+  __device__ void piece(uint32_t r, T s) const {
+    const uint32_t n = (uint32_t)((in_off[r + 1] - 1) / W - in_off[r] / W + 1);
+    (void)__hip_atomic_fetch_add(&sums[r], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_waitcnt(0);
+    if (__hip_atomic_fetch_add(&arrived[r], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) !=
+        n - 1u)
+      return;
+    __builtin_amdgcn_s_waitcnt(0);
+    const T total = __hip_atomic_exchange(&sums[r], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&arrived[r], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    finish(r, total);
+  }
+  // the row that entered window k, if any: the last one to begin before it
+  __device__ void head(uint64_t k, T s) const {
+    const uint32_t r = win_row[k];
+    if (r && in_off[r] > k * W) piece(r - 1, s);
+  }
+  __device__ void tail(uint64_t k, T s) const { piece(win_row[k + 1] - 1, s); }
+};
+
+template <bool kLast>
+__global__ __launch_bounds__(BLOCK) void k_pull_exact(CsrView in, const uint32_t *win_row,
+                                                      PrExactOp<kLast> op, uint64_t nwin) {
+  __shared__ WindowShared<PX_EPT> sh;
+  const uint64_t k = blockIdx.x;
+  if (k >= nwin) return;
+  window_reduce<PX_EPT>(in, win_row, k, op, sh);
 }
 
 }  // namespace pr
@@ -1470,6 +1547,70 @@ void run_binned(Graph &g, PrWork &w, float alpha, int iters, grus_stats *st) {
     st->kernel_launches = launches;
   }
 }
+
+// iterations of the exact pull
+void run_exact_pull(Graph &g, PrWork &w, float alpha, int iters, grus_stats *st) {
+  Context &ctx = *g.ctx;
+  const uint64_t V = g.V;
+  const CsrView out = g.csr(), in = g.csc();
+  constexpr uint32_t win = PX_EPT * BLOCK;
+  if (w.px_for != in.off) {
+    w.px_for = nullptr;
+    w.px_nwin = in.E / win + 1;
+    w.px_win_row.alloc((w.px_nwin + 1) * 4);
+    w.px_sums.alloc(V * 8);
+    w.px_arrived.alloc(V * 4);
+    for (Buf &b : w.px_contrib) b.alloc(V * 4);
+    fill_u64(ctx, w.px_sums.as<uint64_t>(), V, 0);
+    fill_u32(ctx, w.px_arrived.as<uint32_t>(), V, 0);
+    build_window_rows(ctx, in.off, V, w.px_nwin, w.px_win_row.as<uint32_t>(), win);
+    w.px_for = in.off;
+  }
+  g.result.ensure(V * 4);
+  float *rank = g.result.as<float>();
+  const float base = (float)((1.0 - (double)alpha) / (double)V);
+  const unsigned nwin = (unsigned)w.px_nwin;
+  const uint32_t *rows = w.px_win_row.as<uint32_t>();
+  auto *sums = w.px_sums.as<unsigned long long>();
+  uint32_t *arrived = w.px_arrived.as<uint32_t>();
+  GRUS_HIP(hipEventRecord(ctx.ev0, ctx.stream));
+  pr::k_init_contrib<<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(
+      out.off, V, base, w.px_contrib[0].as<float>());
+  GRUS_LAUNCH_CHECK();
+  uint64_t launches = 1;
+  if (iters == 0) {  // r0 = (1-a)/V everywhere
+    uint32_t b;
+    memcpy(&b, &base, 4);
+    fill_u32(ctx, reinterpret_cast<uint32_t *>(rank), V, b);
+    launches++;
+  }
+  for (int it = 0; it < iters; it++) {
+    const float *c = w.px_contrib[it & 1].as<float>();
+    float *next = w.px_contrib[(it + 1) & 1].as<float>();
+    if (it == iters - 1) {
+      const pr::PrExactOp<true> op{in.off, rows, c, rank, out.off, base, alpha, sums, arrived};
+      pr::k_pull_exact<true><<<nwin, BLOCK, 0, ctx.stream>>>(in, rows, op, w.px_nwin);
+    } else {
+      const pr::PrExactOp<false> op{in.off, rows, c, next, out.off, base, alpha, sums, arrived};
+      pr::k_pull_exact<false><<<nwin, BLOCK, 0, ctx.stream>>>(in, rows, op, w.px_nwin);
+    }
+    GRUS_LAUNCH_CHECK();
+    launches++;
+  }
+  GRUS_HIP(hipEventRecord(ctx.ev1, ctx.stream));
+  GRUS_HIP(hipEventSynchronize(ctx.ev1));
+  float ms = 0;
+  GRUS_HIP(hipEventElapsedTime(&ms, ctx.ev0, ctx.ev1));
+  if (st) {
+    *st = grus_stats{};
+    st->device_ms = ms;
+    st->iterations = (uint32_t)iters;
+    st->vertices_reached = V;
+    st->edges_reached = g.E;
+    st->kernel_launches = launches;
+  }
+}
+
 // the weight stream of the binned layout (for SSSP pull rounds): the CSR
 // weights sorted stably by destination bin, as d2 was, so w2 lines up with
 // d2 entry by entry
@@ -1616,6 +1757,12 @@ void run_pagerank(Graph &g, float alpha, int iters, grus_stats *st) {
   const int bits = ctx.tuning.pr_bin_bits ? (int)ctx.tuning.pr_bin_bits : PB_BITS;
   if (layout > 4 || bits < 6 || bits > 24) raise(GRUS_E_INVALID, "PageRank layout tuning");
   CsrView out = g.csr();
+  // small graphs: the binned layout's sums without its streams
+  if (layout == 0 && !ctx.tuning.pr_bin_bits && !ctx.tuning.pr_task_edges &&
+      g.placement == GRUS_PLACE_HBM && V <= PX_MAX_V && g.E <= PX_MAX_E) {
+    run_exact_pull(g, w, alpha, iters, st);
+    return;
+  }
   // binned push (automatic choice on HBM graphs that fit it; bins of at
   // most 2^14 destinations, the LDS accumulators)
   if ((layout == 0 || layout == 4) && g.placement == GRUS_PLACE_HBM) {

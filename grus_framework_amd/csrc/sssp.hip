@@ -166,7 +166,7 @@ struct PullMinOp {
 
 __global__ __launch_bounds__(BLOCK) void k_pull_min_window(CsrView in, const uint32_t *win_row,
                                                            PullMinOp op, uint64_t nwin) {
-  __shared__ WindowShared sh;
+  __shared__ WindowShared<> sh;
   // a window finishes at most one row per edge (plus none for empty rows)
   __shared__ uint32_t s_near[WIN + 2], s_far[WIN + 2];
   __shared__ uint32_t s_nn, s_nf, s_bn, s_bf;

@@ -25,6 +25,10 @@
 // order of every reduction is fixed, so results are bit-identical run to
 // run even for floating point.
 //
+// The edges per thread are a parameter (a multiple of 4, WIN_EPT unless
+// given): fewer make more and shorter windows, which a small graph needs to
+// fill the chip.
+//
 // An Op provides: type T; identity(); combine(a, b); value(edge, column);
 // finish(row, total); empty(row); head(k, t) / tail(k, t) and head_at(k) /
 // tail_at(k).
@@ -37,57 +41,60 @@ namespace mgg {
 constexpr int WIN_EPT = 8;              // edges per thread
 constexpr int WIN = WIN_EPT * BLOCK;    // edges per window
 
-// win_row[k] = first row r with off[r] >= k*WIN (V if none), k in [0, nwin]
+// win_row[k] = first row r with off[r] >= k*win (V if none), k in [0, nwin]
 void build_window_rows(Context &ctx, const uint64_t *off, uint64_t V, uint64_t nwin,
-                       uint32_t *win_row);
+                       uint32_t *win_row, uint32_t win = WIN);
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // LDS the window reduction needs (kept out of the template so that callers
 // can add their own shared arrays)
+template <int EPT = WIN_EPT>
 struct WindowShared {
-  uint32_t start[WIN + 2];  // segment starts relative to the window's first edge
-  uint32_t row[WIN + 2];    // row of segment j >= 1
+  uint32_t start[EPT * BLOCK + 2];  // segment starts relative to the window's first edge
+  uint32_t row[EPT * BLOCK + 2];    // row of segment j >= 1
   uint32_t cnt[BLOCK / WAVE];
   uint32_t wkey[BLOCK / WAVE];
   uint64_t wsum[BLOCK / WAVE];  // holds an Op::T of at most 8 bytes
 };
 
-template <class Op>
+template <int EPT = WIN_EPT, class Op>
 __device__ __forceinline__ void window_reduce(const CsrView &in, const uint32_t *win_row,
-                                              uint64_t k, Op &op, WindowShared &sh) {
+                                              uint64_t k, Op &op, WindowShared<EPT> &sh) {
   using T = typename Op::T;
+  static_assert(EPT % 4 == 0, "columns are loaded four at a time");
+  constexpr int WINE = EPT * BLOCK;
   static_assert(sizeof(T) <= sizeof(uint64_t), "partials are staged in 8-byte slots");
   constexpr int NW = BLOCK / WAVE;
   constexpr uint32_t NONE = 0xFFFFFFFFu;
-  const uint64_t e0 = k * WIN;
-  const uint64_t e1 = e0 + WIN < in.E ? e0 + WIN : in.E;
+  const uint64_t e0 = k * WINE;
+  const uint64_t e1 = e0 + WINE < in.E ? e0 + WINE : in.E;
   const uint32_t len = (uint32_t)(e1 - e0);
   const uint32_t tid = threadIdx.x, lane = lane_id(), wid = tid / WAVE;
-  const uint32_t p0 = tid * WIN_EPT;
+  const uint32_t p0 = tid * EPT;
 
   // 1. per-edge values
-  T v[WIN_EPT];
+  T v[EPT];
   {
     const uint64_t g0 = e0 + p0;
-    // a thread's WIN_EPT columns lie wholly on one side of the HBM / host
-    // split (a multiple of 64) and are 32-byte aligned on either side
-    if (p0 + WIN_EPT <= len) {
+    // a thread's EPT columns lie wholly on one side of the HBM / host
+    // split (a multiple of 64) and are 16-byte aligned on either side
+    if (p0 + EPT <= len) {
       const u32x4 *cp = reinterpret_cast<const u32x4 *>(
           g0 < in.split ? in.col + g0 : in.col_far + (g0 - in.split));
-      const u32x4 c0 = __builtin_nontemporal_load(cp);
-      const u32x4 c1 = __builtin_nontemporal_load(cp + 1);
-      v[0] = op.value(g0 + 0, c0.x);
-      v[1] = op.value(g0 + 1, c0.y);
-      v[2] = op.value(g0 + 2, c0.z);
-      v[3] = op.value(g0 + 3, c0.w);
-      v[4] = op.value(g0 + 4, c1.x);
-      v[5] = op.value(g0 + 5, c1.y);
-      v[6] = op.value(g0 + 6, c1.z);
-      v[7] = op.value(g0 + 7, c1.w);
+      u32x4 c[EPT / 4];
+#pragma unroll
+      for (int i = 0; i < EPT / 4; i++) c[i] = __builtin_nontemporal_load(cp + i);
+#pragma unroll
+      for (int i = 0; i < EPT / 4; i++) {
+        v[4 * i + 0] = op.value(g0 + 4 * i + 0, c[i].x);
+        v[4 * i + 1] = op.value(g0 + 4 * i + 1, c[i].y);
+        v[4 * i + 2] = op.value(g0 + 4 * i + 2, c[i].z);
+        v[4 * i + 3] = op.value(g0 + 4 * i + 3, c[i].w);
+      }
     } else {
 #pragma unroll
-      for (int q = 0; q < WIN_EPT; q++) {
+      for (int q = 0; q < EPT; q++) {
         v[q] = op.identity();
         if (p0 + q < len) v[q] = op.value(g0 + q, edge_col(in, g0 + q));
       }
@@ -149,7 +156,7 @@ __device__ __forceinline__ void window_reduce(const CsrView &in, const uint32_t 
     bool first = true;
     T sum = op.identity();
 #pragma unroll
-    for (int q = 0; q < WIN_EPT; q++) {
+    for (int q = 0; q < EPT; q++) {
       const uint32_t p = p0 + q;
       if (p < len) {
         while (p >= end) {  // segment j closes before edge p
@@ -215,7 +222,7 @@ __device__ __forceinline__ void window_reduce(const CsrView &in, const uint32_t 
   }
   // the window's last segment is closed (or left open) by the thread of the
   // last edge
-  if (len - p0 <= WIN_EPT) {
+  if (len - p0 <= EPT) {
     if (key == 0) {
       op.head(k, S);
     } else {

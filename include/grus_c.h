@@ -109,7 +109,10 @@ typedef struct grus_tuning {
                              which run one persistent launch, x max(2, 80 /
                              mean degree); unweighted graphs: one bucket) */
   uint32_t pr_layout;     /* PageRank edge layout: 0 automatic (= 4 where it
-                             applies, else 2); 1 degree-sorted relabelled copy
+                             applies, else 2; HBM graphs of at most 2^20
+                             vertices and 2^23 edges pull into 4's sums
+                             instead, with the same ranks, unless pr_bin_bits
+                             or pr_task_edges is set); 1 degree-sorted relabelled copy
                              (symmetric HBM graphs); 2 plain pull over the
                              in-edges; 3 blocked (propagation blocking over
                              bins of 2^pr_bin_bits destinations; HBM graphs
