@@ -34,6 +34,7 @@
 
 #include "advance.hpp"
 #include "apps.hpp"
+#include "bfs_thin.hpp"
 
 namespace mgg {
 
@@ -44,6 +45,11 @@ struct BfsWork {
   Buf cand;  // sparse bottom-up step: the unvisited vertices
   Buf first_in;                     // first in-neighbour of every vertex (GRUS_NO_VERTEX if none)
   const void *first_for = nullptr;  // in-edge columns first_in was built from
+  Buf pad;                          // thin levels: padded rows of a low-degree graph
+  uint32_t pad_deg = 0;             // columns per padded row
+  const void *pad_for = nullptr;    // out-edge columns they were built from
+  Buf thin_flags;                   // their grid barrier's flags
+  uint32_t thin_tag = 0;            // level tags handed out so far
   PushWork push;
   uint64_t cap_v = 0;
   // two-stage steps: two staging buffers of frontier rows, the stream that
@@ -541,6 +547,52 @@ __global__ __launch_bounds__(BLOCK) void k_pull_long(CsrView in, const uint64_t 
 
 }  // namespace bfs
 
+namespace {
+// Thin levels (bfs_thin.hpp): frontier sizes at which one workgroup takes
+// over and gives up, and the same for the cooperative grid.  A level of one
+// workgroup takes 1.6-2.2 us up to 300 vertices and 7 us at 1300, where one
+// CU's memory pipeline is what bounds it; a level of the grid takes 3.1 us at
+// 1000 and 4.2 us at 6000 (32 workgroups; 16 and 64 measured 3.0 and 3.2, 5.6
+// and 4.1).  Past GRID_HI a level is launched from the host, edge-balanced.
+constexpr uint32_t SOLO_IN = 512, SOLO_HI = 768;
+constexpr uint32_t GRID_LO = 256, GRID_HI = 16384;
+constexpr int THIN_T = 256, SOLO_T = 1024;
+constexpr unsigned THIN_BLOCKS = 32;
+constexpr uint64_t THIN_DEG = 16;  // largest maximum degree whose rows are padded
+
+// the padded rows of g, built on first use; null where thin levels do not
+// apply (long rows, edges outside HBM, or a device budget, which the
+// workspace reserve does not count them in)
+const uint4 *thin_rows(Graph &g, BfsWork &w) {
+  Context &ctx = *g.ctx;
+  if (g.max_deg == 0 || g.max_deg > THIN_DEG || g.placement != GRUS_PLACE_HBM ||
+      devmem_budget(ctx.device))
+    return nullptr;
+  const CsrView out = g.csr();
+  if (w.pad_for != out.col) {
+    const uint32_t D = g.max_deg <= 4 ? 4 : g.max_deg <= 8 ? 8 : 16;
+    w.pad.alloc(g.V * D * 4);
+    bfs::k_pad_cols<<<grid_cap(ctx, g.V * D, BLOCK), BLOCK, 0, ctx.stream>>>(out, D,
+                                                                           w.pad.as<uint32_t>());
+    GRUS_LAUNCH_CHECK();
+    w.pad_deg = D;
+    w.pad_for = out.col;
+  }
+  return w.pad.as<const uint4>();
+}
+
+// workgroups of the cooperative thin kernel (0: it may not run here: under a
+// CU mask or beside other contexts its grid might not be resident)
+unsigned thin_grid(const Context &ctx) {
+  if (ctx.cu_masked || ctx.shared_device) return 0;
+  int per_cu = 0;
+  GRUS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+      &per_cu, reinterpret_cast<const void *>(bfs::k_thin<THIN_T, false>),
+      bfs::thin_threads(THIN_T, false), 0));
+  return std::min({THIN_BLOCKS, bfs::THIN_MAX_G, (unsigned)std::max(0, per_cu * ctx.cu_count)});
+}
+}  // namespace
+
 void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
   Context &ctx = *g.ctx;
   ctx.activate();
@@ -605,6 +657,8 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
   // instead of every bitmap word; the host knows how many are left from
   // the vertices reached so far and the in-degree-0 count
   const uint64_t n_unreach = unreach ? g.unreachable_count : 0;
+  const uint4 *thin = dir == GRUS_DIR_PULL ? nullptr : thin_rows(g, w);
+  const unsigned thin_blocks = thin ? thin_grid(ctx) : 0;
   // GRUS_TRACE=1 prints one line per level (mode, frontier, host time)
   static const bool trace = getenv("GRUS_TRACE") != nullptr;
   auto t_level = std::chrono::steady_clock::now();
@@ -659,6 +713,71 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
                         &cnt->long_count);  // scratch counter, re-zeroed below
         GRUS_HIP(hipMemsetAsync(cnt, 0, sizeof(StepCounters), ctx.stream));
         launches += 1;
+      }
+      const bool solo = nf <= (thin_blocks ? SOLO_IN : SOLO_HI);
+      if (thin && (solo || (thin_blocks && nf <= GRID_HI))) {
+        auto *tc = reinterpret_cast<bfs::ThinCtl *>(ctx.d_ctl.as<uint64_t>() + 8);
+        bfs::ThinParams p{};
+        p.pad = thin;
+        p.pad_q = w.pad_deg / 4;
+        p.off = out.off;
+        p.q0 = w.q[0].as<uint32_t>();
+        p.q1 = w.q[1].as<uint32_t>();
+        p.cur = (uint32_t)cur;
+        p.nf = (uint32_t)nf;
+        p.lo = solo ? 1 : GRID_LO;
+        p.hi = solo ? SOLO_HI : GRID_HI;
+        p.max_levels = 1u << 20;
+        p.level = level;
+        if (!w.thin_flags.p || w.thin_tag > (1u << 24) - 2 * p.max_levels) {
+          w.thin_flags.ensure(2 * bfs::THIN_MAX_G * 8);
+          fill_u64(ctx, w.thin_flags.as<uint64_t>(), 2 * bfs::THIN_MAX_G, 0);
+          w.thin_tag = 0;
+        }
+        p.tag = w.thin_tag + 1;
+        p.flags = w.thin_flags.as<unsigned long long>();
+        p.label = label;
+        p.visited = w.visited.as<uint64_t>();
+        p.ctl = tc;
+        p.timeout = ctx.wall_ticks_per_ms() * 20000;  // 20 s per barrier wait
+        if (solo) {
+          bfs::k_thin<SOLO_T, true><<<1, SOLO_T, 0, ctx.stream>>>(p);
+          GRUS_LAUNCH_CHECK();
+        } else {
+          void *args[] = {&p};
+          GRUS_HIP(hipLaunchCooperativeKernel(
+              reinterpret_cast<const void *>(bfs::k_thin<THIN_T, false>), dim3(thin_blocks),
+              dim3(bfs::thin_threads(THIN_T, false)), args, 0, ctx.stream));
+        }
+        launches++;
+        ctx.publish_ctl(8 + sizeof(bfs::ThinCtl) / 8);
+        bfs::ThinCtl r;
+        std::memcpy(&r, ctx.h_ctl + 8, sizeof r);
+        w.thin_tag += std::min(r.levels, p.max_levels) + 1;
+        if (r.status) raise(GRUS_E_TIMEOUT, "bfs thin levels aborted (barrier timeout)");
+        if (r.nf > V || r.levels == 0 || r.cur > 1 || r.e_add < mf)
+          raise(GRUS_E_HIP, "bfs thin levels reported an impossible state");
+        if (trace) {
+          auto now = std::chrono::steady_clock::now();
+          fprintf(stderr, "bfs levels %u-%u %s: nf=%llu -> %u %.1f us\n", level,
+                  level + r.levels - 1, solo ? "solo" : "grid", (unsigned long long)nf, r.nf,
+                  std::chrono::duration<double, std::micro>(now - t_level).count());
+          t_level = now;
+        }
+        // the launch counted the out-edges of what it expanded, this
+        // frontier's among them, and those of the frontier it left
+        const uint64_t e_new = r.e_add - mf + r.mf;
+        level += r.levels;
+        cur = (int)r.cur;
+        prev_nf = r.prev_nf;
+        nf = r.nf;
+        mf = r.mf;
+        mu = mu >= e_new ? mu - e_new : 0;
+        v_reached += r.v_add;
+        e_reached += e_new;
+        have_queue = true;
+        have_bitmap = false;
+        continue;
       }
       if (nf <= bfs::SL_F && mf <= bfs::SL_E) {
         // small levels: one workgroup runs them back to back on the device
