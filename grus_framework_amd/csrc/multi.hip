@@ -553,11 +553,63 @@ __global__ void k_publish(uint64_t *d, uint64_t *h, uint32_t n) {
 }
 
 // ---- extraction ----
+// Rows of slots [s0, s0 + n) of the vertex-major [V][128] distances, widened,
+// to out[(slot - s0) * V + v].  A workgroup turns a tile of TR_V vertices by
+// TR_S slots through LDS, so it reads runs of TR_S entries and writes runs of
+// TR_V (a gather of one slot's column touches a cache line per vertex: 128
+// rows at V = 2^18 took 128 x 3.7 us and a copy and a wait each).
+constexpr uint32_t TR_V = 64, TR_S = 32;
 template <class T>
-__global__ void k_gather_col(const T *dist, uint64_t V, uint32_t slot, uint32_t *row) {
-  uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-  uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (; i < V; i += stride) row[i] = wide_dist(dist[i * 128 + slot]);
+__global__ __launch_bounds__(BLOCK) void k_rows_out(const T *dist, uint64_t V, uint32_t s0,
+                                                    uint32_t n, uint32_t *out) {
+  __shared__ uint32_t tile[TR_S][TR_V + 1];
+  const uint32_t sb = blockIdx.y * TR_S;  // first slot of the tile, from s0
+  for (uint64_t v0 = (uint64_t)blockIdx.x * TR_V; v0 < V; v0 += (uint64_t)gridDim.x * TR_V) {
+    for (uint32_t i = threadIdx.x; i < TR_V * TR_S; i += BLOCK) {
+      const uint32_t s = i % TR_S, v = i / TR_S;
+      if (v0 + v < V && sb + s < n) tile[s][v] = wide_dist(dist[(v0 + v) * 128 + s0 + sb + s]);
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < TR_V * TR_S; i += BLOCK) {
+      const uint32_t v = i % TR_V, s = i / TR_V;
+      if (v0 + v < V && sb + s < n) out[(uint64_t)(sb + s) * V + v0 + v] = tile[s][v];
+    }
+    __syncthreads();  // the tile is rewritten
+  }
+}
+
+// finite entries of the slots in (lo, hi)
+template <class T>
+__global__ __launch_bounds__(BLOCK) void k_count_slots(const T *dist, uint64_t V, uint64_t lo,
+                                                       uint64_t hi, unsigned long long *out) {
+  constexpr uint32_t PER = 16 / sizeof(T);  // entries of a 16-byte load
+  const uint32_t s = (threadIdx.x * PER) % 128;  // BLOCK * PER is a multiple of 128
+  uint32_t mine = 0;  // bit k: entry k of this thread's loads belongs to a slot asked for
+#pragma unroll
+  for (uint32_t k = 0; k < PER; k++) mine |= (uint32_t)slot_in(lo, hi, s + k) << k;
+  unsigned long long n = 0;
+  const uint64_t end = V * 128;
+  for (uint64_t i = ((uint64_t)blockIdx.x * BLOCK + threadIdx.x) * PER; mine && i < end;
+       i += (uint64_t)gridDim.x * BLOCK * PER) {
+    const uint4 x = *reinterpret_cast<const uint4 *>(dist + i);
+    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+    for (uint32_t k = 0; k < PER; k++) {
+      const T e = sizeof(T) == 2 ? (T)(w[k / 2] >> (16 * (k & 1))) : (T)w[k];
+      n += e != (T)inf_of<T>() && ((mine >> k) & 1u);
+    }
+  }
+  block_add_u64(n, out);
+}
+
+// vertices reached, summed over the BFS lanes in mask
+__global__ __launch_bounds__(BLOCK) void k_count_visits(const uint64_t *visit, uint64_t V,
+                                                        uint64_t mask, unsigned long long *out) {
+  unsigned long long n = 0;
+  for (uint64_t v = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; v < V;
+       v += (uint64_t)gridDim.x * BLOCK)
+    n += (unsigned)__popcll(visit[v] & mask);
+  block_add_u64(n, out);
 }
 
 // the block's sums land in out[0], out[1] with one atomic pair per block
@@ -989,44 +1041,6 @@ std::vector<int> MsEngine::step() {
   return done;
 }
 
-void MsEngine::extract(int slot, uint32_t *host_out, uint64_t *reached, uint64_t *checksum,
-                       uint32_t *device_out) {
-  Context &ctx = *ctx_;
-  ctx.activate();
-  const uint64_t V = g_.V;
-  uint32_t *row;
-  if (kind_ == MsKind::BFS) {
-    row = vals_.as<uint32_t>() + (uint64_t)slot * V;
-  } else {
-    row = device_out ? device_out : row_.as<uint32_t>();
-    if (narrow_)
-      ms::k_gather_col<uint16_t><<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(
-          vals_.as<uint16_t>(), V, (uint32_t)slot, row);
-    else
-      ms::k_gather_col<uint32_t><<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(
-          vals_.as<uint32_t>(), V, (uint32_t)slot, row);
-    GRUS_LAUNCH_CHECK();
-  }
-  if (device_out && row != device_out)
-    GRUS_HIP(hipMemcpyAsync(device_out, row, V * 4, hipMemcpyDeviceToDevice, ctx.stream));
-  if (reached || checksum) {
-    auto *d = digest_.as<unsigned long long>();
-    GRUS_HIP(hipMemsetAsync(d, 0, 16, ctx.stream));
-    ms::k_digest<<<grid_cap(ctx, V, BLOCK, 4), BLOCK, 0, ctx.stream>>>(row, V, d);
-    GRUS_LAUNCH_CHECK();
-    unsigned long long h[2];
-    GRUS_HIP(hipMemcpyAsync(h, d, 16, hipMemcpyDeviceToHost, ctx.stream));
-    if (host_out)
-      GRUS_HIP(hipMemcpyAsync(host_out, row, V * 4, hipMemcpyDeviceToHost, ctx.stream));
-    ctx.sync();
-    if (checksum) *checksum = h[0];
-    if (reached) *reached = h[1];
-  } else if (host_out) {
-    GRUS_HIP(hipMemcpyAsync(host_out, row, V * 4, hipMemcpyDeviceToHost, ctx.stream));
-    ctx.sync();
-  }
-}
-
 void MsEngine::digest(SlotMask mask, uint64_t *reached, uint64_t *checksum) {
   if (!mask) return;
   Context &ctx = *ctx_;
@@ -1054,6 +1068,65 @@ void MsEngine::digest(SlotMask mask, uint64_t *reached, uint64_t *checksum) {
     checksum[sl] = h[2 * sl];
     reached[sl] = h[2 * sl + 1];
   }
+}
+
+uint64_t MsEngine::reached(SlotMask mask) {
+  if (!mask || !g_.V) return 0;
+  Context &ctx = *ctx_;
+  ctx.activate();
+  const uint64_t V = g_.V;
+  auto *d = digest_.as<unsigned long long>();
+  fill_u64(ctx, digest_.as<uint64_t>(), 1, 0);
+  const uint64_t lo = (uint64_t)mask, hi = (uint64_t)(mask >> 64);
+  if (kind_ == MsKind::BFS)
+    ms::k_count_visits<<<grid_cap(ctx, V, BLOCK, 4), BLOCK, 0, ctx.stream>>>(
+        visit_.as<uint64_t>(), V, lo, d);
+  else if (narrow_)
+    ms::k_count_slots<uint16_t><<<grid_cap(ctx, V * 16, BLOCK, 8), BLOCK, 0, ctx.stream>>>(
+        vals_.as<uint16_t>(), V, lo, hi, d);
+  else
+    ms::k_count_slots<uint32_t><<<grid_cap(ctx, V * 32, BLOCK, 8), BLOCK, 0, ctx.stream>>>(
+        vals_.as<uint32_t>(), V, lo, hi, d);
+  GRUS_LAUNCH_CHECK();
+  return read_u64(reinterpret_cast<const uint64_t *>(d));
+}
+
+void MsEngine::copy_out(int slot0, int n, uint32_t *host_out) {
+  Context &ctx = *ctx_;
+  ctx.activate();
+  const uint64_t V = g_.V;
+  if (kind_ == MsKind::BFS) {  // the rows lie one behind the other
+    GRUS_HIP(hipMemcpyAsync(host_out, vals_.as<uint32_t>() + (uint64_t)slot0 * V,
+                            (uint64_t)n * V * 4, hipMemcpyDeviceToHost, ctx.stream));
+    ctx.sync();
+    return;
+  }
+  // as many rows at a time as ROWS_OUT bytes hold, from a buffer kept with
+  // the engine; under a device budget, which has no room for it, one at a time
+  constexpr uint64_t ROWS_OUT = 64ull << 20;
+  uint64_t rows = 1;
+  uint32_t *stage = row_.as<uint32_t>();
+  if (!devmem_budget(ctx.device) && V) {
+    rows = std::min<uint64_t>((uint64_t)n, std::max<uint64_t>(1, ROWS_OUT / (V * 4)));
+    if (rows > 1) {
+      rows_.ensure(rows * V * 4);
+      stage = rows_.as<uint32_t>();
+    }
+  }
+  for (uint64_t at = 0; at < (uint64_t)n; at += rows) {
+    const uint32_t m = (uint32_t)std::min<uint64_t>(rows, (uint64_t)n - at);
+    const dim3 grid(grid_cap(ctx, V, ms::TR_V, 8), (unsigned)div_up(m, ms::TR_S));
+    if (narrow_)
+      ms::k_rows_out<uint16_t><<<grid, BLOCK, 0, ctx.stream>>>(vals_.as<uint16_t>(), V,
+                                                              (uint32_t)(slot0 + at), m, stage);
+    else
+      ms::k_rows_out<uint32_t><<<grid, BLOCK, 0, ctx.stream>>>(vals_.as<uint32_t>(), V,
+                                                              (uint32_t)(slot0 + at), m, stage);
+    GRUS_LAUNCH_CHECK();
+    GRUS_HIP(hipMemcpyAsync(host_out + at * V, stage, (uint64_t)m * V * 4, hipMemcpyDeviceToHost,
+                            ctx.stream));
+  }
+  ctx.sync();
 }
 
 void MsEngine::release(int slot) {
@@ -1089,16 +1162,17 @@ void run_multi(Graph &g, MsKind kind, const uint32_t *srcs, int k, uint32_t *out
   GRUS_HIP(hipEventSynchronize(ctx.ev1));
   float ms = 0;
   GRUS_HIP(hipEventElapsedTime(&ms, ctx.ev0, ctx.ev1));
-  // the reached counts of every slot in one pass over the engine's state;
-  // the rows are gathered one by one only when they are copied out
   SlotMask all = 0;
   for (int sl : slots) all |= slot_bit(sl);
-  uint64_t reached[128], checksum[128];
-  e.digest(all, reached, checksum);
-  uint64_t vr = 0;
-  for (int sl : slots) vr += reached[sl];
-  if (out)
-    for (int i = 0; i < k; i++) e.extract(slots[i], out + (uint64_t)i * g.V, nullptr, nullptr);
+  const uint64_t vr = st ? e.reached(all) : 0;
+  if (out) {  // runs of consecutive slots (an idle engine hands out 0, 1, 2, ...)
+    for (int i = 0; i < k;) {
+      int j = i + 1;
+      while (j < k && slots[j] == slots[j - 1] + 1) j++;
+      e.copy_out(slots[i], j - i, out + (uint64_t)i * g.V);
+      i = j;
+    }
+  }
   for (int sl : slots) e.release(sl);
   if (st) {
     *st = grus_stats{};

@@ -74,13 +74,14 @@ class MsEngine {
   std::vector<int> admit(const uint32_t *srcs, int n);
   // one expansion step of every busy slot; returns slots that finished
   std::vector<int> step();
-  // slot result (V u32) into a device row, then optionally to host memory;
-  // reached = finite entries, checksum = sum over v of mix64(v << 32 | value)
-  void extract(int slot, uint32_t *host_out, uint64_t *reached, uint64_t *checksum,
-               uint32_t *device_out = nullptr);
-  // reached / checksum (as extract) of every slot in mask, in one pass over
-  // the engine's state; results land at [slot]
+  // reached = finite entries and checksum = sum over v of mix64(v << 32 |
+  // value) of every slot in mask, in one pass over the engine's state;
+  // results land at [slot]
   void digest(SlotMask mask, uint64_t *reached, uint64_t *checksum);
+  // finite entries of the slots in mask, all together
+  uint64_t reached(SlotMask mask);
+  // the rows of slots [slot0, slot0 + n), n * V u32, to host memory
+  void copy_out(int slot0, int n, uint32_t *host_out);
   void release(int slot);  // slot becomes free (reset lazily at next admit)
   Context &ctx() { return *ctx_; }
   uint64_t steps() const { return t_; }
@@ -101,7 +102,7 @@ class MsEngine {
   bool narrow_ = false;
   uint64_t t_ = 0;         // global step counter
   uint64_t qn_ = 0, front_edges_ = 0;
-  Buf visit_, front_, next_, vals_, queue_, longq_, row_, digest_, srcs_dev_, cnt_, push_cnt_;
+  Buf visit_, front_, next_, vals_, queue_, longq_, row_, rows_, digest_, srcs_dev_, cnt_, push_cnt_;
   Buf hmirror_;  // pinned host words: the counters as published, then read-back scratch
   PushWork push_;
   Buf scan_tmp_;  // the step's scan temporaries, owned: a step allocates nothing

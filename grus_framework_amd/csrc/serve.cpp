@@ -384,7 +384,7 @@ class ServerImpl : public Server {
         for (SlotMask m = done; m; m &= m - 1) {
           const int sl = slot_lowest(m);
           const Query &q = slot_q[sl];
-          if (opts_.copy_results) eng->extract(sl, q.out, nullptr, nullptr);
+          if (opts_.copy_results && q.out) eng->copy_out(sl, 1, q.out);
           eng->release(sl);
           finish(q, GRUS_OK, reached[sl], checksum[sl]);
         }
