@@ -163,7 +163,7 @@ unsigned push_grid(Context &ctx, uint64_t total) { return grid_cap(ctx, total, L
 #define GATHER_PER_CU 2
 #endif
 
-// A workgroup copies LB_CHUNK consecutive positions: thread 0 finds the
+// A workgroup copies LB_CHUNK consecutive positions: two waves find the
 // queue entries that own the chunk's ends, the owners' scan values and row
 // starts are staged in LDS, and each thread copies LB_CHUNK / BLOCK edges in
 // coalesced rounds (rows are contiguous, so consecutive positions of one
@@ -176,18 +176,12 @@ __global__ __launch_bounds__(BLOCK) void k_gather_rows(CsrView g, const uint32_t
                                                        uint64_t k1, uint32_t *col, uint32_t *w) {
   __shared__ uint64_t sS[LB_WIN];
   __shared__ uint64_t sRow[LB_WIN];
-  __shared__ uint32_t s_i0, s_n;
+  __shared__ uint32_t s_own[2];
   for (uint64_t c0 = k0 + (uint64_t)blockIdx.x * LB_CHUNK; c0 < k1;
        c0 += (uint64_t)gridDim.x * LB_CHUNK) {
     const uint64_t c1 = c0 + LB_CHUNK < k1 ? c0 + LB_CHUNK : k1;
-    if (threadIdx.x == 0) {
-      const uint32_t i0 = upper_bound_u64(S, 0, F + 1, c0) - 1;
-      const uint32_t i1 = upper_bound_u64(S, i0, F + 1, c1 - 1) - 1;
-      s_i0 = i0;
-      s_n = i1 - i0 + 2;
-    }
-    __syncthreads();
-    const uint32_t i0 = s_i0, n = s_n;
+    chunk_owners(S, F, c0, c1, s_own);
+    const uint32_t i0 = s_own[0], n = s_own[1] - i0 + 2;
     const bool staged = n <= LB_WIN;
     if (staged) {
       for (uint32_t t = threadIdx.x; t < n; t += blockDim.x) {

@@ -80,6 +80,35 @@ __device__ __forceinline__ uint32_t upper_bound_u64(const uint64_t *a, uint32_t 
   return lo;
 }
 
+// The same by a whole wave (every lane calls it with the same arguments, in
+// global memory): 64 probes a step, so a queue of 4096 takes two dependent
+// loads and one of 2^24 four, where one thread's binary search took 12 and 24.
+__device__ __forceinline__ uint32_t wave_upper_bound_u64(const uint64_t *a, uint32_t lo,
+                                                         uint32_t hi, uint64_t key) {
+  for (;;) {
+    const uint32_t step = (hi - lo + WAVE - 1) / WAVE;
+    const uint64_t idx = (uint64_t)lo + (uint64_t)lane_id() * step;
+    // a is non-decreasing, so the probes at most key are the first c lanes
+    const uint32_t c = (uint32_t)__popcll(__ballot(idx < hi && a[idx] <= key));
+    if (step <= 1 || c == 0) return lo + c;
+    const uint64_t end = (uint64_t)lo + (uint64_t)c * step;
+    lo += (c - 1) * step + 1;
+    if (end < hi) hi = (uint32_t)end;
+  }
+}
+
+// own[0], own[1] (LDS) <- the queue entries that own positions c0 and c1 - 1
+// of the edge space scanned in S; one wave each.  Ends with a barrier.
+__device__ __forceinline__ void chunk_owners(const uint64_t *S, uint32_t F, uint64_t c0,
+                                             uint64_t c1, uint32_t *own) {
+  const uint32_t wid = threadIdx.x / WAVE;
+  if (wid < 2) {
+    const uint32_t i = wave_upper_bound_u64(S, 0, F + 1, wid ? c1 - 1 : c0) - 1;
+    if (lane_id() == 0) own[wid] = i;
+  }
+  __syncthreads();
+}
+
 // Edge-balanced push over queue q[0..F) with S = exclusive scan of its
 // out-degrees (S[F] = total), for the positions [k0, k1) of the frontier's
 // edge space.  Job supplies update/generate/next-queue.  kStaged: the edges
@@ -93,20 +122,14 @@ __global__ __launch_bounds__(BLOCK) void k_push_lb(CsrView g, const uint32_t *q,
   __shared__ uint64_t sS[LB_WIN];
   __shared__ uint64_t sRow[LB_WIN];
   __shared__ uint32_t sQ[LB_WIN];
-  __shared__ uint32_t s_i0, s_n;
+  __shared__ uint32_t s_own[2];
   __shared__ uint32_t s_app[BLOCK / WAVE + 1];
   uint64_t my_edges = 0;
   for (uint64_t c0 = k0 + (uint64_t)blockIdx.x * LB_CHUNK; c0 < total;
        c0 += (uint64_t)gridDim.x * LB_CHUNK) {
     uint64_t c1 = c0 + LB_CHUNK < total ? c0 + LB_CHUNK : total;
-    if (threadIdx.x == 0) {
-      uint32_t i0 = upper_bound_u64(S, 0, F + 1, c0) - 1;
-      uint32_t i1 = upper_bound_u64(S, i0, F + 1, c1 - 1) - 1;
-      s_i0 = i0;
-      s_n = i1 - i0 + 2;
-    }
-    __syncthreads();
-    const uint32_t i0 = s_i0, n = s_n;
+    chunk_owners(S, F, c0, c1, s_own);
+    const uint32_t i0 = s_own[0], n = s_own[1] - i0 + 2;
     const bool staged = n <= LB_WIN;
     if (staged) {
       for (uint32_t t = threadIdx.x; t < n; t += blockDim.x) {
