@@ -226,7 +226,11 @@ __global__ void k_first_in(CsrView in, uint32_t *first) {
 // latencies, the second an L2-resident bitmap word (reading the first
 // neighbour through the offsets added a dependent, uncoalesced column
 // load).  Most RMAT vertices find a parent at their first (lowest-id)
-// in-neighbour.
+// in-neighbour.  The vertices that do not are gathered in LDS and scanned 64
+// at a time: a scan is a chain of dependent loads, and word by word every
+// word with one such vertex paid it, with most lanes idle (RMAT s24, dense
+// steps 184 -> 150 us on average; 4 words a step or 8 in-edges a round
+// measured the same within 3%, more waves at fewer registers slower).
 constexpr int PULL_UNROLL = 8;
 constexpr int PULL_BATCH = 4;  // in-edges tested per dependent load round
 __global__ __launch_bounds__(BLOCK) void k_pull(CsrView in, const uint64_t *out_off,
@@ -234,14 +238,20 @@ __global__ __launch_bounds__(BLOCK) void k_pull(CsrView in, const uint64_t *out_
                                                 uint64_t *visited, uint64_t *front_next,
                                                 uint32_t *label, uint32_t next_level, uint32_t K,
                                                 uint32_t *longq, StepCounters *cnt, uint64_t W) {
+  constexpr uint32_t SPAN = PULL_UNROLL * WAVE;
+  __shared__ uint16_t s_pend[BLOCK / WAVE][SPAN];        // vertices to scan, from w0 * 64
+  __shared__ uint32_t s_hit[BLOCK / WAVE][SPAN / 32];    // those of them with a parent
+  const uint32_t wid = threadIdx.x / WAVE;
+  uint16_t *pend = s_pend[wid];
+  uint32_t *hit = s_hit[wid];
   uint64_t wave = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) / WAVE;
   uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
   uint32_t lane = lane_id();
   uint32_t my_found = 0;
   uint64_t my_edges = 0;
   for (uint64_t w0 = wave * PULL_UNROLL; w0 < W; w0 += nwaves * PULL_UNROLL) {
-    uint64_t vis[PULL_UNROLL], beg[PULL_UNROLL], end[PULL_UNROLL];
-    bool active[PULL_UNROLL], found[PULL_UNROLL];
+    uint64_t vis[PULL_UNROLL], deg[PULL_UNROLL];
+    bool found[PULL_UNROLL];
     uint32_t first[PULL_UNROLL];
     // visited words, first in-neighbours and offsets: independent loads
 #pragma unroll
@@ -250,31 +260,37 @@ __global__ __launch_bounds__(BLOCK) void k_pull(CsrView in, const uint64_t *out_
       const bool in_range = v < in.V;
       vis[j] = (w0 + j < W) ? visited[w0 + j] : ~0ull;
       first[j] = in_range ? first_in[v] : GRUS_NO_VERTEX;
-      beg[j] = in_range ? in.off[v] : 0;
-      end[j] = in_range ? in.off[v + 1] : 0;
+      deg[j] = in_range ? in.off[v + 1] - in.off[v] : 0;
     }
+    uint32_t np = 0;  // vertices to scan (wave-uniform)
 #pragma unroll
     for (int j = 0; j < PULL_UNROLL; j++) {
       // pull_selector (bfs.cu:80-87): label == INFINIT, read as a clear
       // visited bit (bits past V are set at init)
-      active[j] = ((vis[j] >> lane) & 1ull) == 0;
-      found[j] = active[j] && first[j] != GRUS_NO_VERTEX && bm_test(front, first[j]);
+      const bool active = ((vis[j] >> lane) & 1ull) == 0;
+      found[j] = active && first[j] != GRUS_NO_VERTEX && bm_test(front, first[j]);
+      const bool scan = active && !found[j] && deg[j] > 1;
+      const uint64_t m = __ballot(scan);
+      if (scan) pend[np + lane_rank(m)] = (uint16_t)(j * WAVE + lane);
+      np += (uint32_t)__popcll(m);
     }
-#pragma unroll
-    for (int j = 0; j < PULL_UNROLL; j++) {
-      if (vis[j] == ~0ull) {
-        if (lane == 0 && w0 + j < W) front_next[w0 + j] = 0;
-        continue;
-      }
-      uint32_t v = (uint32_t)((w0 + j) * 64 + lane);
+    if (lane < SPAN / 32) hit[lane] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (uint32_t i0 = 0; i0 < np; i0 += WAVE) {
       bool is_long = false;
-      if (active[j] && !found[j] && beg[j] < end[j]) {
-        uint64_t e = beg[j] + 1;
-        uint64_t lim = (end[j] - beg[j] > K) ? beg[j] + K : end[j];
+      uint32_t v = 0;
+      if (i0 + lane < np) {
+        const uint32_t x = pend[i0 + lane];
+        v = (uint32_t)(w0 * 64) + x;
+        const uint64_t b = in.off[v], d = in.off[v + 1];  // (read just before: cached)
+        const uint64_t lim = (d - b > K) ? b + K : d;
+        bool ok = false;
         // PULL_BATCH columns, then their PULL_BATCH frontier words, are
         // loaded independently: one column -> bitmap latency chain per batch
         // instead of per edge (a batch may read past the parent it finds)
-        for (; e < lim && !found[j]; e += PULL_BATCH) {
+        for (uint64_t e = b + 1; e < lim && !ok; e += PULL_BATCH) {
           uint32_t c[PULL_BATCH];
 #pragma unroll
           for (int q = 0; q < PULL_BATCH; q++) c[q] = (e + q < lim) ? edge_col(in, e + q) : 0u;
@@ -282,23 +298,32 @@ __global__ __launch_bounds__(BLOCK) void k_pull(CsrView in, const uint64_t *out_
 #pragma unroll
           for (int q = 0; q < PULL_BATCH; q++) fw[q] = (e + q < lim) ? front[c[q] >> 6] : 0ull;
 #pragma unroll
-          for (int q = 0; q < PULL_BATCH; q++) found[j] = found[j] || ((fw[q] >> (c[q] & 63)) & 1ull);
+          for (int q = 0; q < PULL_BATCH; q++) ok = ok || ((fw[q] >> (c[q] & 63)) & 1ull);
         }
-        is_long = !found[j] && lim < end[j];
+        is_long = !ok && lim < d;
+        if (ok) atomicOr(&hit[x / 32], 1u << (x % 32));
       }
-      uint64_t m = __ballot(found[j]);
+      const uint32_t slot = wave_append(&cnt->long_count, is_long);
+      if (is_long) longq[slot] = v;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int j = 0; j < PULL_UNROLL; j++) {
+      if (w0 + j >= W) continue;
+      const uint64_t m = __ballot(found[j]) | hit[2 * j] | ((uint64_t)hit[2 * j + 1] << 32);
       if (lane == 0) {
         front_next[w0 + j] = m;
         if (m) visited[w0 + j] = vis[j] | m;
       }
-      if (found[j]) {
+      if ((m >> lane) & 1ull) {
+        const uint32_t v = (uint32_t)((w0 + j) * 64 + lane);
         label[v] = next_level;
         my_found++;
         // out-degree: the in-edge row itself on a symmetric graph
-        my_edges += (out_off == in.off) ? end[j] - beg[j] : out_off[v + 1] - out_off[v];
+        my_edges += (out_off == in.off) ? deg[j] : out_off[v + 1] - out_off[v];
       }
-      uint32_t slot = wave_append(&cnt->long_count, is_long);
-      if (is_long) longq[slot] = v;
     }
   }
   block_add_counts(my_found, my_edges, &cnt->next_count,
