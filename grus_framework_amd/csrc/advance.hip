@@ -140,13 +140,14 @@ __global__ __launch_bounds__(BLOCK) void k_reached(const uint64_t *off, const ui
 
 void reached_stats(Context &ctx, const uint64_t *off, const uint32_t *val, uint64_t V,
                    uint64_t *vr, uint64_t *er) {
+  // words 40 and 41 of the control block are nobody else's: zero since the
+  // context began, and again whenever they were published
   auto *acc = reinterpret_cast<unsigned long long *>(ctx.d_ctl.p) + 40;
-  GRUS_HIP(hipMemsetAsync(acc, 0, 16, ctx.stream));
   if (V) {
-    k_reached<<<grid_cap(ctx, V, BLOCK, 4), BLOCK, 0, ctx.stream>>>(off, val, V, acc);
+    k_reached<<<grid_cap(ctx, V, BLOCK, 8), BLOCK, 0, ctx.stream>>>(off, val, V, acc);
     GRUS_LAUNCH_CHECK();
   }
-  ctx.read_ctl(42);
+  ctx.publish_ctl(42);
   *vr = ctx.h_ctl[40];
   *er = ctx.h_ctl[41];
 }

@@ -32,7 +32,7 @@ struct StepCounters {
   uint32_t long_count;   // bottom-up vertices handed to a cooperative scan
   uint64_t next_edges;   // sum of out-degrees of the next frontier
   uint32_t far_count;    // vertices appended to the far queue (SSSP)
-  uint32_t min_far;      // minimum live far distance (SSSP threshold advance)
+  uint32_t min_far;      // SSSP far split: largest complement of a distance left far (0: none)
   uint32_t rem_count;    // BFS bottom-up: vertices still unvisited after the step
   uint32_t pad32;
   uint64_t pad[4];

@@ -15,6 +15,7 @@
 // stamps (u32), which never need clearing between rounds.
 #include <algorithm>
 #include <cstdlib>
+#include <cstring>
 
 #include "advance.hpp"
 #include "apps.hpp"
@@ -204,11 +205,13 @@ __global__ void k_pull_min_fixup(CsrView in, const uint32_t *win_row, PullMinOp 
   window_fixup(in, win_row, k, op);
 }
 
-// the first queue is {src}, stamped like every later queue
+// the first queue is {src}, stamped like every later queue; the step counters
+// start from zero
 __global__ void k_init(uint32_t *dist, uint64_t V, uint32_t src, uint32_t *q0,
-                       uint32_t *near_stamp, uint32_t id) {
+                       uint32_t *near_stamp, uint32_t id, StepCounters *cnt) {
   uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
   uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  if (i == 0) *cnt = StepCounters{};
   for (; i < V; i += stride) {
     dist[i] = (i == src) ? 0u : INFINIT;  // SSSPInit sssp.cu:21
     if (i == 0) {
@@ -218,54 +221,226 @@ __global__ void k_init(uint32_t *dist, uint64_t V, uint32_t src, uint32_t *q0,
   }
 }
 
-// smallest distance >= T among far entries
-__global__ void k_far_min(const uint32_t *far, uint32_t n, const uint32_t *dist, uint32_t T,
-                          uint32_t *out) {
-  uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-  uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  uint32_t m = 0xFFFFFFFFu;
-  for (; i < n; i += stride) {
-    uint32_t d = dist[far[i]];
-    if (d >= T && d < m) m = d;
-  }
-  for (int o = 32; o > 0; o >>= 1) {
-    uint32_t x = __shfl_xor(m, o);
-    m = x < m ? x : m;
-  }
-  if (lane_id() == 0 && m != 0xFFFFFFFFu) atomicMin(out, m);
-}
-
-// split the far queue at the new threshold: [T_old, T) -> near, >= T -> far'
-// (entries below T_old were already relaxed at their final near distance)
-__global__ void k_far_split(const uint32_t *far, uint32_t n, const uint32_t *dist,
-                            const uint64_t *out_off, uint32_t T_old, uint32_t T,
-                            uint32_t *near_stamp, uint32_t near_id, uint32_t *far_stamp,
-                            uint32_t far_id, uint32_t *qn, uint32_t *far_out,
-                            StepCounters *cnt) {
-  uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  uint64_t first = blockIdx.x * (uint64_t)blockDim.x + (threadIdx.x & ~(uint64_t)(WAVE - 1));
+// Split of the far queue at the new threshold: [T_old, T) -> near, >= T ->
+// far' (entries below T_old were relaxed at their final near distance), with
+// the smallest distance of far', as the largest complement, for a split that
+// finds its bucket empty.  A workgroup takes SPLIT_PER entries a thread and
+// reserves its slots of either queue once: with an atomic per wave the two
+// counters were what the pass waited for (RMAT s20, 188 K entries: minimum
+// and split 34 + 44 us).
+constexpr uint32_t SPLIT_PER = 4;
+__global__ __launch_bounds__(BLOCK) void k_far_split(
+    const uint32_t *far, uint32_t n, const uint32_t *dist, const uint64_t *out_off,
+    uint32_t T_old, uint32_t T, uint32_t *near_stamp, uint32_t near_id, uint32_t *far_stamp,
+    uint32_t far_id, uint32_t *qn, uint32_t *far_out, StepCounters *cnt) {
+  __shared__ uint32_t s_app[BLOCK / WAVE + 1];
+  __shared__ uint32_t s_max;
+  if (threadIdx.x == 0) s_max = 0;
   uint64_t my_edges = 0;
-  for (uint64_t base = first; base < n; base += stride) {
-    uint64_t i = base + lane_id();
-    int to = 0;
-    uint32_t v = 0;
-    if (i < n) {
-      v = far[i];
-      uint32_t d = dist[v];
-      if (d >= T_old) {
-        if (d < T) to = atomicExch(&near_stamp[v], near_id) != near_id ? 1 : 0;
-        else to = atomicExch(&far_stamp[v], far_id) != far_id ? 2 : 0;
+  uint32_t top = 0;  // largest complement
+  constexpr uint32_t SPAN = SPLIT_PER * BLOCK;
+  for (uint64_t base = (uint64_t)blockIdx.x * SPAN; base < n; base += (uint64_t)gridDim.x * SPAN) {
+    uint32_t v[SPLIT_PER], to_near = 0, to_far = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < SPLIT_PER; k++) {
+      const uint64_t i = base + k * BLOCK + threadIdx.x;
+      v[k] = i < n ? far[i] : 0u;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < SPLIT_PER; k++) {
+      const uint64_t i = base + k * BLOCK + threadIdx.x;
+      const uint32_t d = i < n ? dist[v[k]] : 0u;
+      if (i >= n || d < T_old) continue;
+      if (d < T) {
+        if (atomicExch(&near_stamp[v[k]], near_id) != near_id) to_near |= 1u << k;
+      } else {
+        top = max(top, ~d);
+        if (atomicExch(&far_stamp[v[k]], far_id) != far_id) to_far |= 1u << k;
       }
     }
-    uint32_t s1 = wave_append(&cnt->next_count, to == 1);
-    if (to == 1) {
-      qn[s1] = v;
-      my_edges += out_off[v + 1] - out_off[v];
+    uint32_t s1 = block_reserve(&cnt->next_count, (uint32_t)__popc(to_near), s_app);
+    uint32_t s2 = block_reserve(&cnt->far_count, (uint32_t)__popc(to_far), s_app);
+#pragma unroll
+    for (uint32_t k = 0; k < SPLIT_PER; k++) {
+      if ((to_near >> k) & 1u) {
+        qn[s1++] = v[k];
+        my_edges += out_off[v[k] + 1] - out_off[v[k]];
+      }
+      if ((to_far >> k) & 1u) far_out[s2++] = v[k];
     }
-    uint32_t s2 = wave_append(&cnt->far_count, to == 2);
-    if (to == 2) far_out[s2] = v;
   }
+  __syncthreads();
+  if (top) atomicMax(&s_max, top);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_max) atomicMax(&cnt->min_far, s_max);
   block_add_u64(my_edges, (unsigned long long *)&cnt->next_edges);
+}
+
+// Near rounds and far splits with little to do, back to back in one
+// workgroup: while the near queue has at most SR_F vertices and SR_E
+// out-edges (or is empty and the far queue holds at most SR_FAR), the
+// workgroup relaxes the queue, splits the far queue when the near one runs
+// dry, and goes on, with workgroup barriers in between.  The first and the
+// last rounds of most runs are such rounds; each takes four launches and a
+// read-back (~45 us) on its own.  A call on RMAT s8 0.36 -> 0.10 ms, s12 0.68
+// -> 0.39 ms, s22 2.63 -> 2.15 ms.  SR_E: a workgroup relaxes 4096 edges in
+// about 4 us, so 16384 cost what launching the round would.
+constexpr uint32_t SR_T = 1024;
+constexpr uint32_t SR_F = SR_T;
+constexpr uint32_t SR_PER = 4;  // edges per thread in flight together
+constexpr uint64_t SR_E = 16384;
+constexpr uint32_t SR_FAR = 8192;
+constexpr uint32_t SR_ROUNDS = 1u << 16;  // per launch
+
+struct SmallRounds {
+  uint64_t T, mf, relaxed;
+  uint32_t nn, nfar, cur, fcur, stamp, cur_id, far_id, fmin, rounds, pad;
+};
+
+struct SmallParams {
+  CsrView g;
+  uint32_t *dist, *q0, *q1, *far0, *far1, *near_stamp, *far_stamp;
+  SmallRounds s;  // state on entry (mf, relaxed and rounds are outputs)
+  uint64_t delta, max_edges;  // max_edges <= SR_E
+  SmallRounds *out;
+};
+
+__global__ __launch_bounds__(SR_T) void k_small_rounds(SmallParams p) {
+  __shared__ uint64_t sRow[SR_F];
+  __shared__ uint32_t sS[SR_F + 1];  // exclusive prefix of the degrees (at most SR_E when used)
+  __shared__ uint32_t sQ[SR_F];
+  __shared__ uint64_t s_wsum[SR_T / WAVE];
+  __shared__ uint32_t s_nn, s_nf, s_min;
+  const CsrView g = p.g;
+  uint32_t *q[2] = {p.q0, p.q1}, *far[2] = {p.far0, p.far1};
+  const uint32_t t = threadIdx.x, lane = lane_id(), wid = t / WAVE;
+  SmallRounds s = p.s;  // every thread holds the same state
+  s.mf = s.relaxed = 0;
+  s.rounds = 0;
+  uint64_t sum = 0;
+  for (;;) {
+    // out-degree sum of the near queue, and its prefix when it fits
+    uint64_t mine = 0;
+    for (uint32_t i = t; i < s.nn; i += SR_T) {
+      const uint32_t u = q[s.cur][i];
+      const uint64_t a = g.off[u], d = g.off[u + 1] - a;
+      if (i < SR_F) {
+        sQ[i] = u;
+        sRow[i] = a;
+      }
+      mine += d;
+    }
+    uint64_t x = mine;
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+      const uint64_t y = __shfl_up(x, o);
+      if ((int)lane >= o) x += y;
+    }
+    if (lane == WAVE - 1) s_wsum[wid] = x;
+    if (t == 0) {
+      s_nn = s_nf = 0;
+      s_min = 0xFFFFFFFFu;
+    }
+    __syncthreads();
+    uint64_t before = 0;
+    sum = 0;
+    for (uint32_t w = 0; w < SR_T / WAVE; w++) {
+      before += (w < wid) ? s_wsum[w] : 0ull;
+      sum += s_wsum[w];
+    }
+    if (s.rounds >= SR_ROUNDS) break;
+    if (s.nn) {
+      if (s.nn > SR_F || sum > p.max_edges) break;
+      if (t < s.nn) sS[t] = (uint32_t)(before + x - mine);
+      if (t == 0) sS[s.nn] = (uint32_t)sum;
+      __syncthreads();
+      s.rounds++;
+      s.relaxed += s.nn;
+      const uint32_t Tk = s.T < 0xFFFFFFFFull ? (uint32_t)s.T : 0xFFFFFFFFu;
+      const uint32_t near_id = ++s.stamp;
+      for (uint32_t k0 = 0; k0 < sum; k0 += SR_T * SR_PER) {
+        uint32_t v[SR_PER], nd[SR_PER], old[SR_PER];
+#pragma unroll
+        for (uint32_t r = 0; r < SR_PER; r++) {
+          const uint32_t k = k0 + r * SR_T + t;
+          nd[r] = INFINIT;
+          v[r] = 0;
+          if (k < sum) {
+            uint32_t lo = 0, hi = s.nn;  // sS[lo] <= k < sS[hi]
+            while (hi - lo > 1) {
+              const uint32_t mid = (lo + hi) / 2;
+              if (sS[mid] <= k) lo = mid;
+              else hi = mid;
+            }
+            const uint64_t e = sRow[lo] + (k - sS[lo]);
+            v[r] = edge_col(g, e);
+            // the queued vertex's distance as of now: the value it was queued
+            // with, or lower
+            const uint64_t c = (uint64_t)ld_agent(&p.dist[sQ[lo]]) + edge_w(g, e);
+            nd[r] = c < INFINIT ? (uint32_t)c : INFINIT;
+          }
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < SR_PER; r++)  // a stale-high read only lets a useless atomic through
+          old[r] = nd[r] < INFINIT && nd[r] < p.dist[v[r]] ? atomicMin(&p.dist[v[r]], nd[r]) : 0u;
+#pragma unroll
+        for (uint32_t r = 0; r < SR_PER; r++) {
+          if (old[r] <= nd[r]) continue;
+          if (nd[r] < Tk) {
+            if (atomicExch(&p.near_stamp[v[r]], near_id) != near_id)
+              q[s.cur ^ 1][atomicAdd(&s_nn, 1u)] = v[r];
+          } else if (atomicExch(&p.far_stamp[v[r]], s.far_id) != s.far_id) {
+            far[s.fcur][s.nfar + atomicAdd(&s_nf, 1u)] = v[r];
+          }
+        }
+      }
+      __syncthreads();
+      s.nn = s_nn;
+      s.nfar += s_nf;
+      s.cur ^= 1;
+      s.cur_id = near_id;
+      s.fmin = 0xFFFFFFFFu;  // the round may have added far vertices below it
+    } else if (s.nfar) {
+      if (s.nfar > SR_FAR) break;
+      // the next bucket, or the bucket of the smallest far distance where the
+      // last split found its own empty
+      const uint64_t Tn = s.fmin != 0xFFFFFFFFu ? ((uint64_t)s.fmin / p.delta + 1) * p.delta
+                                                : s.T + p.delta;
+      const uint32_t Tk = s.T < 0xFFFFFFFFull ? (uint32_t)s.T : 0xFFFFFFFFu;
+      const uint32_t Tnk = Tn < 0xFFFFFFFFull ? (uint32_t)Tn : 0xFFFFFFFFu;
+      s.far_id = ++s.stamp;
+      const uint32_t near_id = ++s.stamp;
+      uint32_t m = 0xFFFFFFFFu;
+      for (uint32_t i = t; i < s.nfar; i += SR_T) {
+        const uint32_t v = far[s.fcur][i];
+        const uint32_t d = ld_agent(&p.dist[v]);
+        if (d < Tk) continue;
+        if (d < Tnk) {
+          if (atomicExch(&p.near_stamp[v], near_id) != near_id)
+            q[s.cur][atomicAdd(&s_nn, 1u)] = v;
+        } else {
+          m = min(m, d);
+          if (atomicExch(&p.far_stamp[v], s.far_id) != s.far_id)
+            far[s.fcur ^ 1][atomicAdd(&s_nf, 1u)] = v;
+        }
+      }
+      if (m != 0xFFFFFFFFu) atomicMin(&s_min, m);
+      __syncthreads();
+      s.nn = s_nn;
+      s.nfar = s_nf;
+      s.fcur ^= 1;
+      s.T = Tn;
+      s.cur_id = near_id;
+      s.fmin = s.nn ? 0xFFFFFFFFu : s_min;
+    } else {
+      break;
+    }
+    __syncthreads();  // the counts are read before the next round clears them
+  }
+  if (t == 0) {
+    s.mf = sum;
+    *p.out = s;
+  }
 }
 
 __global__ void k_weight_sum(const uint32_t *w, uint64_t E, unsigned long long *out) {
@@ -722,12 +897,6 @@ void run_sssp(Graph &g, uint32_t src, grus_stats *st) {
   uint32_t *dist = g.result.as<uint32_t>();
   auto *cnt = reinterpret_cast<StepCounters *>(ctx.d_ctl.p);
   const StepCounters *hc = reinterpret_cast<const StepCounters *>(ctx.h_ctl);
-  uint64_t src_deg;
-  {
-    uint64_t o[2];
-    GRUS_HIP(hipMemcpy(o, g.off.as<uint64_t>() + src, 16, hipMemcpyDeviceToHost));
-    src_deg = o[1] - o[0];
-  }
   uint64_t launches = 0, rounds = 0, relaxed_vertices = 0, pull_rounds = 0, local_passes = 0;
   // low-degree graphs (grids, road-like): one persistent cooperative launch
   static const bool no_persist = getenv("GRUS_NO_PERSISTENT") != nullptr;
@@ -758,7 +927,7 @@ void run_sssp(Graph &g, uint32_t src, grus_stats *st) {
   const uint64_t wraps0 = w.wraps;
   GRUS_HIP(hipEventRecord(ctx.ev0, ctx.stream));
   sssp::k_init<<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(
-      dist, V, src, w.q[0].as<uint32_t>(), w.near_stamp.as<uint32_t>(), cur_id);
+      dist, V, src, w.q[0].as<uint32_t>(), w.near_stamp.as<uint32_t>(), cur_id, cnt);
   GRUS_LAUNCH_CHECK();
   launches++;
   if (persistent) {
@@ -766,16 +935,68 @@ void run_sssp(Graph &g, uint32_t src, grus_stats *st) {
     launches++;
   }
   int cur = 0, fcur = 0;
-  uint64_t nn = persistent ? 0 : 1, mf = src_deg, nfar = 0;
+  uint64_t nn = persistent ? 0 : 1, mf = 0, nfar = 0;  // (the source's degree: counted on the device)
   uint64_t T = delta;
   uint32_t far_id = w.next_stamp(ctx, V);
+  // a pull threshold that the caller chose holds for small rounds too
+  const uint64_t small_edges =
+      ctx.tuning.sssp_pull_div ? std::min(sssp::SR_E, pull_edges) : sssp::SR_E;
+  uint32_t fmin = 0xFFFFFFFFu;  // smallest far distance, where a split left it known
   const uint64_t round_cap = 64 * V + 1024;
   const uint64_t W = V / 64 + 1;
   for (;;) {
-    while (nn) {
+    // (the counters are zero here: cleared by k_init, then by publish_ctl)
+    if (w.stamp < 0xFFF00000u && ((nn && nn <= sssp::SR_F && mf <= small_edges) ||
+                                  (!nn && nfar && nfar <= sssp::SR_FAR))) {
+      // small rounds: one workgroup runs them back to back on the device
+      auto *so = reinterpret_cast<sssp::SmallRounds *>(ctx.d_ctl.as<uint64_t>() + 8);
+      sssp::SmallParams p{};
+      p.g = out;
+      p.dist = dist;
+      p.q0 = w.q[0].as<uint32_t>();
+      p.q1 = w.q[1].as<uint32_t>();
+      p.far0 = w.far[0].as<uint32_t>();
+      p.far1 = w.far[1].as<uint32_t>();
+      p.near_stamp = w.near_stamp.as<uint32_t>();
+      p.far_stamp = w.far_stamp.as<uint32_t>();
+      p.s.T = T;
+      p.s.nn = (uint32_t)nn;
+      p.s.nfar = (uint32_t)nfar;
+      p.s.cur = (uint32_t)cur;
+      p.s.fcur = (uint32_t)fcur;
+      p.s.stamp = w.stamp;
+      p.s.cur_id = cur_id;
+      p.s.far_id = far_id;
+      p.s.fmin = fmin;
+      p.delta = delta;
+      p.max_edges = small_edges;
+      p.out = so;
+      sssp::k_small_rounds<<<1, sssp::SR_T, 0, ctx.stream>>>(p);
+      GRUS_LAUNCH_CHECK();
+      launches++;
+      ctx.publish_ctl(8 + sizeof(sssp::SmallRounds) / 8);
+      sssp::SmallRounds r;
+      memcpy(&r, ctx.h_ctl + 8, sizeof r);
+      if (r.nn > V || r.nfar > V || r.cur > 1 || r.fcur > 1 || r.stamp < w.stamp)
+        raise(GRUS_E_HIP, "sssp small rounds reported an impossible state");
+      rounds += r.rounds;
+      if (rounds > round_cap) raise(GRUS_E_HIP, "sssp did not converge");
+      relaxed_vertices += r.relaxed;
+      nn = r.nn;
+      mf = r.mf;
+      nfar = r.nfar;
+      T = r.T;
+      cur = (int)r.cur;
+      fcur = (int)r.fcur;
+      w.stamp = r.stamp;
+      cur_id = r.cur_id;
+      far_id = r.far_id;
+      fmin = r.fmin;
+      if (!nn && !nfar) break;
+    }
+    if (nn) {
       if (++rounds > round_cap) raise(GRUS_E_HIP, "sssp did not converge");
       relaxed_vertices += nn;
-      GRUS_HIP(hipMemsetAsync(cnt, 0, sizeof(StepCounters), ctx.stream));
       const uint32_t Tk = (uint32_t)std::min<uint64_t>(T, 0xFFFFFFFFull);
       const uint32_t near_id = w.next_stamp(ctx, V);
       if (binned_pull && mf > pull_edges) {
@@ -843,7 +1064,6 @@ void run_sssp(Graph &g, uint32_t src, grus_stats *st) {
         launches += 4;
         pull_rounds++;
       } else {
-        push_scan_degrees(ctx, w.push, out.off, w.q[cur].as<uint32_t>(), (uint32_t)nn);
         sssp::job_t job{dist,
                         w.near_stamp.as<uint32_t>(),
                         w.far_stamp.as<uint32_t>(),
@@ -851,43 +1071,52 @@ void run_sssp(Graph &g, uint32_t src, grus_stats *st) {
                         Tk,
                         near_id,
                         far_id};
-        push_advance(ctx, w.push, out, w.q[cur].as<uint32_t>(), (uint32_t)nn, mf, job,
-                     w.q[cur ^ 1].as<uint32_t>(), cnt, w.far[fcur].as<uint32_t>() + nfar);
-        launches += 4;
+        uint32_t *qn = w.q[cur ^ 1].as<uint32_t>(), *qfar = w.far[fcur].as<uint32_t>() + nfar;
+        if (nn <= PUSH_SMALL_F) {  // one launch, the degree scan done in LDS
+          push_advance_small(ctx, out, w.q[cur].as<uint32_t>(), (uint32_t)nn, mf, job, qn, cnt,
+                             qfar);
+          launches += 1;
+        } else {
+          push_scan_degrees(ctx, w.push, out.off, w.q[cur].as<uint32_t>(), (uint32_t)nn);
+          push_advance(ctx, w.push, out, w.q[cur].as<uint32_t>(), (uint32_t)nn, mf, job, qn, cnt,
+                       qfar);
+          launches += 3;
+        }
       }
-      ctx.read_ctl(3);
+      ctx.publish_ctl(sizeof(StepCounters) / 8);  // read the round's counters and clear them
+      launches++;
       nn = hc->next_count;
       mf = hc->next_edges;
       nfar += hc->far_count;
+      fmin = 0xFFFFFFFFu;  // the round may have added far vertices below it
+      // the next round reads nn queue entries, the next split nfar far ones
+      if (nn > V || nfar > V) raise(GRUS_E_HIP, "sssp round reported impossible counts");
       cur ^= 1;
       cur_id = near_id;
+      continue;
     }
     if (nfar == 0) break;
-    // advance the threshold to the bucket of the smallest live far distance
-    GRUS_HIP(hipMemsetAsync(cnt, 0, sizeof(StepCounters), ctx.stream));
-    GRUS_HIP(hipMemsetAsync(&cnt->min_far, 0xFF, 4, ctx.stream));
-    uint32_t Tk = (uint32_t)std::min<uint64_t>(T, 0xFFFFFFFFull);
-    sssp::k_far_min<<<grid_cap(ctx, nfar, BLOCK), BLOCK, 0, ctx.stream>>>(
-        w.far[fcur].as<uint32_t>(), (uint32_t)nfar, dist, Tk, &cnt->min_far);
-    GRUS_LAUNCH_CHECK();
-    ctx.read_ctl(3);
-    uint32_t mn = hc->min_far;
-    if (mn == 0xFFFFFFFFu) break;  // every far entry was stale
-    uint64_t T_new = ((uint64_t)mn / delta + 1) * delta;
+    // Advance the threshold by one bucket and split the far queue, in one
+    // pass.  T is a multiple of delta and every live far distance lies at T
+    // or beyond, so a bucket that holds one is the bucket of the smallest; an
+    // empty one is followed by the bucket of the minimum its split found.
+    const uint32_t Tk = (uint32_t)std::min<uint64_t>(T, 0xFFFFFFFFull);
+    const uint64_t T_new = fmin != 0xFFFFFFFFu ? ((uint64_t)fmin / delta + 1) * delta : T + delta;
     far_id = w.next_stamp(ctx, V);
-    uint32_t near_id = w.next_stamp(ctx, V);
-    GRUS_HIP(hipMemsetAsync(cnt, 0, sizeof(StepCounters), ctx.stream));
-    sssp::k_far_split<<<grid_cap(ctx, nfar, BLOCK), BLOCK, 0, ctx.stream>>>(
+    const uint32_t near_id = w.next_stamp(ctx, V);
+    sssp::k_far_split<<<grid_cap(ctx, nfar, BLOCK * sssp::SPLIT_PER, 8), BLOCK, 0, ctx.stream>>>(
         w.far[fcur].as<uint32_t>(), (uint32_t)nfar, dist, out.off, Tk,
         (uint32_t)std::min<uint64_t>(T_new, 0xFFFFFFFFull), w.near_stamp.as<uint32_t>(),
         near_id, w.far_stamp.as<uint32_t>(), far_id, w.q[cur].as<uint32_t>(),
         w.far[fcur ^ 1].as<uint32_t>(), cnt);
     GRUS_LAUNCH_CHECK();
-    launches += 3;
-    ctx.read_ctl(3);
+    ctx.publish_ctl(sizeof(StepCounters) / 8);
+    launches += 2;
     nn = hc->next_count;
     mf = hc->next_edges;
     nfar = hc->far_count;
+    fmin = nn ? 0xFFFFFFFFu : ~hc->min_far;  // (as the largest complement; 0: none)
+    if (nn > V || nfar > V) raise(GRUS_E_HIP, "sssp split reported impossible counts");
     fcur ^= 1;
     T = T_new;
     cur_id = near_id;
