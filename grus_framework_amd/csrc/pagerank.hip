@@ -18,7 +18,7 @@
 // blocking over the pull (3) and a degree-sorted relabelled pull (1).
 //
 // Binned push (pr_layout = 4; build_binned, k_bp_scatter, k_bp_accum):
-// destinations are cut into bins of 2^14 vertices and the out-edges of each
+// destinations are cut into bins of 2^11 to 2^14 vertices and the out-edges of each
 // source into groups whose destinations share a bin.  Phase 1 writes one
 // value per group into per-bin runs; phase 2 streams each bin's 16-bit edge
 // entries and group values and adds them into LDS accumulators as 64-bit
@@ -59,6 +59,7 @@
 // line each, and the scatter costs more than they did; so it is opt-in.
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "advance.hpp"
 #include "apps.hpp"
@@ -71,11 +72,11 @@ constexpr int PB_BITS = 14;   // blocked layout: 16K destinations per bin
 // Exact pull: edges per thread (4 measured 7.3 us an iteration on RMAT s12, 8
 // measured 9.2), and the largest graphs that take it.  It gathers contrib
 // per edge, so it wants contrib in an XCD's 4 MB L2 (V <= 2^20), and its time
-// grows with E where the binned layout's starts at 20-70 us (us per iteration
-// exact / binned, the latter with 2^14-vertex bins: RMAT s12 7 / 25, s16 15 /
-// 65, s18 (7.6 M edges) 41 / 69, s19 79 / 80, s20 156 / 82).
+// grows with E faster than the binned layout's (us per iteration exact /
+// binned: RMAT s12 7.3 / 11.5, s14 9.1 / 12.7, s16 (1.8 M edges) 14.9 / 15.2,
+// s18 41 / 30; directed 50 K vertices, 594 K edges 9 / 12.5).
 constexpr int PX_EPT = 4;
-constexpr uint64_t PX_MAX_V = 1ull << 20, PX_MAX_E = 1ull << 23;
+constexpr uint64_t PX_MAX_V = 1ull << 20, PX_MAX_E = 1ull << 21;
 
 struct PrWork {
   Buf contrib[2], win_row, head_sum, tail_sum;
@@ -98,16 +99,20 @@ struct PrWork {
   // slot offset of every run; rbase = runs started before every slab;
   // val = group values (bin-major);
   // d2 = phase-2 edge stream (u16); gs512 = first group of every slab;
-  // task / multi = phase-2 tasks and the bins split over several tasks;
   // gacc = fixed-point sums of split bins (kept zero between iterations)
-  Buf bp_p1, bp_ch_u0, bp_ch_i0, bp_ch_r0, bp_rtab, bp_rbase, bp_val, bp_d2, bp_gs512, bp_task,
-      bp_multi, bp_gacc;
-  uint64_t bp_G = 0, bp_nch = 0, bp_ntask = 0, bp_nmulti = 0;
+  Buf bp_p1, bp_ch_u0, bp_ch_i0, bp_ch_r0, bp_rtab, bp_rbase, bp_val, bp_d2, bp_gs512, bp_gacc;
+  // phase-2 tasks and the bins split over several of them: PageRank's cut
+  // and the SSSP pull rounds'
+  struct Tasks {
+    Buf task, multi;
+    uint64_t ntask = 0, nmulti = 0;
+    uint64_t edges = 0;  // task size it was cut with (0: not cut)
+  } bp_pr, bp_sp;
+  uint64_t bp_G = 0, bp_nch = 0;
   uint32_t bp_nbins = 0;
   int bp_bits = 0;
   const void *bp_for = nullptr;
   std::vector<uint32_t> bp_bstart;  // first phase-2 edge of every bin (host)
-  uint64_t bp_task_edges = 0;       // task size the task table was cut with
   // SSSP pull rounds over the same layout: w2 = edge weights in phase-2
   // stream order (slab-transposed like d2); gmin = minima of the bins split
   // over several tasks (all 0xFFFFFFFF between rounds)
@@ -483,12 +488,15 @@ __global__ __launch_bounds__(BLOCK) void k_bp_scatter(const uint32_t *ch_u0, con
 // LDS accumulators as fixed-point integers, so the sums do not depend on
 // the order of the atomics.  A bin's only task finishes its rows; pieces of
 // split bins add their sums into gacc, which k_bp_finish completes.
-template <bool kLast>
+//
+// MAXB >= bits sizes the accumulators: with bins of 2^12 vertices two
+// workgroups fit a CU instead of one.
+template <bool kLast, int MAXB>
 __global__ __launch_bounds__(BP_BLOCK) void k_bp_accum(
     const BpTask *tasks, const uint16_t *d2, const uint32_t *gs512, const float *val, uint64_t V,
     int bits, const uint64_t *out_off, float *next, unsigned long long *gacc, float base,
     float alpha) {
-  __shared__ unsigned long long acc[1 << BP_MAX_BITS];
+  __shared__ unsigned long long acc[1 << MAXB];
   __shared__ float win[BP_BLOCK / WAVE][BP_SLAB];
   const BpTask t = tasks[blockIdx.x];
   const uint64_t v0 = (uint64_t)t.bin << bits;
@@ -558,7 +566,7 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_accum(
     if (sb >= t.e0 && sb + BP_SLAB <= t.e1) {  // wave-uniform: the whole slab is the task's
 #pragma unroll
       for (int q = 0; q < BP_EPT; q++)
-        atomicAdd(&acc[ent[q] & ((1u << BP_MAX_BITS) - 1u)], to_fixed(x[q]));
+        atomicAdd(&acc[ent[q] & ((1u << MAXB) - 1u)], to_fixed(x[q]));
     } else {
       // a slab shared with a neighbouring bin (or padding): entries outside
       // the task add zero; their destination bits stay inside the array
@@ -566,7 +574,7 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_accum(
       for (int q = 0; q < BP_EPT; q++) {
         const uint32_t pe = sb + WAVE * q + lane;
         const unsigned long long keep = 0ull - (unsigned long long)(pe >= t.e0 && pe < t.e1);
-        atomicAdd(&acc[ent[q] & ((1u << BP_MAX_BITS) - 1u)], to_fixed(x[q]) & keep);
+        atomicAdd(&acc[ent[q] & ((1u << MAXB) - 1u)], to_fixed(x[q]) & keep);
       }
     }
     // the window is rewritten by the next slab only after these reads
@@ -575,7 +583,7 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_accum(
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
   __syncthreads();
-  constexpr int R = (1 << BP_MAX_BITS) / BP_BLOCK;  // rows per thread at most
+  constexpr int R = (1 << MAXB) / BP_BLOCK;  // rows per thread at most
   if (!t.single) {
 #pragma unroll
     for (int r = 0; r < R; r++) {
@@ -593,18 +601,19 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_accum(
     }
   } else {
     // degrees of all the thread's rows are requested before any is used
+    constexpr int U = R < BP_UNROLL ? R : BP_UNROLL;
 #pragma unroll
-    for (int rb = 0; rb < R; rb += BP_UNROLL) {
-      uint64_t a[BP_UNROLL], b[BP_UNROLL];
+    for (int rb = 0; rb < R; rb += U) {
+      uint64_t a[U], b[U];
 #pragma unroll
-      for (int q = 0; q < BP_UNROLL; q++) {
+      for (int q = 0; q < U; q++) {
         const uint32_t i = threadIdx.x + BP_BLOCK * (rb + q);
         const uint64_t v = v0 + (i < nb ? i : nb - 1u);
         a[q] = out_off[v];
         b[q] = out_off[v + 1];
       }
 #pragma unroll
-      for (int q = 0; q < BP_UNROLL; q++) {
+      for (int q = 0; q < U; q++) {
         const uint32_t i = threadIdx.x + BP_BLOCK * (rb + q);
         if (i < nb) {
           const float rank = finish_row(from_fixed(acc[i]), base, alpha);
@@ -641,12 +650,11 @@ __global__ __launch_bounds__(BLOCK) void k_bp_finish(const uint32_t *mbins, int 
 // appends both lists with one global atomic each (a block scan of the
 // per-thread counts): an atomic per wave on the two counters serialised
 // ~10^5 waves per round.
-constexpr int BPR = (1 << BP_MAX_BITS) / BP_BLOCK;  // rows per thread at most
-static_assert(BPR <= 32, "row bits per thread");
-
-template <class Best>
+template <int MAXB, class Best>
 __device__ __forceinline__ void finish_rows(uint64_t v0, uint32_t nb, Best best_of,
                                             const BinnedMinArgs &a) {
+  constexpr int BPR = (1 << MAXB) / BP_BLOCK;  // rows per thread at most
+  static_assert(BPR >= 1 && BPR <= 32, "row bits per thread");
   constexpr uint32_t NW = BP_BLOCK / WAVE;
   __shared__ uint32_t s_w[NW];
   __shared__ uint32_t s_base[2];
@@ -739,12 +747,12 @@ struct W2Slab {
   }
 };
 
-template <typename WT, typename VT>
+template <int MAXB, typename WT, typename VT>
 __global__ __launch_bounds__(BP_BLOCK) void k_bp_min(const BpTask *tasks, const uint16_t *d2,
                                                      const WT *w2, const uint32_t *gs512,
                                                      const VT *val, uint64_t V, int bits,
                                                      BinnedMinArgs a, uint32_t *gmin) {
-  __shared__ uint32_t acc[1 << BP_MAX_BITS];
+  __shared__ uint32_t acc[1 << MAXB];
   __shared__ uint32_t win[BP_BLOCK / WAVE][BP_SLAB];
   const BpTask t = tasks[blockIdx.x];
   const uint64_t v0 = (uint64_t)t.bin << bits;
@@ -814,7 +822,7 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_min(const BpTask *tasks, const 
       const uint32_t pe = sb + WAVE * q + lane;
       const bool mine = whole || (pe >= t.e0 && pe < t.e1);
       if (mine && x[q] < INFINIT && c < INFINIT)
-        atomicMin(&acc[ent[q] & ((1u << BP_MAX_BITS) - 1u)], (uint32_t)c);
+        atomicMin(&acc[ent[q] & ((1u << MAXB) - 1u)], (uint32_t)c);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -823,23 +831,24 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_min(const BpTask *tasks, const 
   __syncthreads();
   if (!t.single) {  // block-uniform
 #pragma unroll
-    for (int r = 0; r < BPR; r++) {
+    for (int r = 0; r < (1 << MAXB) / BP_BLOCK; r++) {
       const uint32_t i = threadIdx.x + BP_BLOCK * r;
       if (i < nb && acc[i] != 0xFFFFFFFFu) atomicMin(&gmin[v0 + i], acc[i]);
     }
     return;
   }
-  finish_rows(v0, nb, [&](uint32_t i) { return acc[i]; }, a);
+  finish_rows<MAXB>(v0, nb, [&](uint32_t i) { return acc[i]; }, a);
 }
 
 // rows of the bins split over several tasks, one workgroup per bin; resets
 // gmin for the next round
+template <int MAXB>
 __global__ __launch_bounds__(BP_BLOCK) void k_bp_min_finish(const uint32_t *mbins, int bits,
                                                             uint64_t V, uint32_t *gmin,
                                                             BinnedMinArgs a) {
   const uint64_t v0 = (uint64_t)mbins[blockIdx.x] << bits;
   const uint32_t nb = (uint32_t)((V - v0) < (1ull << bits) ? (V - v0) : (1ull << bits));
-  finish_rows(v0, nb, [&](uint32_t i) {
+  finish_rows<MAXB>(v0, nb, [&](uint32_t i) {
     const uint32_t best = gmin[v0 + i];
     if (best != 0xFFFFFFFFu) gmin[v0 + i] = 0xFFFFFFFFu;
     return best;
@@ -1254,7 +1263,7 @@ bool build_blocked(Graph &g, PrWork &w, int bits) {
 //   phase 2  streams each bin's edges in (source, destination) order as
 //            u16 entries (group-start flag, destination in the bin) next to
 //            the bin's slice of val[], and adds the values into LDS
-//            accumulators.  Bins with more than BP_TASK_EDGES edges are
+//            accumulators.  Bins with more edges than a task are
 //            split into several tasks whose partial sums meet in gacc.
 // Every access of both phases is a sequential stream except the LDS
 // atomics, the reads of contrib inside one chunk's source range and the
@@ -1262,7 +1271,29 @@ bool build_blocked(Graph &g, PrWork &w, int bits) {
 // the graph does not fit the layout or the device lacks memory for the
 // build (peak ~ 40E + 16V bytes).
 constexpr uint32_t BP_CHUNK_GROUPS = 32768;
-constexpr uint64_t BP_TASK_EDGES = 1ull << 18;  // automatic task size
+
+// Automatic bin width and task sizes.  2^14-vertex bins leave a graph of V
+// vertices V / 2^14 bins to spread over 256 CUs; narrower bins make more and
+// smaller accumulators but more groups to write and read.  Tasks of E / 512
+// edges give every CU two, down to 2^14 edges (E / 128 below that), where a
+// task's own clearing and finishing shows, and up to a size of each use: the
+// bins of the largest graphs are split as little as fills the chip, because
+// every piece adds its whole bin to memory.  Measured on RMAT, ms per SSSP
+// run / us per PageRank iteration:
+//   s16  2^14 bins, 2^18 edges 0.95 / 65   2^11 and E/128 0.49 / 23
+//   s18  1.01 / 69                          2^11, 2^14 edges 0.63 / 42
+//   s20  1.14 / 84                          2^12 and E/512 0.92 / 78
+//   s21  - / 152                            2^12 and E/512 1.17 / 121
+//   s22  2.15 / 250                         2^13 and E/512 1.96 / 227
+//   s24  SSSP 2^14, 2^18 edges 6.28, 2^19 6.52; PageRank 1035, 2^19 956
+int automatic_bin_bits(uint64_t V) {
+  return V <= (1ull << 19) ? 11 : V <= (1ull << 21) ? 12 : V <= (1ull << 22) ? 13 : PB_BITS;
+}
+uint64_t automatic_task_edges(uint64_t E, uint64_t most) {
+  const uint64_t fill = std::max(E / 512, std::min<uint64_t>(E / 128, 1ull << 14));
+  return std::max<uint64_t>(256, std::min(fill, most));
+}
+constexpr uint64_t BP_TASK_PR = 1ull << 19, BP_TASK_SP = 1ull << 18;
 
 bool build_binned(Graph &g, PrWork &w, int bits) {
   Context &ctx = *g.ctx;
@@ -1275,9 +1306,10 @@ bool build_binned(Graph &g, PrWork &w, int bits) {
   GRUS_HIP(hipMemGetInfo(&free_b, &total_b));
   if (free_b < 48 * E + 16 * V + (1ull << 30)) return false;
   for (Buf *b : {&w.bp_p1, &w.bp_ch_u0, &w.bp_ch_i0, &w.bp_ch_r0, &w.bp_rtab, &w.bp_rbase,
-                 &w.bp_val, &w.bp_d2, &w.bp_gs512, &w.bp_task, &w.bp_multi, &w.bp_gacc,
-                 &w.bp_w2})
+                 &w.bp_val, &w.bp_d2, &w.bp_gs512, &w.bp_gacc, &w.bp_w2})
     b->release();
+  w.bp_pr = {};
+  w.bp_sp = {};
   w.bp_for = nullptr;
   w.bp_w2_for = nullptr;
   const unsigned rows_grid = grid_cap(ctx, V * WAVE, BLOCK);
@@ -1295,13 +1327,14 @@ bool build_binned(Graph &g, PrWork &w, int bits) {
                           ctx.stream));
   ctx.sync();
   const uint64_t G = (uint64_t)last[0] + last[1];
-  // groups per source (goff) -> phase-1 chunks, on the host (a source has
-  // at most nbins <= 8192 groups, so it always fits a chunk)
-  static const uint64_t chunk_groups = [] {
-    const char *e = getenv("GRUS_BP_CHUNK_GROUPS");  // experiments only
-    const long v = e ? atol(e) : 0;
-    return v >= (long)pr::BP_MAX_BINS ? (uint64_t)v : (uint64_t)BP_CHUNK_GROUPS;
-  }();
+  // groups per source (goff) -> phase-1 chunks, on the host (a source with
+  // more groups than a chunk takes is a chunk of its own: a chunk has at most
+  // nbins runs however many groups)
+  // Chunks of G / 512 groups, two workgroups per CU, between 4096 (whole
+  // slabs mostly) and BP_CHUNK_GROUPS.  RMAT, us per PageRank iteration with
+  // 32768 / G / 512 groups: s16 24 / 15, s18 37 / 30, s20 74 / 73; with G /
+  // 1024 groups s18 31, s20 76.
+  const uint64_t chunk_groups = std::max<uint64_t>(4096, std::min<uint64_t>(BP_CHUNK_GROUPS, G / 512));
   std::vector<uint32_t> ch_u0, ch_i0;
   {
     Buf goff;
@@ -1436,7 +1469,6 @@ bool build_binned(Graph &g, PrWork &w, int bits) {
   GRUS_HIP(hipMemsetAsync(w.bp_val.p, 0, (G + pr::BP_SLAB) * 4, ctx.stream));
   ctx.sync();  // host vectors above are copied before they go out of scope
   w.bp_bstart = std::move(bstart);
-  w.bp_task_edges = 0;
   w.bp_G = G;
   w.bp_nch = nch;
   w.bp_nbins = (uint32_t)nbins;
@@ -1447,7 +1479,7 @@ bool build_binned(Graph &g, PrWork &w, int bits) {
 
 // phase-2 tasks: every bin's edge range cut into equal pieces of at most
 // task_edges edges (an empty bin still gets one task: its rows are finished)
-void build_binned_tasks(Graph &g, PrWork &w, uint64_t task_edges) {
+void build_binned_tasks(Graph &g, PrWork &w, PrWork::Tasks &t, uint64_t task_edges) {
   Context &ctx = *g.ctx;
   std::vector<pr::BpTask> tasks;
   std::vector<uint32_t> multi;
@@ -1461,23 +1493,19 @@ void build_binned_tasks(Graph &g, PrWork &w, uint64_t task_edges) {
                                  (uint32_t)(e0 + n * (q + 1) / parts), (uint32_t)b,
                                  parts == 1 ? 1u : 0u});
   }
-  w.bp_task.alloc(tasks.size() * sizeof(pr::BpTask));
-  GRUS_HIP(hipMemcpyAsync(w.bp_task.p, tasks.data(), tasks.size() * sizeof(pr::BpTask),
+  t.task.alloc(tasks.size() * sizeof(pr::BpTask));
+  GRUS_HIP(hipMemcpyAsync(t.task.p, tasks.data(), tasks.size() * sizeof(pr::BpTask),
                           hipMemcpyHostToDevice, ctx.stream));
-  w.bp_multi.release();
+  t.multi.release();
   if (!multi.empty()) {
-    w.bp_multi.alloc(multi.size() * 4);
-    GRUS_HIP(hipMemcpyAsync(w.bp_multi.p, multi.data(), multi.size() * 4, hipMemcpyHostToDevice,
+    t.multi.alloc(multi.size() * 4);
+    GRUS_HIP(hipMemcpyAsync(t.multi.p, multi.data(), multi.size() * 4, hipMemcpyHostToDevice,
                             ctx.stream));
-    if (!w.bp_gacc.p) {
-      w.bp_gacc.alloc(g.V * 8);
-      GRUS_HIP(hipMemsetAsync(w.bp_gacc.p, 0, g.V * 8, ctx.stream));
-    }
   }
   ctx.sync();  // the host vectors are copied before they go out of scope
-  w.bp_ntask = tasks.size();
-  w.bp_nmulti = multi.size();
-  w.bp_task_edges = task_edges;
+  t.ntask = tasks.size();
+  t.nmulti = multi.size();
+  t.edges = task_edges;
 }
 
 // iterations over the binned push layout (graph already built for it)
@@ -1491,10 +1519,28 @@ void run_binned(Graph &g, PrWork &w, float alpha, int iters, grus_stats *st) {
   const float base = (float)((1.0 - (double)alpha) / (double)V);
   const int bits = w.bp_bits;
   const unsigned fin_grid =
-      (unsigned)(w.bp_nmulti * std::max<uint64_t>(1, (1ull << bits) / BLOCK));
+      (unsigned)(w.bp_pr.nmulti * std::max<uint64_t>(1, (1ull << bits) / BLOCK));
   float *contrib = w.contrib[0].as<float>();
-  const pr::BpTask *tasks = w.bp_task.as<const pr::BpTask>();
+  const pr::BpTask *tasks = w.bp_pr.task.as<const pr::BpTask>();
+  if (w.bp_pr.nmulti && !w.bp_gacc.p) {
+    w.bp_gacc.alloc(V * 8);
+    fill_u64(ctx, w.bp_gacc.as<uint64_t>(), V, 0);
+  }
   unsigned long long *gacc = w.bp_gacc.as<unsigned long long>();
+  // one of the accumulation kernels' sizes
+  auto accum = [&](auto last, float *next) {
+    constexpr bool kLast = decltype(last)::value;
+    const unsigned nt = (unsigned)w.bp_pr.ntask;
+    auto go = [&](auto maxb) {
+      pr::k_bp_accum<kLast, decltype(maxb)::value><<<nt, pr::BP_BLOCK, 0, ctx.stream>>>(
+          tasks, w.bp_d2.as<uint16_t>(), w.bp_gs512.as<uint32_t>(), w.bp_val.as<float>(), V, bits,
+          out.off, next, gacc, base, alpha);
+      GRUS_LAUNCH_CHECK();
+    };
+    if (bits <= 12) go(std::integral_constant<int, 12>());
+    else if (bits == 13) go(std::integral_constant<int, 13>());
+    else go(std::integral_constant<int, 14>());
+  };
   GRUS_HIP(hipEventRecord(ctx.ev0, ctx.stream));
   pr::k_init_contrib<<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(out.off, V, base, contrib);
   GRUS_LAUNCH_CHECK();
@@ -1515,24 +1561,18 @@ void run_binned(Graph &g, PrWork &w, float alpha, int iters, grus_stats *st) {
         pr::ContribValue{contrib}, w.bp_val.as<uint32_t>());
     GRUS_LAUNCH_CHECK();
     if (last) {
-      pr::k_bp_accum<true><<<(unsigned)w.bp_ntask, pr::BP_BLOCK, 0, ctx.stream>>>(
-          tasks, w.bp_d2.as<uint16_t>(), w.bp_gs512.as<uint32_t>(), w.bp_val.as<float>(), V, bits,
-          out.off, next, gacc, base, alpha);
-      GRUS_LAUNCH_CHECK();
-      if (w.bp_nmulti)
+      accum(std::true_type(), next);
+      if (w.bp_pr.nmulti)
         pr::k_bp_finish<true><<<fin_grid, BLOCK, 0, ctx.stream>>>(
-            w.bp_multi.as<uint32_t>(), bits, V, gacc, out.off, next, base, alpha);
+            w.bp_pr.multi.as<uint32_t>(), bits, V, gacc, out.off, next, base, alpha);
     } else {
-      pr::k_bp_accum<false><<<(unsigned)w.bp_ntask, pr::BP_BLOCK, 0, ctx.stream>>>(
-          tasks, w.bp_d2.as<uint16_t>(), w.bp_gs512.as<uint32_t>(), w.bp_val.as<float>(), V, bits,
-          out.off, next, gacc, base, alpha);
-      GRUS_LAUNCH_CHECK();
-      if (w.bp_nmulti)
+      accum(std::false_type(), next);
+      if (w.bp_pr.nmulti)
         pr::k_bp_finish<false><<<fin_grid, BLOCK, 0, ctx.stream>>>(
-            w.bp_multi.as<uint32_t>(), bits, V, gacc, out.off, next, base, alpha);
+            w.bp_pr.multi.as<uint32_t>(), bits, V, gacc, out.off, next, base, alpha);
     }
     GRUS_LAUNCH_CHECK();
-    launches += w.bp_nmulti ? 3 : 2;
+    launches += w.bp_pr.nmulti ? 3 : 2;
   }
   GRUS_HIP(hipEventRecord(ctx.ev1, ctx.stream));
   GRUS_HIP(hipEventSynchronize(ctx.ev1));
@@ -1672,15 +1712,18 @@ bool sssp_binned_ready(Graph &g) {
   PrWork &w = *g.pr;
   if (w.bp_unusable_for == out.off) return false;
   if (w.bp_for != out.off) {  // a layout PageRank already built is used as it is
-    const int bits = std::min(ctx.tuning.pr_bin_bits ? (int)ctx.tuning.pr_bin_bits : PB_BITS,
-                              pr::BP_MAX_BITS);
+    const int bits = std::min(
+        ctx.tuning.pr_bin_bits ? (int)ctx.tuning.pr_bin_bits : automatic_bin_bits(g.V),
+        pr::BP_MAX_BITS);
     if (!build_binned(g, w, bits)) {
       w.bp_unusable_for = out.off;
       return false;
     }
   }
-  if (w.bp_task_edges == 0)
-    build_binned_tasks(g, w, ctx.tuning.pr_task_edges ? ctx.tuning.pr_task_edges : BP_TASK_EDGES);
+  if (w.bp_sp.edges == 0)
+    build_binned_tasks(g, w, w.bp_sp,
+                       ctx.tuning.pr_task_edges ? ctx.tuning.pr_task_edges
+                                                : automatic_task_edges(g.E, BP_TASK_SP));
   if (w.bp_w2_for != out.off && !build_binned_weights(g, w)) {
     w.bp_unusable_for = out.off;
     return false;
@@ -1703,26 +1746,30 @@ void binned_min_launch(Graph &g, PrWork &w, const BinnedMinArgs &a, Src src) {
       w.bp_p1.as<uint16_t>(), w.bp_rbase.as<uint32_t>(), w.bp_rtab.as<uint32_t>(), w.bp_nbins,
       src, val);
   GRUS_LAUNCH_CHECK();
-  const pr::BpTask *tasks = w.bp_task.as<const pr::BpTask>();
+  const pr::BpTask *tasks = w.bp_sp.task.as<const pr::BpTask>();
   const uint16_t *d2 = w.bp_d2.as<uint16_t>();
   const uint32_t *gs = w.bp_gs512.as<uint32_t>();
   uint32_t *gmin = w.bp_gmin.as<uint32_t>();
-  const unsigned nt = (unsigned)w.bp_ntask;
-  if (w.bp_w2_bytes == 1)
-    pr::k_bp_min<<<nt, pr::BP_BLOCK, 0, ctx.stream>>>(tasks, d2, w.bp_w2.as<uint8_t>(), gs,
-                                                      (const VT *)val, g.V, bits, a, gmin);
-  else if (w.bp_w2_bytes == 2)
-    pr::k_bp_min<<<nt, pr::BP_BLOCK, 0, ctx.stream>>>(tasks, d2, w.bp_w2.as<uint16_t>(), gs,
-                                                      (const VT *)val, g.V, bits, a, gmin);
-  else
-    pr::k_bp_min<<<nt, pr::BP_BLOCK, 0, ctx.stream>>>(tasks, d2, w.bp_w2.as<uint32_t>(), gs,
-                                                      (const VT *)val, g.V, bits, a, gmin);
-  GRUS_LAUNCH_CHECK();
-  if (w.bp_nmulti) {
-    pr::k_bp_min_finish<<<(unsigned)w.bp_nmulti, pr::BP_BLOCK, 0, ctx.stream>>>(
-        w.bp_multi.as<uint32_t>(), bits, g.V, gmin, a);
-    GRUS_LAUNCH_CHECK();
-  }
+  const unsigned nt = (unsigned)w.bp_sp.ntask, nm = (unsigned)w.bp_sp.nmulti;
+  auto go = [&](auto maxb) {
+    constexpr int MAXB = decltype(maxb)::value;
+    auto min = [&](const auto *w2) {
+      pr::k_bp_min<MAXB><<<nt, pr::BP_BLOCK, 0, ctx.stream>>>(tasks, d2, w2, gs, (const VT *)val,
+                                                              g.V, bits, a, gmin);
+      GRUS_LAUNCH_CHECK();
+    };
+    if (w.bp_w2_bytes == 1) min(w.bp_w2.as<const uint8_t>());
+    else if (w.bp_w2_bytes == 2) min(w.bp_w2.as<const uint16_t>());
+    else min(w.bp_w2.as<const uint32_t>());
+    if (nm) {
+      pr::k_bp_min_finish<MAXB><<<nm, pr::BP_BLOCK, 0, ctx.stream>>>(
+          w.bp_sp.multi.as<uint32_t>(), bits, g.V, gmin, a);
+      GRUS_LAUNCH_CHECK();
+    }
+  };
+  if (bits <= 12) go(std::integral_constant<int, 12>());
+  else if (bits == 13) go(std::integral_constant<int, 13>());
+  else go(std::integral_constant<int, 14>());
 }
 }  // namespace
 
@@ -1766,11 +1813,12 @@ void run_pagerank(Graph &g, float alpha, int iters, grus_stats *st) {
   // binned push (automatic choice on HBM graphs that fit it; bins of at
   // most 2^14 destinations, the LDS accumulators)
   if ((layout == 0 || layout == 4) && g.placement == GRUS_PLACE_HBM) {
-    const int bb = std::min(bits, pr::BP_MAX_BITS);
+    const int bb = std::min(ctx.tuning.pr_bin_bits ? bits : automatic_bin_bits(V), pr::BP_MAX_BITS);
     bool binned = true;
     if (w.bp_for != out.off || w.bp_bits != bb) binned = build_binned(g, w, bb);
-    const uint64_t te = ctx.tuning.pr_task_edges ? ctx.tuning.pr_task_edges : BP_TASK_EDGES;
-    if (binned && w.bp_task_edges != te) build_binned_tasks(g, w, te);
+    const uint64_t te = ctx.tuning.pr_task_edges ? ctx.tuning.pr_task_edges
+                                                 : automatic_task_edges(g.E, BP_TASK_PR);
+    if (binned && w.bp_pr.edges != te) build_binned_tasks(g, w, w.bp_pr, te);
     if (binned) {
       run_binned(g, w, alpha, iters, st);
       return;

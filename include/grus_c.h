@@ -110,7 +110,7 @@ typedef struct grus_tuning {
                              mean degree); unweighted graphs: one bucket) */
   uint32_t pr_layout;     /* PageRank edge layout: 0 automatic (= 4 where it
                              applies, else 2; HBM graphs of at most 2^20
-                             vertices and 2^23 edges pull into 4's sums
+                             vertices and 2^21 edges pull into 4's sums
                              instead, with the same ranks, unless pr_bin_bits
                              or pr_task_edges is set); 1 degree-sorted relabelled copy
                              (symmetric HBM graphs); 2 plain pull over the
@@ -125,7 +125,8 @@ typedef struct grus_tuning {
                              (same ranks up to float rounding).  Every layout
                              is bit-identical run to run. */
   uint32_t pr_bin_bits;   /* blocked / binned layout bin width, log2 (0 =
-                             automatic: 14; layout 4 caps it at 14) */
+                             automatic: 14; layout 4: 11 to 14 by the number
+                             of vertices, at most 14) */
   uint32_t sssp_pull_div; /* SSSP: a round pulls (each unsettled vertex takes
                              the min over its in-neighbours in the frontier)
                              when the frontier's out-edges exceed
@@ -139,7 +140,8 @@ typedef struct grus_tuning {
                              round); 0 = automatic (256), at most 256 */
   uint32_t pr_task_edges; /* binned PageRank layout: edges per accumulation
                              task; a bin with more edges is split over several
-                             tasks (0 = automatic, 2^18) */
+                             tasks (0 = automatic: about E / 512, at most
+                             2^19; 2^18 for SSSP pull rounds) */
   uint32_t sssp_pull_layout; /* SSSP pull rounds: 0 automatic (= 2 where it
                              applies, else 1); 1 window reduction over the
                              in-edges; 2 binned push over PageRank's binned
