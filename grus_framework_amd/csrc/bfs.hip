@@ -34,6 +34,7 @@
 
 #include "advance.hpp"
 #include "apps.hpp"
+#include "bfs_all.hpp"
 #include "bfs_thin.hpp"
 
 namespace mgg {
@@ -48,7 +49,9 @@ struct BfsWork {
   Buf pad;                          // thin levels: padded rows of a low-degree graph
   uint32_t pad_deg = 0;             // columns per padded row
   const void *pad_for = nullptr;    // out-edge columns they were built from
-  Buf thin_flags;                   // their grid barrier's flags
+  Buf front2, all_flags;            // whole traversals: third bitmap, barrier flags
+  uint32_t all_tag = 0;             // their barrier tags handed out so far
+  Buf thin_flags;                   // thin levels: their grid barrier's flags
   uint32_t thin_tag = 0;            // level tags handed out so far
   PushWork push;
   uint64_t cap_v = 0;
@@ -609,12 +612,93 @@ const uint4 *thin_rows(Graph &g, BfsWork &w) {
 // workgroups of the cooperative thin kernel (0: it may not run here: under a
 // CU mask or beside other contexts its grid might not be resident)
 unsigned thin_grid(const Context &ctx) {
-  if (ctx.cu_masked || ctx.shared_device) return 0;
+  if (!ctx.cooperative()) return 0;
   int per_cu = 0;
   GRUS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
       &per_cu, reinterpret_cast<const void *>(bfs::k_thin<THIN_T, false>),
       bfs::thin_threads(THIN_T, false), 0));
   return std::min({THIN_BLOCKS, bfs::THIN_MAX_G, (unsigned)std::max(0, per_cu * ctx.cu_count)});
+}
+// workgroups of a whole traversal in one launch (0: it does not apply)
+unsigned all_grid(const Graph &g) {
+  const Context &ctx = *g.ctx;
+  const uint64_t W = g.words();
+  if (g.V > bfs::ALL_MAX_V || g.placement != GRUS_PLACE_HBM) return 0;
+  if (W <= bfs::ALL_OWN) return 1;  // one workgroup needs no grid barrier
+  const unsigned want = (unsigned)std::min<uint64_t>(bfs::ALL_MAX_G, div_up(W, 4));
+  if (!ctx.cooperative()) return 0;
+  // one per CU at most: resident
+  return div_up(W, ctx.cu_count) > bfs::ALL_OWN ? 0 : std::min(want, (unsigned)ctx.cu_count);
+}
+
+// a whole traversal in one launch (bfs_all.hpp); false when the runtime
+// refuses the launch
+bool run_bfs_all(Graph &g, BfsWork &w, uint32_t src, const CsrView &in, const uint32_t *first_in,
+                 const uint64_t *unreach, double alpha, double beta, uint32_t K, unsigned blocks,
+                 grus_stats *st) {
+  Context &ctx = *g.ctx;
+  const uint64_t W = g.words();
+  w.front2.ensure((W + 1) * 8);
+  constexpr uint64_t NF = 2 * 2 * bfs::ALL_MAX_G;
+  // a traversal takes at most V + 2 barriers
+  if (!w.all_flags.p || w.all_tag > (1u << 24) - 2 * bfs::ALL_MAX_V) {
+    w.all_flags.ensure(NF * 8);
+    fill_u64(ctx, w.all_flags.as<uint64_t>(), NF, 0);
+    w.all_tag = 0;
+  }
+  bfs::AllParams p{};
+  p.out = g.csr();
+  p.in = in;
+  p.first_in = first_in;
+  p.unreachable = unreach;
+  p.visited = w.visited.as<uint64_t>();
+  p.front[0] = w.front[0].as<uint64_t>();
+  p.front[1] = w.front[1].as<uint64_t>();
+  p.front[2] = w.front2.as<uint64_t>();
+  p.huge[0] = w.q[0].as<uint32_t>();
+  p.huge[1] = w.q[1].as<uint32_t>();
+  p.label = g.result.as<uint32_t>();
+  p.src = src;
+  p.K = K;
+  p.W = (uint32_t)W;
+  p.own = (uint32_t)div_up(W, blocks);
+  p.alpha = alpha;
+  p.beta = beta;
+  p.flags = w.all_flags.as<unsigned long long>();
+  p.tag = w.all_tag + 1;
+  p.ctl = reinterpret_cast<bfs::AllCtl *>(ctx.d_ctl.as<uint64_t>() + 8);
+  p.timeout = ctx.wall_ticks_per_ms() * 20000;  // 20 s per barrier wait
+  const size_t lds = (W + 2 * p.own) * 8;
+  GRUS_HIP(hipEventRecord(ctx.ev0, ctx.stream));
+  if (blocks == 1) {
+    bfs::k_bfs_all<<<1, bfs::ALL_T, lds, ctx.stream>>>(p);
+    GRUS_LAUNCH_CHECK();
+  } else {
+    void *args[] = {&p};
+    if (!ctx.launch_cooperative(reinterpret_cast<const void *>(bfs::k_bfs_all), blocks, bfs::ALL_T,
+                                args, lds))
+      return false;
+  }
+  GRUS_HIP(hipEventRecord(ctx.ev1, ctx.stream));
+  ctx.publish_ctl(8 + sizeof(bfs::AllCtl) / 8);
+  bfs::AllCtl r;
+  std::memcpy(&r, ctx.h_ctl + 8, sizeof r);
+  w.all_tag += std::min<uint32_t>(r.levels, (uint32_t)bfs::ALL_MAX_V) + 2;
+  if (r.status) raise(GRUS_E_TIMEOUT, "bfs aborted (barrier timeout)");
+  if (r.levels == 0 || r.levels > g.V + 1 || r.v_reached > g.V)
+    raise(GRUS_E_HIP, "bfs reported an impossible state");
+  if (st) {
+    float ms = 0;
+    GRUS_HIP(hipEventElapsedTime(&ms, ctx.ev0, ctx.ev1));
+    *st = grus_stats{};
+    st->device_ms = ms;
+    st->iterations = r.levels;
+    st->pull_iterations = r.pulls;
+    st->vertices_reached = r.v_reached;
+    st->edges_reached = r.e_reached;
+    st->kernel_launches = 1;
+  }
+  return true;
 }
 }  // namespace
 
@@ -656,6 +740,10 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
   const double beta = ctx.tuning.bfs_beta > 0 ? ctx.tuning.bfs_beta : 64.0;
   const uint32_t K = ctx.tuning.bu_thread_edges ? ctx.tuning.bu_thread_edges : 32;
 
+  const uint4 *thin = dir == GRUS_DIR_PULL ? nullptr : thin_rows(g, w);
+  if (const unsigned blocks = dir == GRUS_DIR_AUTO && !thin ? all_grid(g) : 0) {
+    if (run_bfs_all(g, w, src, in, first_in, unreach, alpha, beta, K, blocks, st)) return;
+  }
   uint64_t src_deg = 0;
   {
     uint64_t o[2];
@@ -682,8 +770,7 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
   // instead of every bitmap word; the host knows how many are left from
   // the vertices reached so far and the in-degree-0 count
   const uint64_t n_unreach = unreach ? g.unreachable_count : 0;
-  const uint4 *thin = dir == GRUS_DIR_PULL ? nullptr : thin_rows(g, w);
-  const unsigned thin_blocks = thin ? thin_grid(ctx) : 0;
+  unsigned thin_blocks = thin ? thin_grid(ctx) : 0;
   // GRUS_TRACE=1 prints one line per level (mode, frontier, host time)
   static const bool trace = getenv("GRUS_TRACE") != nullptr;
   auto t_level = std::chrono::steady_clock::now();
@@ -770,9 +857,11 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
           GRUS_LAUNCH_CHECK();
         } else {
           void *args[] = {&p};
-          GRUS_HIP(hipLaunchCooperativeKernel(
-              reinterpret_cast<const void *>(bfs::k_thin<THIN_T, false>), dim3(thin_blocks),
-              dim3(bfs::thin_threads(THIN_T, false)), args, 0, ctx.stream));
+          if (!ctx.launch_cooperative(reinterpret_cast<const void *>(bfs::k_thin<THIN_T, false>),
+                                      thin_blocks, bfs::thin_threads(THIN_T, false), args, 0)) {
+            thin_blocks = 0;  // this level is launched below
+            continue;
+          }
         }
         launches++;
         ctx.publish_ctl(8 + sizeof(bfs::ThinCtl) / 8);

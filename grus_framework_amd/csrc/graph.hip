@@ -171,6 +171,16 @@ void Context::set_cu_mask(const uint32_t *mask, uint32_t words) {
   cu_count = words ? n : cu_total;
 }
 
+bool Context::launch_cooperative(const void *kernel, unsigned blocks, unsigned threads,
+                                 void **args, size_t lds) {
+  if (hipLaunchCooperativeKernel(kernel, dim3(blocks), dim3(threads), args, (unsigned)lds,
+                                 stream) == hipSuccess)
+    return true;
+  (void)hipGetLastError();
+  coop_refused = true;
+  return false;
+}
+
 namespace {
 __global__ void k_publish_ctl(uint64_t *d, uint64_t *h, uint32_t n) {
   const uint32_t i = threadIdx.x;

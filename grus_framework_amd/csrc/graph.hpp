@@ -94,6 +94,9 @@ struct Context {
   // other contexts run kernels on the device at the same time (server
   // workers): no cooperative persistent launches, whose grid must be resident
   bool shared_device = false;
+  // set once the runtime has refused a cooperative launch (another process
+  // may hold the device's one cooperative queue): not asked again
+  bool coop_refused = false;
   int wall_khz = 100000;  // device wall clock rate (wall_clock64 ticks per ms)
   grus_tuning tuning{};
   uint64_t *h_ctl = nullptr;  // pinned host mirror of the control block
@@ -109,6 +112,13 @@ struct Context {
   // zeroes them on the device; then wait.  Replaces a copy and the next
   // step's memset (two launches) in per-level read-backs.
   void publish_ctl(size_t n);
+  // whether cooperative grids may be launched: under a CU mask or beside other
+  // contexts' kernels a grid might not be resident
+  bool cooperative() const { return !cu_masked && !shared_device && !coop_refused; }
+  // launches a cooperative grid on the stream; false when the runtime refuses
+  // (the caller then takes its other path)
+  bool launch_cooperative(const void *kernel, unsigned blocks, unsigned threads, void **args,
+                          size_t lds);
   // replace the stream by one restricted to the CUs set in mask (words == 0:
   // all CUs); waits for the old stream first
   void set_cu_mask(const uint32_t *mask, uint32_t words);

@@ -805,8 +805,9 @@ uint32_t pick_delta(Graph &g, SsspWork &w, bool persistent) {
 }  // namespace
 
 namespace {
-// one cooperative launch for the whole traversal (low max degree)
-void run_sssp_persistent(Graph &g, SsspWork &w, uint32_t src, uint64_t delta, uint64_t *rounds,
+// one cooperative launch for the whole traversal (low max degree); false
+// when the runtime refuses it
+bool run_sssp_persistent(Graph &g, SsspWork &w, uint32_t src, uint64_t delta, uint64_t *rounds,
                          uint64_t *passes) {
   Context &ctx = *g.ctx;
   const uint64_t V = g.V;
@@ -871,8 +872,9 @@ void run_sssp_persistent(Graph &g, SsspWork &w, uint32_t src, uint64_t delta, ui
   unsigned want = env_blocks > 0 ? (unsigned)env_blocks : (unsigned)std::max(1, ctx.cu_count / 2);
   unsigned grid = std::max(1u, std::min(want, (unsigned)(ctx.cu_count * per_cu)));
   void *args[] = {&p};
-  GRUS_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(sssp::k_persistent),
-                                      dim3(grid), dim3(BLOCK), args, 0, ctx.stream));
+  if (!ctx.launch_cooperative(reinterpret_cast<const void *>(sssp::k_persistent), grid, BLOCK, args,
+                              0))
+    return false;
   sssp::PCtl out;
   GRUS_HIP(hipMemcpyAsync(&out, w.pctl.p, sizeof out, hipMemcpyDeviceToHost, ctx.stream));
   ctx.sync();
@@ -880,6 +882,7 @@ void run_sssp_persistent(Graph &g, SsspWork &w, uint32_t src, uint64_t delta, ui
   *rounds = out.rounds;
   *passes = out.passes;
   if (out.status) raise(GRUS_E_TIMEOUT, "persistent sssp aborted (barrier timeout or round cap)");
+  return true;
 }
 }  // namespace
 
@@ -903,7 +906,7 @@ void run_sssp(Graph &g, uint32_t src, grus_stats *st) {
   // (not under a CU mask: a cooperative grid must be co-resident, and the
   // runtime's residency check does not know the mask; nor beside other
   // contexts' kernels)
-  const bool persistent = g.max_deg <= 32 && !no_persist && !ctx.cu_masked && !ctx.shared_device;
+  const bool persistent = g.max_deg <= 32 && !no_persist && ctx.cooperative();
   const uint64_t delta = pick_delta(g, w, persistent);
   // a round pulls when its frontier's out-edges exceed E / pull_div
   // (automatic: 16, measured best of 4..128 on RMAT s24; 0xFFFFFFFF: never)
@@ -931,7 +934,10 @@ void run_sssp(Graph &g, uint32_t src, grus_stats *st) {
   GRUS_LAUNCH_CHECK();
   launches++;
   if (persistent) {
-    run_sssp_persistent(g, w, src, delta, &rounds, &local_passes);
+    if (!run_sssp_persistent(g, w, src, delta, &rounds, &local_passes)) {
+      run_sssp(g, src, st);  // (the context now knows: the host-driven path)
+      return;
+    }
     launches++;
   }
   int cur = 0, fcur = 0;
