@@ -1098,7 +1098,6 @@ void MsEngine::copy_out(int slot0, int n, uint32_t *host_out) {
   if (kind_ == MsKind::BFS) {  // the rows lie one behind the other
     GRUS_HIP(hipMemcpyAsync(host_out, vals_.as<uint32_t>() + (uint64_t)slot0 * V,
                             (uint64_t)n * V * 4, hipMemcpyDeviceToHost, ctx.stream));
-    ctx.sync();
     return;
   }
   // as many rows at a time as ROWS_OUT bytes hold, from a buffer kept with
@@ -1126,7 +1125,6 @@ void MsEngine::copy_out(int slot0, int n, uint32_t *host_out) {
     GRUS_HIP(hipMemcpyAsync(host_out + at * V, stage, (uint64_t)m * V * 4, hipMemcpyDeviceToHost,
                             ctx.stream));
   }
-  ctx.sync();
 }
 
 void MsEngine::release(int slot) {
@@ -1172,6 +1170,7 @@ void run_multi(Graph &g, MsKind kind, const uint32_t *srcs, int k, uint32_t *out
       e.copy_out(slots[i], j - i, out + (uint64_t)i * g.V);
       i = j;
     }
+    ctx.sync();
   }
   for (int sl : slots) e.release(sl);
   if (st) {

@@ -80,7 +80,8 @@ class MsEngine {
   void digest(SlotMask mask, uint64_t *reached, uint64_t *checksum);
   // finite entries of the slots in mask, all together
   uint64_t reached(SlotMask mask);
-  // the rows of slots [slot0, slot0 + n), n * V u32, to host memory
+  // the rows of slots [slot0, slot0 + n), n * V u32, to host memory: queued on
+  // the engine's stream, done once the caller has synchronised it
   void copy_out(int slot0, int n, uint32_t *host_out);
   void release(int slot);  // slot becomes free (reset lazily at next admit)
   Context &ctx() { return *ctx_; }

@@ -17,8 +17,7 @@
 // step per level whatever it holds.  Load is light while the engines of a
 // kind, each serving one query at a time, would empty the queue within the
 // time of one batch (running means of both times, per kind; until a batch
-// has run, a batch is taken to cost 32 single queries, about what one of 64
-// lanes costs on RMAT graphs), or while at most solo_max queries wait when
+// has run, 16 waiting queries start one, so that its time is known), or while at most solo_max queries wait when
 // the caller sets it.  Measured on RMAT scale 22 at 1100 queries/s (50/50
 // BFS/SSSP): p50 5 ms when every query is served alone, 99-120 ms when a
 // queue of 8 already starts a batch (which then slows the single queries
@@ -63,6 +62,14 @@ double now_us() {
   return (double)duration_cast<nanoseconds>(steady_clock::now().time_since_epoch()).count() /
          1e3;
 }
+
+// Waiting queries of a kind that start the first batch of that kind.  What a
+// batch costs next to single queries depends on the graph: as much as 32 of
+// them on RMAT scale 22, as two or three at scale 16, where a single query is
+// mostly launches.  Taken to cost 32 until one had run, 128 queries at scale
+// 16 were all served alone and no batch ever ran (256 mixed queries 23-35 ms;
+// 8.4 ms with the first batch started at 16).
+constexpr size_t kLearnBatch = 16;
 
 struct Query {
   uint64_t id;
@@ -381,10 +388,16 @@ class ServerImpl : public Server {
         // pass over the engine's state) and reported at once
         uint64_t reached[128], checksum[128];
         eng->digest(done, reached, checksum);
+        if (opts_.copy_results) {  // every copy in flight, then one wait
+          for (SlotMask m = done; m; m &= m - 1) {
+            const int sl = slot_lowest(m);
+            if (slot_q[sl].out) eng->copy_out(sl, 1, slot_q[sl].out);
+          }
+          eng->ctx().sync();
+        }
         for (SlotMask m = done; m; m &= m - 1) {
           const int sl = slot_lowest(m);
           const Query &q = slot_q[sl];
-          if (opts_.copy_results && q.out) eng->copy_out(sl, 1, q.out);
           eng->release(sl);
           finish(q, GRUS_OK, reached[sl], checksum[sl]);
         }
@@ -447,8 +460,8 @@ class ServerImpl : public Server {
     const size_t n = pending_[kind].size();
     if (n == 0) return false;
     if (opts_.solo_max > 0 || solo_ms_[kind] <= 0) return (int)n <= solo_max_;
-    const double batch = batch_ms_[kind] > 0 ? batch_ms_[kind] : 32 * solo_ms_[kind];
-    return (double)n * solo_ms_[kind] <= opts_.max_inflight_batches * batch;
+    if (batch_ms_[kind] <= 0) return n < kLearnBatch;
+    return (double)n * solo_ms_[kind] <= opts_.max_inflight_batches * batch_ms_[kind];
   }
 
   // running mean (weight 1/8 to the newest), 0 = nothing measured yet
