@@ -391,6 +391,34 @@ __global__ void k_transpose_keys(const uint64_t *off, const uint32_t *col, uint6
       keys[e] = ((uint64_t)col[e] << 32) | u;
 }
 
+// Sum over the edges of h(u, v, w) - h(v, u, w) for a hash h of 64 bits: 0 if
+// the edges are their own reverses, weights included, and by a chance of
+// 2^-64 otherwise.  A lane walks a short row, the wave a long one together.
+__device__ __forceinline__ uint64_t edge_hash(uint32_t u, uint32_t v, uint32_t w) {
+  return mix64(mix64(((uint64_t)u << 32) | v) + w);
+}
+__global__ void k_mirror_sum(const uint64_t *off, const uint32_t *col, const uint32_t *w,
+                             uint64_t V, unsigned long long *sum) {
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  const uint32_t lane = lane_id();
+  unsigned long long s = 0;
+  for (uint64_t b = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x - lane; b < V; b += stride) {
+    const uint64_t u = b + lane;
+    const uint64_t e0 = u < V ? off[u] : 0, e1 = u < V ? off[u + 1] : 0;
+    const bool is_long = e1 - e0 > 32;
+    for (uint64_t e = e0; e < e1 && !is_long; e++)
+      s += edge_hash((uint32_t)u, col[e], w[e]) - edge_hash(col[e], (uint32_t)u, w[e]);
+    for (uint64_t m = __ballot(is_long); m; m &= m - 1) {
+      const int l = __ffsll((unsigned long long)m) - 1;
+      const uint64_t a = __shfl(e0, l), z = __shfl(e1, l);
+      for (uint64_t e = a + lane; e < z; e += WAVE)
+        s += edge_hash((uint32_t)(b + l), col[e], w[e]) - edge_hash(col[e], (uint32_t)(b + l), w[e]);
+    }
+  }
+  s = wave_sum(s);
+  if (lane == 0 && s) atomicAdd(sum, s);
+}
+
 __global__ void k_iota_u32(uint32_t *a, uint64_t n) {
   uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
   uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -502,6 +530,21 @@ const uint64_t *Graph::unreachable() {
   return unreachable_bm.as<const uint64_t>();
 }
 
+bool Graph::weights_mirror() {
+  if (mirror < 0 && !weighted) mirror = 1;
+  if (mirror < 0) {
+    auto *sum = reinterpret_cast<unsigned long long *>(ctx->d_ctl.p);
+    GRUS_HIP(hipMemsetAsync(sum, 0, 8, ctx->stream));
+    k_mirror_sum<<<grid_for(ctx, V), BLOCK, 0, ctx->stream>>>(
+        off.as<uint64_t>(), col.as<uint32_t>(), w.as<uint32_t>(), V, sum);
+    GRUS_LAUNCH_CHECK();
+    ctx->read_ctl(1);
+    mirror = ctx->h_ctl[0] == 0;
+    GRUS_HIP(hipMemsetAsync(sum, 0, 8, ctx->stream));
+  }
+  return mirror == 1;
+}
+
 Graph::~Graph() {
   if (ctx) (void)hipSetDevice(ctx->device);
 }
@@ -509,11 +552,13 @@ Graph::~Graph() {
 std::unique_ptr<Graph> graph_view(Graph &g, Context *ctx) {
   g.csc();          // directed graphs: the in-edges, built once on g
   g.unreachable();  // the in-degree-0 bitmap
+  if (g.symmetric && g.placement == GRUS_PLACE_HBM) g.weights_mirror();
   auto v = std::make_unique<Graph>(ctx);
   v->V = g.V;
   v->E = g.E;
   v->weighted = g.weighted;
   v->symmetric = g.symmetric;
+  v->mirror = g.mirror;
   v->placement = g.placement;
   v->split = g.split;
   v->max_deg_vertex = g.max_deg_vertex;

@@ -164,6 +164,7 @@ struct Graph {
   uint64_t isolated = 0;
   Buf unreachable_bm;  // bit v set: in-degree 0 (never discovered by a traversal)
   bool unreachable_ready = false;
+  int mirror = -1;  // weights_mirror(), once it has been found out
   uint64_t unreachable_count = 0;  // vertices with in-degree 0 (set by unreachable())
   uint64_t host_bytes = 0;
   // workspaces and last result
@@ -186,6 +187,9 @@ struct Graph {
   uint64_t words() const { return (V + 63) / 64; }
   void compute_derived();         // max degree vertex, isolated count
   const uint64_t *unreachable();  // in-degree-0 bitmap (builds CSC if directed)
+  // a graph declared symmetric: the weight of every edge is its reverse's too
+  // (looked at once; always so without weights)
+  bool weights_mirror();
   uint64_t device_bytes() const;
 };
 

@@ -25,6 +25,15 @@ namespace mgg {
 
 namespace ms {
 
+// *word |= bits, for a word that every wave of a launch sets: atomics on one
+// address run one after the other, so a wave whose bits are there already
+// leaves it at a read (130000 waves that did not: 8.5 ms for a batch at scale
+// 18 where it now takes 4.5).
+__device__ __forceinline__ void or_bits(uint64_t *word, uint64_t bits) {
+  auto *p = (unsigned long long *)word;
+  if (bits & ~__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(p, bits);
+}
+
 constexpr uint32_t K_PULL = 32;
 constexpr uint32_t CHUNK = 64;       // SSSP relax: out-edges per wave task (one per lane)
 #ifndef SSSP_SPARSE_LANES
@@ -237,7 +246,7 @@ __global__ __launch_bounds__(BLOCK) void k_bfs_finalize(const uint64_t *off, uin
     }
   }
   __syncthreads();
-  if (threadIdx.x == 0 && s_alive) atomicOr((unsigned long long *)&cnt->alive, s_alive);
+  if (threadIdx.x == 0) or_bits(&cnt->alive, s_alive);
   block_add_u64(edges, (unsigned long long *)&cnt->front_edges);
 }
 
@@ -466,16 +475,269 @@ __global__ __launch_bounds__(BLOCK) void k_sssp_relax(CsrView g, const uint32_t 
   imp_a = wave_or(imp_a) | __ballot(dimp_a);
   imp_b = wave_or(imp_b) | __ballot(dimp_b);
   if (lane == 0) {
-    if (imp_a) atomicOr((unsigned long long *)&cnt->slot_alive[0], imp_a);
-    if (imp_b) atomicOr((unsigned long long *)&cnt->slot_alive[1], imp_b);
+    or_bits(&cnt->slot_alive[0], imp_a);
+    or_bits(&cnt->slot_alive[1], imp_b);
   }
   if (NARROW) {
     ovf_a = wave_or(ovf_a) | __ballot(dovf_a);
     ovf_b = wave_or(ovf_b) | __ballot(dovf_b);
     if (lane == 0) {
-      if (ovf_a) atomicOr((unsigned long long *)&cnt->overflow[0], ovf_a);
-      if (ovf_b) atomicOr((unsigned long long *)&cnt->overflow[1], ovf_b);
+      or_bits(&cnt->overflow[0], ovf_a);
+      or_bits(&cnt->overflow[1], ovf_b);
     }
+  }
+}
+
+// The same step from the other side, for frontiers that cover much of the
+// graph: a wave takes PULL_EDGES in-edges (more on very dense graphs) and,
+// row by row, the minimum over the in-neighbours on the frontier of their
+// distances plus the weight, in registers (16-bit entries: one saturating
+// packed add and one packed minimum for two queries).  A push reads the row
+// of every out-edge's head and lowers it with a compare-and-swap; here a row
+// is read and written once, with a plain store when all its edges are the
+// workgroup's (a row that workgroups share is lowered as a push does).  Lanes
+// whose queries have no frontier at the in-neighbour read nothing.
+// Bound by the row reads, 256 bytes per edge: RMAT scale 18, 8 M edges, 128
+// queries 393..470 us for the dense steps (4.5..5.3 TB/s, mostly out of the
+// caches), push 1080..1363; scale 16 128..161 us against 271..439.  64 edges
+// a wave: 4.43 ms for the batch at scale 18, 4.67 with 128, 5.1 with 256 (a
+// row's end and its share of the latency weigh more than the start of a
+// wave); 1, 2, 4, 8 and 16 waves a workgroup 4.86, 4.51, 4.44, 4.62, 5.4.
+// 32-bit entries have 4 rows in flight: 8.9 ms, and 10.4 with 8 (registers).
+constexpr uint32_t PULL_EDGES = 64;
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+constexpr uint32_t PULL_WAVES = 4;  // waves of a workgroup
+
+// entries of two queries: the pair a lane holds
+template <bool NARROW>
+struct Pair;
+template <>
+struct Pair<true> {
+  uint32_t x;  // two 16-bit entries
+  static __device__ __forceinline__ Pair inf() { return {0xFFFFFFFFu}; }
+  static __device__ __forceinline__ Pair load(const uint32_t *dist, uint64_t v, uint32_t p) {
+    return {(dist + v * 64)[p]};
+  }
+  __device__ __forceinline__ Pair plus(uint32_t w) const {  // w <= 0xFFFF; saturates at "unreached"
+    const u16x2 a = __builtin_bit_cast(u16x2, x), b = {(uint16_t)w, (uint16_t)w};
+    return {__builtin_bit_cast(uint32_t, __builtin_elementwise_add_sat(a, b))};
+  }
+  __device__ __forceinline__ Pair min(Pair o) const {
+    return {__builtin_bit_cast(uint32_t,
+                               __builtin_elementwise_min(__builtin_bit_cast(u16x2, x),
+                                                         __builtin_bit_cast(u16x2, o.x)))};
+  }
+  __device__ __forceinline__ uint32_t a() const { return x & 0xFFFFu; }
+  __device__ __forceinline__ uint32_t b() const { return x >> 16; }
+};
+template <>
+struct Pair<false> {
+  uint32_t xa, xb;
+  static __device__ __forceinline__ Pair inf() { return {INFINIT, INFINIT}; }
+  static __device__ __forceinline__ Pair load(const uint32_t *dist, uint64_t v, uint32_t p) {
+    const uint2 y = reinterpret_cast<const uint2 *>(dist)[v * 64 + p];
+    return {y.x, y.y};
+  }
+  static __device__ __forceinline__ uint32_t add(uint32_t d, uint32_t w) {
+    const uint64_t s = (uint64_t)d + w;
+    return s < INFINIT ? (uint32_t)s : INFINIT;
+  }
+  __device__ __forceinline__ Pair plus(uint32_t w) const { return {add(xa, w), add(xb, w)}; }
+  __device__ __forceinline__ Pair min(Pair o) const {
+    return {xa < o.xa ? xa : o.xa, xb < o.xb ? xb : o.xb};
+  }
+  __device__ __forceinline__ uint32_t a() const { return xa; }
+  __device__ __forceinline__ uint32_t b() const { return xb; }
+};
+
+// first[i]: the row that holds in-edge i * per
+__global__ void k_pull_first(const uint64_t *off, uint64_t V, uint32_t per, uint64_t n,
+                             uint32_t *first) {
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n;
+       i += (uint64_t)gridDim.x * blockDim.x) {
+    uint64_t lo = 0, hi = V;  // off[lo] <= i * per < off[hi]
+    while (hi - lo > 1) {
+      const uint64_t mid = (lo + hi) / 2;
+      if (off[mid] <= i * per) lo = mid;
+      else hi = mid;
+    }
+    first[i] = (uint32_t)lo;
+  }
+}
+
+template <bool NARROW>
+__global__ __launch_bounds__(PULL_WAVES * WAVE) void k_sssp_pull(CsrView in, uint32_t per,
+                                                                 const uint32_t *first,
+                                                                 const uint64_t *front,
+                                                                 uint64_t *next, uint32_t *dist,
+                                                                 MsCounters *cnt) {
+  using P = Pair<NARROW>;
+  // what a wave holds of the row it shares with the wave before it (head)
+  // and of the row it shares with the wave after it (tail)
+  __shared__ P s_acc[2][PULL_WAVES][WAVE], s_low[2][PULL_WAVES][WAVE];
+  __shared__ uint32_t s_row[2][PULL_WAVES];  // that row, or INFINIT
+  __shared__ uint32_t s_span[PULL_WAVES];    // the head's row goes on past the wave
+  constexpr uint32_t INF = NARROW ? INF16 : INFINIT;
+  const uint32_t lane = lane_id();
+  const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const uint64_t g0 = blockIdx.x * (uint64_t)PULL_WAVES * per;  // the workgroup's edges
+  const uint64_t e0 = g0 + (uint64_t)wv * per, e1 = e0 + per < in.E ? e0 + per : in.E;
+  uint64_t imp_a = 0, imp_b = 0, ovf_a = 0, ovf_b = 0;  // bit p: lane p's slot
+  // lowers row r to acc; `whole`: no other wave holds edges of the row
+  auto finish = [&](uint64_t r, bool whole, P cur, P acc, P low) {
+    const P res = cur.min(acc);
+    const bool ia = res.a() < cur.a(), ib = res.b() < cur.b();
+    if (NARROW) {  // a finite distance plus a weight that 16 bits do not hold
+      ovf_a |= __ballot(res.a() == INF) & __ballot(low.a() != INF);
+      ovf_b |= __ballot(res.b() == INF) & __ballot(low.b() != INF);
+    }
+    const uint64_t ba = __ballot(ia), bb = __ballot(ib), m = ba | bb;
+    imp_a |= ba;
+    imp_b |= bb;
+    if (!m) return;
+    if (lane == 0) {
+      if (whole) next[r] = m;
+      else atomicOr((unsigned long long *)&next[r], (unsigned long long)m);
+    }
+    if constexpr (NARROW) {
+      uint32_t *wp = &dist[r * 64 + lane];
+      if (whole) {
+        if (ia || ib) *wp = res.x;
+      } else {
+        if (ia) cas_min16(wp, 0, res.a(), cur.x);
+        if (ib) cas_min16(wp, 1, res.b(), *wp);
+      }
+    } else {
+      uint32_t *pp = &dist[(r * 64 + lane) * 2];
+      if (whole) {
+        if (ia) pp[0] = res.xa;
+        if (ib) pp[1] = res.xb;
+      } else {
+        if (ia) atomicMin(pp, res.xa);
+        if (ib) atomicMin(pp + 1, res.xb);
+      }
+    }
+  };
+  if (lane == 0) {
+    s_row[0][wv] = s_row[1][wv] = INFINIT;
+    s_span[wv] = 0;
+  }
+  if (e0 < e1) {
+    // the row that holds edge e0, and the ends of it and the next 63 rows
+    uint64_t r = first[blockIdx.x * PULL_WAVES + wv], rb = r;
+    uint64_t w_end = in.off[rb + 1 + lane < in.V ? rb + 1 + lane : in.V];
+    const uint32_t r0 = (uint32_t)r;
+    const bool shared0 = in.off[r] < e0;
+    if (shared0) s_acc[0][wv][lane] = s_low[0][wv][lane] = P::inf();
+    uint32_t open = INFINIT;  // the row that cur, acc and low belong to
+    P cur = P::inf(), acc = cur, low = cur;  // low: the least distance a weight was added to
+    auto close = [&]() {      // the open row has no more edges here
+      if (open == INFINIT) return;
+      if (shared0 && open == r0) {
+        s_acc[0][wv][lane] = acc;
+        s_low[0][wv][lane] = low;
+        if (lane == 0) s_row[0][wv] = r0;
+      } else {
+        finish(open, true, cur, acc, low);
+      }
+    };
+    for (uint64_t base = e0; base < e1; base += WAVE) {
+      const uint32_t n = (uint32_t)(e1 - base < WAVE ? e1 - base : WAVE);
+      const bool valid = lane < n;
+      const uint32_t my_u = valid ? edge_col(in, base + lane) : 0u;
+      uint32_t my_w = valid ? edge_w(in, base + lane) : 0u;
+      if (NARROW) my_w = my_w < 0xFFFFu ? my_w : 0xFFFFu;
+      const uint64_t my_f = valid ? front[my_u] : 0ull;
+      uint64_t act = __ballot(my_f != 0);
+      // the row of each edge, and the first active edge of each row
+      uint32_t my_r = 0, pos = 0;
+      uint64_t heads = 0;
+      while (pos < n) {
+        const uint64_t row_end = readlane_u64(w_end, (uint32_t)(r - rb));
+        const uint32_t seg = row_end - base < n ? (uint32_t)(row_end - base) : n;
+        if (lane >= pos) my_r = (uint32_t)r;
+        uint64_t m = (act >> pos) << pos;
+        if (seg < 64) m &= (1ull << seg) - 1ull;
+        heads |= m & -m;
+        pos = seg;
+        if (base + pos != row_end || base + pos >= e1) break;
+        do {  // the next row with edges (there is one: e1 <= E)
+          r++;
+          if (r - rb >= WAVE) {
+            rb = r;
+            w_end = in.off[rb + 1 + lane < in.V ? rb + 1 + lane : in.V];
+          }
+        } while (readlane_u64(w_end, (uint32_t)(r - rb)) == row_end);
+      }
+      while (act) {
+        constexpr uint32_t U = NARROW ? 8 : 4;  // rows in flight
+        P d[U], c[U];
+        uint32_t at[U];
+#pragma unroll
+        for (uint32_t i = 0; i < U; i++) {  // every row read issued first
+          at[i] = act ? (uint32_t)__ffsll((unsigned long long)act) - 1 : at[i ? i - 1 : 0];
+          act &= act - 1;
+          d[i] = P::inf();  // (lanes whose queries have no frontier there read nothing)
+          if (__builtin_amdgcn_inverse_ballot_w64(readlane_u64(my_f, at[i])))
+            d[i] = P::load(dist, (uint32_t)__builtin_amdgcn_readlane(my_u, at[i]), lane);
+          c[i] = P::inf();
+          if ((heads >> at[i]) & 1ull) c[i] = P::load(dist, (uint32_t)__builtin_amdgcn_readlane(my_r, at[i]), lane);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < U; i++) {  // (the last edge again: changes nothing)
+          const uint32_t row = __builtin_amdgcn_readlane(my_r, at[i]);
+          if (row != open) {
+            close();
+            open = row;
+            cur = c[i];
+            acc = low = P::inf();
+          }
+          low = low.min(d[i]);
+          acc = acc.min(d[i].plus(__builtin_amdgcn_readlane(my_w, at[i])));
+        }
+      }
+    }
+    // r: the row of the last edge; it goes on past e1, or ends there
+    const bool more = readlane_u64(w_end, (uint32_t)(r - rb)) > e1;
+    if (shared0 && lane == 0) {
+      s_row[0][wv] = r0;
+      s_span[wv] = more && r == r0;
+    }
+    if (more && !(shared0 && r == r0)) {
+      if (open != (uint32_t)r) {
+        close();
+        acc = low = P::inf();
+        open = (uint32_t)r;
+      }
+      s_acc[1][wv][lane] = acc;
+      s_low[1][wv][lane] = low;
+      if (lane == 0) s_row[1][wv] = (uint32_t)r;
+    } else {
+      close();
+    }
+  }
+  __syncthreads();
+  // shared rows: the wave that holds a row's first edges, or the first wave
+  // for the row that the workgroup before it began, gathers the parts
+  auto gather = [&](uint32_t k, bool begins) {
+    const uint32_t row = s_row[k][wv];
+    if (row == INFINIT) return;
+    P acc = s_acc[k][wv][lane], low = s_low[k][wv][lane];
+    bool on = k || s_span[wv];
+    for (uint32_t w = wv + 1; on && w < PULL_WAVES; w++) {
+      acc = acc.min(s_acc[0][w][lane]);
+      low = low.min(s_low[0][w][lane]);
+      on = s_span[w];
+    }
+    finish(row, begins && !on, P::load(dist, row, lane), acc, low);
+  };
+  if (wv == 0) gather(0, false);
+  gather(1, true);
+  if (lane == 0) {
+    or_bits(&cnt->slot_alive[0], imp_a);
+    or_bits(&cnt->slot_alive[1], imp_b);
+    if (NARROW) or_bits(&cnt->overflow[0], ovf_a);
+    if (NARROW) or_bits(&cnt->overflow[1], ovf_b);
   }
 }
 
@@ -532,7 +794,7 @@ __global__ __launch_bounds__(BLOCK) void k_sssp_finalize(const uint64_t *off, ui
       tot += x;
     }
     s_base = tot ? atomicAdd(&cnt->qcount, tot) : 0u;
-    if (s_alive) atomicOr((unsigned long long *)&cnt->alive, s_alive);
+    or_bits(&cnt->alive, s_alive);
   }
   __syncthreads();
   uint32_t slot = s_base + s_wpre[wid] + incl - c;
@@ -789,6 +1051,17 @@ void MsEngine::init() {
   push_.tmp = scan_tmp_.p;
   push_.tmp_bytes = tb;
   dirty_ = all_slots();  // state starts uninitialised
+  // SSSP steps that pull need the in-edges and their weights in HBM (a
+  // directed graph's are not built for this alone)
+  if (kind_ == MsKind::SSSP && g.placement == GRUS_PLACE_HBM && g.E &&
+      (g.symmetric ? g.weights_mirror() : g.csc_ready)) {
+    pull_per_ = ms::PULL_EDGES;
+    while (div_up(g.E, (uint64_t)pull_per_) > V) pull_per_ *= 2;  // (longq_ holds the first rows)
+    const uint64_t n = div_up(g.E, (uint64_t)pull_per_);
+    ms::k_pull_first<<<grid_cap(ctx, n, BLOCK), BLOCK, 0, ctx.stream>>>(
+        g.csc().off, V, pull_per_, n, longq_.as<uint32_t>());
+    GRUS_LAUNCH_CHECK();
+  }
   ctx.sync();
 }
 
@@ -982,7 +1255,26 @@ std::vector<int> MsEngine::step() {
         vals_.as<uint32_t>(), V, run_lanes, (uint32_t)t_, st, queue_.as<uint32_t>(), cnt);
     GRUS_LAUNCH_CHECK();
   } else {
-    if (qn_) {
+    // A step pulls when the frontier's out-edges are over a third of all edges
+    // and the queries take 8 lanes or more.  128 queries on RMAT, whole batch,
+    // by the divisor 1.5 / 2 / 3 / 4 / 6: 4.41 / 4.43 / 4.11 / 4.13 / 4.27 ms
+    // at scale 18, 39.5 / 39.3 / 39.5 / 40.9 / 42.1 at 22 (never: 7.83, 87.0).
+    // By queries at scale 18, push against pull: 8 (4 lanes) 2.55 and 2.80 ms,
+    // 16 3.73 and 2.92, 32 6.29 and 3.04.
+    if (pull_per_ && qn_ && front_edges_ > g_.E / 3 && __builtin_popcountll(run_lanes) >= 8) {
+      const CsrView in = g_.csc();
+      const unsigned grid = (unsigned)div_up(in.E, (uint64_t)pull_per_ * ms::PULL_WAVES);
+      const uint32_t *first = longq_.as<uint32_t>();
+      if (narrow_)
+        ms::k_sssp_pull<true><<<grid, ms::PULL_WAVES * WAVE, 0, ctx.stream>>>(
+            in, pull_per_, first, front_.as<uint64_t>(), next_.as<uint64_t>(),
+            vals_.as<uint32_t>(), cnt);
+      else
+        ms::k_sssp_pull<false><<<grid, ms::PULL_WAVES * WAVE, 0, ctx.stream>>>(
+            in, pull_per_, first, front_.as<uint64_t>(), next_.as<uint64_t>(),
+            vals_.as<uint32_t>(), cnt);
+      GRUS_LAUNCH_CHECK();
+    } else if (qn_) {
       uint64_t *cs = push_.scan_ptr();
       ms::k_chunk_counts<<<grid_cap(ctx, qn_ + 1, BLOCK), BLOCK, 0, ctx.stream>>>(
           out.off, queue_.as<uint32_t>(), (uint32_t)qn_, push_.deg_ptr());

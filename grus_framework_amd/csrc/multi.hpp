@@ -103,6 +103,7 @@ class MsEngine {
   bool narrow_ = false;
   uint64_t t_ = 0;         // global step counter
   uint64_t qn_ = 0, front_edges_ = 0;
+  uint32_t pull_per_ = 0;  // SSSP: in-edges per wave of a pull step; 0: steps only push
   Buf visit_, front_, next_, vals_, queue_, longq_, row_, rows_, digest_, srcs_dev_, cnt_, push_cnt_;
   Buf hmirror_;  // pinned host words: the counters as published, then read-back scratch
   PushWork push_;
