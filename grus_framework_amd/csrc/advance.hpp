@@ -80,23 +80,6 @@ __device__ __forceinline__ uint32_t upper_bound_u64(const uint64_t *a, uint32_t 
   return lo;
 }
 
-// The same by a whole wave (every lane calls it with the same arguments, in
-// global memory): 64 probes a step, so a queue of 4096 takes two dependent
-// loads and one of 2^24 four, where one thread's binary search took 12 and 24.
-__device__ __forceinline__ uint32_t wave_upper_bound_u64(const uint64_t *a, uint32_t lo,
-                                                         uint32_t hi, uint64_t key) {
-  for (;;) {
-    const uint32_t step = (hi - lo + WAVE - 1) / WAVE;
-    const uint64_t idx = (uint64_t)lo + (uint64_t)lane_id() * step;
-    // a is non-decreasing, so the probes at most key are the first c lanes
-    const uint32_t c = (uint32_t)__popcll(__ballot(idx < hi && a[idx] <= key));
-    if (step <= 1 || c == 0) return lo + c;
-    const uint64_t end = (uint64_t)lo + (uint64_t)c * step;
-    lo += (c - 1) * step + 1;
-    if (end < hi) hi = (uint32_t)end;
-  }
-}
-
 // own[0], own[1] (LDS) <- the queue entries that own positions c0 and c1 - 1
 // of the edge space scanned in S; one wave each.  Ends with a barrier.
 __device__ __forceinline__ void chunk_owners(const uint64_t *S, uint32_t F, uint64_t c0,

@@ -382,41 +382,27 @@ __global__ void k_grid_fill(uint32_t R, uint32_t C, const uint64_t *off, uint32_
 }
 
 // ---- transpose: key = (dst << 32) | src for every CSR edge ----
-__global__ void k_transpose_keys(const uint64_t *off, const uint32_t *col, uint64_t V,
+__global__ void k_transpose_keys(const uint64_t *off, const uint32_t *col, uint64_t V, uint64_t E,
                                  uint64_t *keys) {
-  uint64_t wave = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) / WAVE;
-  uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
-  for (uint64_t u = wave; u < V; u += nw)
-    for (uint64_t e = off[u] + lane_id(); e < off[u + 1]; e += WAVE)
-      keys[e] = ((uint64_t)col[e] << 32) | u;
+  grid_edge_rows(off, V, E, [&](uint64_t e, uint32_t u, bool) {
+    keys[e] = ((uint64_t)col[e] << 32) | u;
+  });
 }
 
 // Sum over the edges of h(u, v, w) - h(v, u, w) for a hash h of 64 bits: 0 if
 // the edges are their own reverses, weights included, and by a chance of
-// 2^-64 otherwise.  A lane walks a short row, the wave a long one together.
+// 2^-64 otherwise.
 __device__ __forceinline__ uint64_t edge_hash(uint32_t u, uint32_t v, uint32_t w) {
   return mix64(mix64(((uint64_t)u << 32) | v) + w);
 }
 __global__ void k_mirror_sum(const uint64_t *off, const uint32_t *col, const uint32_t *w,
-                             uint64_t V, unsigned long long *sum) {
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  const uint32_t lane = lane_id();
+                             uint64_t V, uint64_t E, unsigned long long *sum) {
   unsigned long long s = 0;
-  for (uint64_t b = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x - lane; b < V; b += stride) {
-    const uint64_t u = b + lane;
-    const uint64_t e0 = u < V ? off[u] : 0, e1 = u < V ? off[u + 1] : 0;
-    const bool is_long = e1 - e0 > 32;
-    for (uint64_t e = e0; e < e1 && !is_long; e++)
-      s += edge_hash((uint32_t)u, col[e], w[e]) - edge_hash(col[e], (uint32_t)u, w[e]);
-    for (uint64_t m = __ballot(is_long); m; m &= m - 1) {
-      const int l = __ffsll((unsigned long long)m) - 1;
-      const uint64_t a = __shfl(e0, l), z = __shfl(e1, l);
-      for (uint64_t e = a + lane; e < z; e += WAVE)
-        s += edge_hash((uint32_t)(b + l), col[e], w[e]) - edge_hash(col[e], (uint32_t)(b + l), w[e]);
-    }
-  }
+  grid_edge_rows(off, V, E, [&](uint64_t e, uint32_t u, bool) {
+    s += edge_hash(u, col[e], w[e]) - edge_hash(col[e], u, w[e]);
+  });
   s = wave_sum(s);
-  if (lane == 0 && s) atomicAdd(sum, s);
+  if (lane_id() == 0 && s) atomicAdd(sum, s);
 }
 
 __global__ void k_iota_u32(uint32_t *a, uint64_t n) {
@@ -473,8 +459,8 @@ CsrView Graph::csc() {
     kb.alloc(E * 8);
     va.alloc(E * 4);
     vb.alloc(E * 4);
-    k_transpose_keys<<<grid_for(ctx, V * WAVE), BLOCK, 0, ctx->stream>>>(
-        off.as<uint64_t>(), col.as<uint32_t>(), V, ka.as<uint64_t>());
+    k_transpose_keys<<<grid_for(ctx, E), BLOCK, 0, ctx->stream>>>(
+        off.as<uint64_t>(), col.as<uint32_t>(), V, E, ka.as<uint64_t>());
     GRUS_LAUNCH_CHECK();
     k_iota_u32<<<grid_for(ctx, E), BLOCK, 0, ctx->stream>>>(va.as<uint32_t>(), E);
     GRUS_LAUNCH_CHECK();
@@ -535,8 +521,8 @@ bool Graph::weights_mirror() {
   if (mirror < 0) {
     auto *sum = reinterpret_cast<unsigned long long *>(ctx->d_ctl.p);
     GRUS_HIP(hipMemsetAsync(sum, 0, 8, ctx->stream));
-    k_mirror_sum<<<grid_for(ctx, V), BLOCK, 0, ctx->stream>>>(
-        off.as<uint64_t>(), col.as<uint32_t>(), w.as<uint32_t>(), V, sum);
+    k_mirror_sum<<<grid_for(ctx, E), BLOCK, 0, ctx->stream>>>(
+        off.as<uint64_t>(), col.as<uint32_t>(), w.as<uint32_t>(), V, E, sum);
     GRUS_LAUNCH_CHECK();
     ctx->read_ctl(1);
     mirror = ctx->h_ctl[0] == 0;

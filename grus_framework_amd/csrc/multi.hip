@@ -265,12 +265,6 @@ __global__ void k_chunk_counts(const uint64_t *off, const uint32_t *q, uint32_t 
   }
 }
 
-__device__ __forceinline__ uint64_t readlane_u64(uint64_t x, uint32_t i) {
-  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)x, i);
-  const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(x >> 32), i);
-  return ((uint64_t)hi << 32) | lo;
-}
-
 // Lowers 16-bit half `half` of *word to nd (a previous read of the word is
 // `old`); returns once the half is at most nd.  Values only decrease, so
 // every failed compare-and-swap means another lane lowered the word and the

@@ -165,15 +165,11 @@ __global__ void k_perm_from_keys(const uint64_t *keys, uint64_t V, uint32_t *per
   }
 }
 
-// relabelled edge keys (inv[u] << 32 | inv[v]), one wave per row
+// relabelled edge keys (inv[u] << 32 | inv[v])
 __global__ void k_relabel_edges(CsrView g, const uint32_t *inv, uint64_t *keys) {
-  uint64_t wave = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) / WAVE;
-  uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
-  for (uint64_t u = wave; u < g.V; u += nw) {
-    uint64_t nu = (uint64_t)inv[u] << 32;
-    for (uint64_t e = g.off[u] + lane_id(); e < g.off[u + 1]; e += WAVE)
-      keys[e] = nu | inv[edge_col(g, e)];
-  }
+  grid_edge_rows(g.off, g.V, g.E, [&](uint64_t e, uint32_t u, bool) {
+    keys[e] = ((uint64_t)inv[u] << 32) | inv[edge_col(g, e)];
+  });
 }
 
 __global__ void k_scatter_back(const float *r_new, const uint32_t *perm, uint64_t V, float *out) {
@@ -185,40 +181,31 @@ __global__ void k_scatter_back(const float *r_new, const uint32_t *perm, uint64_
 // ---- blocked layout construction (once per graph and bin width) ----
 
 // flag[e] = 1 when CSR edge e starts a group: the first edge of its row or
-// a destination bin different from the previous edge's (wave per row)
-__global__ void k_pb_flags(const uint64_t *off, const uint32_t *col, uint64_t V, int bits,
-                           uint32_t *flag) {
-  uint64_t wave = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) / WAVE;
-  uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
-  for (uint64_t u = wave; u < V; u += nw) {
-    const uint64_t a = off[u], b = off[u + 1];
-    for (uint64_t e = a + lane_id(); e < b; e += WAVE)
-      flag[e] = (e == a || (col[e] >> bits) != (col[e - 1] >> bits)) ? 1u : 0u;
-  }
+// a destination bin different from the previous edge's
+__global__ void k_pb_flags(const uint64_t *off, const uint32_t *col, uint64_t V, uint64_t E,
+                           int bits, uint32_t *flag) {
+  grid_edge_rows(off, V, E, [&](uint64_t e, uint32_t, bool first) {
+    flag[e] = (first || (col[e] >> bits) != (col[e - 1] >> bits)) ? 1u : 0u;
+  });
 }
 
 // group sort keys (bin << 32 | source), indexed by group id = excl[e] for
 // the group's first edge e
-__global__ void k_pb_gkeys(const uint64_t *off, const uint32_t *col, uint64_t V, int bits,
-                           const uint32_t *flag, const uint32_t *excl, uint64_t *gkey) {
-  uint64_t wave = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) / WAVE;
-  uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
-  for (uint64_t u = wave; u < V; u += nw)
-    for (uint64_t e = off[u] + lane_id(); e < off[u + 1]; e += WAVE)
-      if (flag[e]) gkey[excl[e]] = ((uint64_t)(col[e] >> bits) << 32) | u;
+__global__ void k_pb_gkeys(const uint64_t *off, const uint32_t *col, uint64_t V, uint64_t E,
+                           int bits, const uint32_t *flag, const uint32_t *excl, uint64_t *gkey) {
+  grid_edge_rows(off, V, E, [&](uint64_t e, uint32_t u, bool) {
+    if (flag[e]) gkey[excl[e]] = ((uint64_t)(col[e] >> bits) << 32) | u;
+  });
 }
 
 // transpose keys (dst << 32 | src) of every edge; excl[] becomes the group
 // id of each edge in place (excl[e] + flag[e] - 1)
-__global__ void k_pb_tkeys(const uint64_t *off, const uint32_t *col, uint64_t V,
+__global__ void k_pb_tkeys(const uint64_t *off, const uint32_t *col, uint64_t V, uint64_t E,
                            const uint32_t *flag, uint32_t *excl_to_gid, uint64_t *tkey) {
-  uint64_t wave = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) / WAVE;
-  uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
-  for (uint64_t u = wave; u < V; u += nw)
-    for (uint64_t e = off[u] + lane_id(); e < off[u + 1]; e += WAVE) {
-      tkey[e] = ((uint64_t)col[e] << 32) | u;
-      excl_to_gid[e] = excl_to_gid[e] + flag[e] - 1u;
-    }
+  grid_edge_rows(off, V, E, [&](uint64_t e, uint32_t u, bool) {
+    tkey[e] = ((uint64_t)col[e] << 32) | u;
+    excl_to_gid[e] = excl_to_gid[e] + flag[e] - 1u;
+  });
 }
 
 // goff[u] = number of groups of the rows before u, for u in [0, V]
@@ -858,15 +845,14 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_min_finish(const uint32_t *mbin
 // weight stream keys: CSR edge e -> (bin of its destination, weight); the
 // same keys as the d2 sort, so the same stable sort puts the weights in d2's
 // order
-__global__ void k_bp_w2_keys(const uint64_t *off, const uint32_t *col, const uint32_t *w,
-                             uint64_t V, int bits, uint64_t *key, uint32_t *wt) {
-  uint64_t wave = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) / WAVE;
-  uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
-  for (uint64_t u = wave; u < V; u += nw)
-    for (uint64_t e = off[u] + lane_id(); e < off[u + 1]; e += WAVE) {
-      key[e] = col[e] >> bits;
-      wt[e] = w[e];
-    }
+__global__ void k_bp_w2_keys(const uint32_t *col, const uint32_t *w, uint64_t E, int bits,
+                             uint64_t *key, uint32_t *wt) {
+  uint64_t e = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+  uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (; e < E; e += stride) {
+    key[e] = col[e] >> bits;
+    wt[e] = w[e];
+  }
 }
 
 // w2: the sorted weights (narrowed to WT, which holds the largest), padded
@@ -978,18 +964,50 @@ __global__ void k_bp_runs(const uint32_t *rflag, const uint32_t *rexcl, const ui
   for (; i <= nch; i += stride) ch_r0[i] = ch_i0[i] < G ? rexcl[ch_i0[i]] : R;
 }
 
-// phase-2 stream keys: CSR edge e -> (bin of its destination, entry)
-__global__ void k_bp_d2_keys(const uint64_t *off, const uint32_t *col, uint64_t V, int bits,
-                             const uint32_t *flag, uint64_t *key, uint32_t *ent) {
-  uint64_t wave = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) / WAVE;
-  uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
-  const uint32_t mask = (1u << bits) - 1u;
-  for (uint64_t u = wave; u < V; u += nw)
-    for (uint64_t e = off[u] + lane_id(); e < off[u + 1]; e += WAVE) {
-      const uint32_t v = col[e];
-      key[e] = v >> bits;
-      ent[e] = (flag[e] << 15) | (v & mask);
+// next[u]: the end of a chunk that starts at row u, the last row bound within
+// BP_SPAN rows and chunk_groups groups (at least one row)
+__global__ void k_bp_next(const uint64_t *goff, uint64_t V, uint64_t chunk_groups, uint32_t *next) {
+  uint64_t u = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+  uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (; u < V; u += stride) {
+    const uint64_t most = goff[u] + chunk_groups;
+    uint64_t lo = u + 1, hi = u + BP_SPAN < V ? u + BP_SPAN : V;
+    while (lo < hi) {  // the last x in (u, hi] with goff[x] <= most, or u + 1
+      const uint64_t mid = lo + (hi - lo + 1) / 2;
+      if (goff[mid] <= most) lo = mid;
+      else hi = mid - 1;
     }
+    next[u] = (uint32_t)lo;
+  }
+}
+
+// The chunks' first rows and groups, one after the other from row 0, with the
+// end after the last.  One thread: a dependent read a chunk (RMAT scale 24,
+// 8000 chunks).  The host's walk over all of goff, with the copy of its 134 MB,
+// took half of the layout's build there.
+__global__ void k_bp_chunks(const uint64_t *goff, const uint32_t *next, uint64_t V, uint64_t G,
+                            uint32_t most, uint32_t *ch_u0, uint32_t *ch_i0, uint32_t *nch) {
+  uint32_t n = 0;
+  for (uint64_t u = 0; u < V && n + 1 < most; u = next[u]) {
+    ch_u0[n] = (uint32_t)u;
+    ch_i0[n++] = (uint32_t)goff[u];
+  }
+  ch_u0[n] = (uint32_t)V;
+  ch_i0[n] = (uint32_t)G;
+  *nch = n;
+}
+
+// phase-2 stream keys: CSR edge e -> (bin of its destination, entry)
+__global__ void k_bp_d2_keys(const uint32_t *col, uint64_t E, int bits, const uint32_t *flag,
+                             uint64_t *key, uint32_t *ent) {
+  uint64_t e = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+  uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  const uint32_t mask = (1u << bits) - 1u;
+  for (; e < E; e += stride) {
+    const uint32_t v = col[e];
+    key[e] = v >> bits;
+    ent[e] = (flag[e] << 15) | (v & mask);
+  }
 }
 
 // d2 (u16, padded with zeros to a multiple of BP_SLAB, each slab stored
@@ -1147,7 +1165,7 @@ void build_relabelled(Graph &g, PrWork &w) {
   pr::k_perm_from_keys<<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(
       sk, V, w.perm.as<uint32_t>(), inv.as<uint32_t>());
   GRUS_LAUNCH_CHECK();
-  pr::k_relabel_edges<<<grid_cap(ctx, V * WAVE, BLOCK), BLOCK, 0, ctx.stream>>>(
+  pr::k_relabel_edges<<<grid_cap(ctx, g.E, BLOCK), BLOCK, 0, ctx.stream>>>(
       g.csr(), inv.as<uint32_t>(), ka.as<uint64_t>());
   GRUS_LAUNCH_CHECK();
   uint64_t *se = sort_keys_u64(ctx, ka.as<uint64_t>(), kb.as<uint64_t>(), E);
@@ -1183,11 +1201,11 @@ bool build_blocked(Graph &g, PrWork &w, int bits) {
   w.pb_gidx.release();
   w.pb_val.release();
   w.pb_for = nullptr;
-  const unsigned rows_grid = grid_cap(ctx, V * WAVE, BLOCK);
+  const unsigned edge_grid = grid_cap(ctx, E, BLOCK);
   Buf flag, excl;
   flag.alloc(E * 4);
   excl.alloc(E * 4);
-  pr::k_pb_flags<<<rows_grid, BLOCK, 0, ctx.stream>>>(out.off, out.col, V, bits,
+  pr::k_pb_flags<<<edge_grid, BLOCK, 0, ctx.stream>>>(out.off, out.col, V, E, bits,
                                                       flag.as<uint32_t>());
   GRUS_LAUNCH_CHECK();
   scan_excl_u32(ctx, flag.as<uint32_t>(), excl.as<uint32_t>(), E);
@@ -1210,7 +1228,7 @@ bool build_blocked(Graph &g, PrWork &w, int bits) {
     kb.alloc(G * 8);
     va.alloc(G * 4);
     vb.alloc(G * 4);
-    pr::k_pb_gkeys<<<rows_grid, BLOCK, 0, ctx.stream>>>(out.off, out.col, V, bits,
+    pr::k_pb_gkeys<<<edge_grid, BLOCK, 0, ctx.stream>>>(out.off, out.col, V, E, bits,
                                                         flag.as<uint32_t>(), excl.as<uint32_t>(),
                                                         ka.as<uint64_t>());
     GRUS_LAUNCH_CHECK();
@@ -1230,7 +1248,7 @@ bool build_blocked(Graph &g, PrWork &w, int bits) {
     ka.alloc(E * 8);
     kb.alloc(E * 8);
     vb.alloc(E * 4);
-    pr::k_pb_tkeys<<<rows_grid, BLOCK, 0, ctx.stream>>>(out.off, out.col, V, flag.as<uint32_t>(),
+    pr::k_pb_tkeys<<<edge_grid, BLOCK, 0, ctx.stream>>>(out.off, out.col, V, E, flag.as<uint32_t>(),
                                                         excl.as<uint32_t>(), ka.as<uint64_t>());
     GRUS_LAUNCH_CHECK();
     ctx.sync();
@@ -1312,11 +1330,11 @@ bool build_binned(Graph &g, PrWork &w, int bits) {
   w.bp_sp = {};
   w.bp_for = nullptr;
   w.bp_w2_for = nullptr;
-  const unsigned rows_grid = grid_cap(ctx, V * WAVE, BLOCK);
+  const unsigned edge_grid = grid_cap(ctx, E, BLOCK);
   Buf flag, excl;
   flag.alloc(E * 4);
   excl.alloc(E * 4);
-  pr::k_pb_flags<<<rows_grid, BLOCK, 0, ctx.stream>>>(out.off, out.col, V, bits,
+  pr::k_pb_flags<<<edge_grid, BLOCK, 0, ctx.stream>>>(out.off, out.col, V, E, bits,
                                                       flag.as<uint32_t>());
   GRUS_LAUNCH_CHECK();
   scan_excl_u32(ctx, flag.as<uint32_t>(), excl.as<uint32_t>(), E);
@@ -1327,46 +1345,47 @@ bool build_binned(Graph &g, PrWork &w, int bits) {
                           ctx.stream));
   ctx.sync();
   const uint64_t G = (uint64_t)last[0] + last[1];
-  // groups per source (goff) -> phase-1 chunks, on the host (a source with
-  // more groups than a chunk takes is a chunk of its own: a chunk has at most
-  // nbins runs however many groups)
+  // groups per source (goff) -> phase-1 chunks (a source with more groups than
+  // a chunk takes is a chunk of its own: a chunk has at most nbins runs
+  // however many groups)
   // Chunks of G / 512 groups, two workgroups per CU, between 4096 (whole
   // slabs mostly) and BP_CHUNK_GROUPS.  RMAT, us per PageRank iteration with
   // 32768 / G / 512 groups: s16 24 / 15, s18 37 / 30, s20 74 / 73; with G /
   // 1024 groups s18 31, s20 76.
   const uint64_t chunk_groups = std::max<uint64_t>(4096, std::min<uint64_t>(BP_CHUNK_GROUPS, G / 512));
-  std::vector<uint32_t> ch_u0, ch_i0;
+  uint32_t nch = 0;
   {
-    Buf goff;
+    // (two chunks in a row that end for their groups hold more than
+    // chunk_groups together)
+    const uint64_t most = 2 * (G / chunk_groups) + V / pr::BP_SPAN + 4;
+    Buf goff, next, cu, ci, n;
     goff.alloc((V + 1) * 8);
+    next.alloc((V + 1) * 4);
+    cu.alloc(most * 4);
+    ci.alloc(most * 4);
+    n.alloc(4);
     pr::k_pb_goff<<<grid_cap(ctx, V + 1, BLOCK), BLOCK, 0, ctx.stream>>>(
         out.off, V, E, excl.as<uint32_t>(), G, goff.as<uint64_t>());
     GRUS_LAUNCH_CHECK();
-    std::vector<uint64_t> h(V + 1);
-    GRUS_HIP(hipMemcpyAsync(h.data(), goff.p, (V + 1) * 8, hipMemcpyDeviceToHost, ctx.stream));
+    pr::k_bp_next<<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(
+        goff.as<uint64_t>(), V, chunk_groups, next.as<uint32_t>());
+    GRUS_LAUNCH_CHECK();
+    pr::k_bp_chunks<<<1, 1, 0, ctx.stream>>>(goff.as<uint64_t>(), next.as<uint32_t>(), V, G,
+                                             (uint32_t)most, cu.as<uint32_t>(), ci.as<uint32_t>(),
+                                             n.as<uint32_t>());
+    GRUS_LAUNCH_CHECK();
+    GRUS_HIP(hipMemcpyAsync(&nch, n.p, 4, hipMemcpyDeviceToHost, ctx.stream));
     ctx.sync();
-    uint64_t u0 = 0;
-    while (u0 < V) {
-      uint64_t u1 = u0 + 1;
-      while (u1 < V && u1 - u0 < pr::BP_SPAN && h[u1 + 1] - h[u0] <= chunk_groups) u1++;
-      ch_u0.push_back((uint32_t)u0);
-      ch_i0.push_back((uint32_t)h[u0]);
-      u0 = u1;
-    }
-    ch_i0.push_back((uint32_t)G);
+    w.bp_ch_u0.alloc((nch + 1) * 4);
+    w.bp_ch_i0.alloc((nch + 1) * 4);
+    GRUS_HIP(hipMemcpyAsync(w.bp_ch_u0.p, cu.p, (nch + 1) * 4, hipMemcpyDeviceToDevice, ctx.stream));
+    GRUS_HIP(hipMemcpyAsync(w.bp_ch_i0.p, ci.p, (nch + 1) * 4, hipMemcpyDeviceToDevice, ctx.stream));
+    ctx.sync();
   }
-  const uint32_t nch = (uint32_t)ch_u0.size();
-  ch_u0.push_back((uint32_t)V);  // sentinel: the last chunk's end
-  w.bp_ch_u0.alloc((nch + 1) * 4);
-  w.bp_ch_i0.alloc((nch + 1) * 4);
-  GRUS_HIP(hipMemcpyAsync(w.bp_ch_u0.p, ch_u0.data(), (nch + 1) * 4, hipMemcpyHostToDevice,
-                          ctx.stream));
-  GRUS_HIP(hipMemcpyAsync(w.bp_ch_i0.p, ch_i0.data(), (nch + 1) * 4, hipMemcpyHostToDevice,
-                          ctx.stream));
   // group keys (bin << 32 | source), by group id
   Buf gkey, slot;
   gkey.alloc(G * 8);
-  pr::k_pb_gkeys<<<rows_grid, BLOCK, 0, ctx.stream>>>(out.off, out.col, V, bits,
+  pr::k_pb_gkeys<<<edge_grid, BLOCK, 0, ctx.stream>>>(out.off, out.col, V, E, bits,
                                                       flag.as<uint32_t>(), excl.as<uint32_t>(),
                                                       gkey.as<uint64_t>());
   GRUS_LAUNCH_CHECK();
@@ -1442,9 +1461,8 @@ bool build_binned(Graph &g, PrWork &w, int bits) {
     kb.alloc(E * 8);
     vb.alloc(E * 4);
     bs.alloc((nbins + 1) * 4);
-    pr::k_bp_d2_keys<<<rows_grid, BLOCK, 0, ctx.stream>>>(out.off, out.col, V, bits,
-                                                         flag.as<uint32_t>(), ka.as<uint64_t>(),
-                                                         excl.as<uint32_t>());
+    pr::k_bp_d2_keys<<<edge_grid, BLOCK, 0, ctx.stream>>>(out.col, E, bits, flag.as<uint32_t>(),
+                                                         ka.as<uint64_t>(), excl.as<uint32_t>());
     GRUS_LAUNCH_CHECK();
     uint32_t *ent = nullptr;
     uint64_t *key = sort_pairs_u64_u32(ctx, ka.as<uint64_t>(), kb.as<uint64_t>(),
@@ -1657,7 +1675,7 @@ void run_exact_pull(Graph &g, PrWork &w, float alpha, int iters, grus_stats *st)
 bool build_binned_weights(Graph &g, PrWork &w) {
   Context &ctx = *g.ctx;
   const CsrView out = g.csr();
-  const uint64_t V = g.V, E = g.E;
+  const uint64_t E = g.E;
   if (!out.w || out.split < E) return false;
   size_t free_b = 0, total_b = 0;
   GRUS_HIP(hipMemGetInfo(&free_b, &total_b));
@@ -1670,8 +1688,8 @@ bool build_binned_weights(Graph &g, PrWork &w) {
     kb.alloc(E * 8);
     va.alloc(E * 4);
     vb.alloc(E * 4);
-    pr::k_bp_w2_keys<<<grid_cap(ctx, V * WAVE, BLOCK), BLOCK, 0, ctx.stream>>>(
-        out.off, out.col, out.w, V, w.bp_bits, ka.as<uint64_t>(), va.as<uint32_t>());
+    pr::k_bp_w2_keys<<<grid_cap(ctx, E, BLOCK), BLOCK, 0, ctx.stream>>>(
+        out.col, out.w, E, w.bp_bits, ka.as<uint64_t>(), va.as<uint32_t>());
     GRUS_LAUNCH_CHECK();
     // the stream is as narrow as the largest weight allows (RMAT inputs
     // with weights below 256 read one byte per edge instead of four)
