@@ -318,17 +318,32 @@ struct BpTask {
 // (exact), the high word is trunc(y) and the low word trunc(fract(y) *
 // 2^32); fract(y) is exact and has at most 24 significant bits, so both
 // conversions are exact.
-__device__ __forceinline__ unsigned long long to_fixed(float x) {
+__device__ __forceinline__ unsigned long long scaled_to_fixed(float y) {  // y = x * 2^30
   static_assert(BP_FIX == 62, "the split below assumes 2^62");
-  const float y = x * 0x1p30f;
   const uint32_t hi = (uint32_t)y;
   const uint32_t lo = (uint32_t)(__builtin_amdgcn_fractf(y) * 0x1p32f);
   return ((unsigned long long)hi << 32) | lo;
 }
 
+__device__ __forceinline__ unsigned long long to_fixed(float x) {
+  return scaled_to_fixed(x * 0x1p30f);
+}
+
 __device__ __forceinline__ float from_fixed(unsigned long long s) {
   return (float)((double)s * 0x1p-62);
 }
+
+// The accumulator of row i of a bin.  The destinations of a skewed graph share
+// their low bits (RMAT: bit by bit 0 with a chance of 3 in 4), and with row i
+// in slot i a quarter of a wave's additions fell on one of the 32 pairs of LDS
+// banks: 16 of 64 lanes on average, 5.6 with the low six bits mixed with the
+// upper ones.  The stream holds slots, so only the ends of a task compute it;
+// 64 consecutive rows stay in their 64 slots.
+__device__ __forceinline__ uint32_t acc_slot(uint32_t i) {
+  const uint32_t hi = i >> 6;
+  return i ^ ((hi ^ (hi >> 2) ^ (hi >> 3)) & 63u);
+}
+__device__ __forceinline__ uint32_t acc_slots(uint32_t rows) { return (rows + 63u) & ~63u; }
 
 // Phase 1: val[slot(j)] = contrib[src(j)] for every group j.  Workgroup c
 // takes the groups of one source chunk in (bin, source) order, so the
@@ -346,11 +361,11 @@ __device__ __forceinline__ float from_fixed(unsigned long long s) {
 // source order made each wave's loads touch dozens of lines.
 //
 // The value of a source is any 4-byte pattern Src gives: PageRank's
-// contribution, or (SSSP pull rounds) the distance of a frontier vertex.
+// contribution, scaled by 2^30 (exactly) as phase 2 wants it, or (SSSP pull rounds) the distance of a frontier vertex.
 struct ContribValue {
   const float *contrib;
   __device__ __forceinline__ uint32_t operator()(uint32_t u) const {
-    return __float_as_uint(contrib[u]);
+    return __float_as_uint(contrib[u] * 0x1p30f);
   }
 };
 struct FrontDistValue {  // 0xFFFFFFFF: not in the frontier bitmap
@@ -462,9 +477,32 @@ __global__ __launch_bounds__(BLOCK) void k_bp_scatter(const uint32_t *ch_u0, con
   }
 }
 
+// The window value of each entry of a slab (lane l: entries 64 q + l, q =
+// 0..7): its group, counted from the slab's first, is the group starts up to
+// it, less one if the first entry is a start itself.  A row's starts up to a
+// lane are those before the lane in the mask without its first bit, and that
+// bit, as the totals of the rows before, counts in scalar registers: four
+// vector instructions an entry.
+template <typename T>
+__device__ __forceinline__ void window_values(const uint32_t *wd, const T *win, T *x) {
+  uint32_t run = 0;
+#pragma unroll
+  for (int q = 0; q < BP_EPT; q++) {
+    const uint64_t b = __ballot((q & 1) ? (int32_t)wd[q >> 1] < 0 : (wd[q >> 1] & 0x8000u) != 0);
+    const uint32_t b0 = (uint32_t)b & 1u;
+    run = q ? run + b0 : 0u;
+    x[q] = win[run + lane_rank(b >> 1)];
+    run += (uint32_t)__popcll(b >> 1);
+  }
+}
+template <int MAXB>
+__device__ __forceinline__ uint32_t entry_slot(const uint32_t *wd, int q) {
+  return (wd[q >> 1] >> ((q & 1) ? 16 : 0)) & ((1u << MAXB) - 1u);
+}
+
 // Phase 2: one task = a piece of one destination bin's edge stream.  Each
-// stream entry is a u16: bit 15 starts a group, bits 0..14 the destination
-// within the bin.  A wave step takes one slab of BP_SLAB entries (8 per
+// stream entry is a u16: bit 15 starts a group, bits 0..14 the accumulator of
+// the destination within the bin (acc_slot).  A wave step takes one slab of BP_SLAB entries (8 per
 // lane, one 16-byte load; slabs are stored transposed, so lane l gets the
 // entries l, l + 64, ...).  The group index of every entry follows from
 // the slab's first group (gs512) and a wave prefix count of the flags (one
@@ -475,6 +513,16 @@ __global__ __launch_bounds__(BLOCK) void k_bp_scatter(const uint32_t *ch_u0, con
 // LDS accumulators as fixed-point integers, so the sums do not depend on
 // the order of the atomics.  A bin's only task finishes its rows; pieces of
 // split bins add their sums into gacc, which k_bp_finish completes.
+//
+// Bound at RMAT s24 (543 us, 2.0 GB of streams): with parts taken out, the
+// entry stream alone takes 223 us (4.7 TB/s), the instructions and window
+// accesses of the steps 295 alone, the ends of the tasks 90, the additions 20
+// beside the rest.  Two to four slabs on their way per wave instead of one
+// change nothing (551..558 us), so it is issue and LDS, not latency.  617 us
+// before the accumulators were spread over the banks, 552 before the window
+// indexes were counted in scalar registers (172 M vector instructions, now
+// 105 M); s22 154, 126, 118.  Leaving out the window's unused rows (half)
+// costs more in branches than it saves: 990 and 984 us an iteration.
 //
 // MAXB >= bits sizes the accumulators: with bins of 2^12 vertices two
 // workgroups fit a CU instead of one.
@@ -488,72 +536,62 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_accum(
   const BpTask t = tasks[blockIdx.x];
   const uint64_t v0 = (uint64_t)t.bin << bits;
   const uint32_t nb = (uint32_t)((V - v0) < (1ull << bits) ? (V - v0) : (1ull << bits));
-  for (uint32_t i = threadIdx.x; i < nb; i += BP_BLOCK) acc[i] = 0ull;
+  for (uint32_t i = threadIdx.x; i < acc_slots(nb); i += BP_BLOCK) acc[i] = 0ull;
   __syncthreads();
   constexpr uint32_t NW = BP_BLOCK / WAVE;
-  const uint32_t lane = lane_id(), wid = threadIdx.x / WAVE;
+  const uint32_t lane = lane_id();
+  const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   float *wv = win[wid];
   const uint32_t s1 = (uint32_t)((t.e1 + (uint64_t)BP_SLAB - 1) / BP_SLAB);
-  // software pipeline: the next slab's entries load while this one runs
+  // Software pipeline: while a slab is summed, the next one's entries and
+  // window values load.  (Past the task's last slab it reloads that slab,
+  // which keeps the wait counts exact.)  The first groups of the wave's next
+  // 64 slabs are held in a register, a slab per lane.
   uint32_t s = t.e0 / BP_SLAB + wid;
+  auto first_groups = [&](uint32_t from) {
+    const uint64_t k = (uint64_t)from + (uint64_t)lane * NW;
+    uint32_t g = gs512[k < s1 ? k : s1 - 1u];
+    asm volatile("" : "+v"(g));  // (waits here, once in 64 slabs, not at each use)
+    return g;
+  };
+  auto entries = [&](uint32_t slab) {
+    return __builtin_nontemporal_load(
+        reinterpret_cast<const u32x4 *>(d2 + (uint64_t)slab * BP_SLAB) + lane);
+  };
   u32x4 nx = {0, 0, 0, 0};
-  uint32_t ngs = 0;
+  float wl[BP_SLAB / WAVE];
+  uint32_t vg = 0;
+  // the slab's groups, at most BP_SLAB of them: the one its first entry
+  // continues or starts, and every group started inside it (val is padded by
+  // BP_SLAB, so the window loads need no bound)
+  auto window = [&](uint32_t i) {
+    const float *vb = val + (uint32_t)__builtin_amdgcn_readlane(vg, i & 63u);
+#pragma unroll
+    for (int j = 0; j < BP_SLAB / WAVE; j++) wl[j] = vb[lane + WAVE * j];
+  };
   if (s < s1) {
-    nx = __builtin_nontemporal_load(
-        reinterpret_cast<const u32x4 *>(d2 + (uint64_t)s * BP_SLAB + lane * BP_EPT));
-    ngs = gs512[s];
+    vg = first_groups(s);
+    window(0);
+    nx = entries(s);
   }
-  for (; s < s1; s += NW) {
+  for (uint32_t it = 1; s < s1; s += NW, it++) {
     const u32x4 cur = nx;
-    const uint32_t gbase = ngs;  // groups that start before the slab
-    const uint32_t wd[4] = {cur.x, cur.y, cur.z, cur.w};
-    // lane l holds the slab's entries 64 q + l, q = 0..7 (transposed layout)
-    uint32_t ent[BP_EPT];
-#pragma unroll
-    for (int q = 0; q < BP_EPT; q++) ent[q] = (q & 1) ? (wd[q >> 1] >> 16) : (wd[q >> 1] & 0xFFFFu);
-    // group of entry 64 q + l: gbase - 1 + (flags of the rows before q) +
-    // (flags of row q up to lane l); row totals are wave-uniform
-    uint32_t gq[BP_EPT];
-    uint32_t run = gbase - 1u;
-    uint64_t b0 = 0;
-#pragma unroll
-    for (int q = 0; q < BP_EPT; q++) {
-      const uint64_t bq = __ballot(ent[q] >> 15);
-      if (q == 0) b0 = bq;
-      gq[q] = run + lane_rank(bq) + (ent[q] >> 15);
-      run += (uint32_t)__popcll(bq);
-    }
-    // window = the slab's groups: the one its first entry continues (when
-    // that entry starts none) and every group started inside it
-    const uint32_t w0 = (b0 & 1ull) ? gbase : gbase - 1u;
-    // at most BP_SLAB groups from w0 on; val is padded by BP_SLAB, so the
-    // window loads need no bound
-    float wl[BP_SLAB / WAVE];
-#pragma unroll
-    for (int j = 0; j < BP_SLAB / WAVE; j++) wl[j] = val[w0 + lane + WAVE * j];
-    // the next slab's entries are requested after the window, so waiting
-    // for the window does not wait for them (unconditional: past the
-    // task's last slab it reloads that slab, which keeps the wait counts
-    // exact)
-    {
-      const uint32_t sn = s + NW < s1 ? s + NW : s1 - 1u;
-      nx = __builtin_nontemporal_load(
-          reinterpret_cast<const u32x4 *>(d2 + (uint64_t)sn * BP_SLAB + lane * BP_EPT));
-      ngs = gs512[sn];
-    }
 #pragma unroll
     for (int j = 0; j < BP_SLAB / WAVE; j++) wv[lane + WAVE * j] = wl[j];
+    if ((it & 63u) == 0) vg = first_groups(s + NW);
+    window(it);
+    nx = entries(s + NW < s1 ? s + NW : s1 - 1u);
+    const uint32_t wd[4] = {cur.x, cur.y, cur.z, cur.w};
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     float x[BP_EPT];
-#pragma unroll
-    for (int q = 0; q < BP_EPT; q++) x[q] = wv[gq[q] - w0];  // neighbouring lanes: near addresses
+    window_values(wd, wv, x);  // neighbouring lanes: near addresses
     const uint32_t sb = s * BP_SLAB;
     if (sb >= t.e0 && sb + BP_SLAB <= t.e1) {  // wave-uniform: the whole slab is the task's
 #pragma unroll
       for (int q = 0; q < BP_EPT; q++)
-        atomicAdd(&acc[ent[q] & ((1u << MAXB) - 1u)], to_fixed(x[q]));
+        atomicAdd(&acc[entry_slot<MAXB>(wd, q)], scaled_to_fixed(x[q]));
     } else {
       // a slab shared with a neighbouring bin (or padding): entries outside
       // the task add zero; their destination bits stay inside the array
@@ -561,7 +599,7 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_accum(
       for (int q = 0; q < BP_EPT; q++) {
         const uint32_t pe = sb + WAVE * q + lane;
         const unsigned long long keep = 0ull - (unsigned long long)(pe >= t.e0 && pe < t.e1);
-        atomicAdd(&acc[ent[q] & ((1u << MAXB) - 1u)], to_fixed(x[q]) & keep);
+        atomicAdd(&acc[entry_slot<MAXB>(wd, q)], scaled_to_fixed(x[q]) & keep);
       }
     }
     // the window is rewritten by the next slab only after these reads
@@ -576,7 +614,7 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_accum(
     for (int r = 0; r < R; r++) {
       const uint32_t i = threadIdx.x + BP_BLOCK * r;
       if (i < nb) {
-        const unsigned long long sum = acc[i];
+        const unsigned long long sum = acc[acc_slot(i)];
         if (sum) atomicAdd(&gacc[v0 + i], sum);
       }
     }
@@ -584,7 +622,7 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_accum(
 #pragma unroll
     for (int r = 0; r < R; r++) {
       const uint32_t i = threadIdx.x + BP_BLOCK * r;
-      if (i < nb) next[v0 + i] = finish_row(from_fixed(acc[i]), base, alpha);
+      if (i < nb) next[v0 + i] = finish_row(from_fixed(acc[acc_slot(i)]), base, alpha);
     }
   } else {
     // degrees of all the thread's rows are requested before any is used
@@ -603,7 +641,7 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_accum(
       for (int q = 0; q < U; q++) {
         const uint32_t i = threadIdx.x + BP_BLOCK * (rb + q);
         if (i < nb) {
-          const float rank = finish_row(from_fixed(acc[i]), base, alpha);
+          const float rank = finish_row(from_fixed(acc[acc_slot(i)]), base, alpha);
           const uint64_t d = b[q] - a[q];
           next[v0 + i] = d ? rank / (float)d : 0.0f;
         }
@@ -714,23 +752,25 @@ __device__ __forceinline__ void finish_rows(uint64_t v0, uint32_t nb, Best best_
 // lane l's 8 weights of a slab (entries l, l + 64, ...)
 template <typename WT>
 struct W2Slab {
-  uint32_t v[BP_EPT];
-  __device__ __forceinline__ void load(const WT *w2, uint64_t o) {
+  uint32_t v[2 * sizeof(WT)];
+  __device__ __forceinline__ void load(const WT *slab, uint32_t lane) {
     if constexpr (sizeof(WT) == 1) {
-      const uint64_t x = __builtin_nontemporal_load(reinterpret_cast<const uint64_t *>(w2 + o));
-#pragma unroll
-      for (int q = 0; q < BP_EPT; q++) v[q] = (uint32_t)(x >> (8 * q)) & 0xFFu;
-    } else if constexpr (sizeof(WT) == 2) {
-      const u32x4 x = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(w2 + o));
-      const uint32_t wd[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-      for (int q = 0; q < BP_EPT; q++) v[q] = (q & 1) ? (wd[q >> 1] >> 16) : (wd[q >> 1] & 0xFFFFu);
+      const uint64_t x = __builtin_nontemporal_load(reinterpret_cast<const uint64_t *>(slab) + lane);
+      v[0] = (uint32_t)x;
+      v[1] = (uint32_t)(x >> 32);
     } else {
-      const u32x4 x0 = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(w2 + o));
-      const u32x4 x1 = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(w2 + o) + 1);
-      v[0] = x0.x; v[1] = x0.y; v[2] = x0.z; v[3] = x0.w;
-      v[4] = x1.x; v[5] = x1.y; v[6] = x1.z; v[7] = x1.w;
+#pragma unroll
+      for (uint32_t i = 0; i < sizeof(WT) / 2; i++) {
+        const u32x4 x = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(slab) +
+                                                   lane * (sizeof(WT) / 2) + i);
+        v[4 * i] = x.x; v[4 * i + 1] = x.y; v[4 * i + 2] = x.z; v[4 * i + 3] = x.w;
+      }
     }
+  }
+  __device__ __forceinline__ uint32_t weight(int q) const {
+    constexpr int per = 4 / sizeof(WT), b = 8 * sizeof(WT);  // weights a word, bits a weight
+    const uint32_t x = v[q / per] >> (b * (q % per));
+    return b == 32 ? x : x & ((1u << (b & 31)) - 1u);
   }
 };
 
@@ -744,72 +784,63 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_min(const BpTask *tasks, const 
   const BpTask t = tasks[blockIdx.x];
   const uint64_t v0 = (uint64_t)t.bin << bits;
   const uint32_t nb = (uint32_t)((V - v0) < (1ull << bits) ? (V - v0) : (1ull << bits));
-  for (uint32_t i = threadIdx.x; i < nb; i += BP_BLOCK) acc[i] = 0xFFFFFFFFu;
+  for (uint32_t i = threadIdx.x; i < acc_slots(nb); i += BP_BLOCK) acc[i] = 0xFFFFFFFFu;
   __syncthreads();
   constexpr uint32_t NW = BP_BLOCK / WAVE;
-  const uint32_t lane = lane_id(), wid = threadIdx.x / WAVE;
+  const uint32_t lane = lane_id();
+  const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   uint32_t *wv = win[wid];
   const uint32_t s1 = (uint32_t)((t.e1 + (uint64_t)BP_SLAB - 1) / BP_SLAB);
   uint32_t s = t.e0 / BP_SLAB + wid;
+  auto first_groups = [&](uint32_t from) {
+    const uint64_t k = (uint64_t)from + (uint64_t)lane * NW;
+    uint32_t g = gs512[k < s1 ? k : s1 - 1u];
+    asm volatile("" : "+v"(g));  // (waits here, once in 64 slabs, not at each use)
+    return g;
+  };
   u32x4 nx = {0, 0, 0, 0};
   W2Slab<WT> nw{};
-  uint32_t ngs = 0;
+  VT wl[BP_SLAB / WAVE];
+  uint32_t vg = 0;
+  auto entries = [&](uint32_t slab) {
+    const uint64_t o = (uint64_t)slab * BP_SLAB;
+    nx = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(d2 + o) + lane);
+    nw.load(w2 + o, lane);
+  };
+  auto window = [&](uint32_t i) {
+    const VT *vb = val + (uint32_t)__builtin_amdgcn_readlane(vg, i & 63u);
+#pragma unroll
+    for (int j = 0; j < BP_SLAB / WAVE; j++) wl[j] = vb[lane + WAVE * j];
+  };
   if (s < s1) {
-    const uint64_t o = (uint64_t)s * BP_SLAB + lane * BP_EPT;
-    nx = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(d2 + o));
-    nw.load(w2, o);
-    ngs = gs512[s];
+    vg = first_groups(s);
+    window(0);
+    entries(s);
   }
-  for (; s < s1; s += NW) {
+  for (uint32_t it = 1; s < s1; s += NW, it++) {
     const u32x4 cur = nx;
     const W2Slab<WT> cw = nw;
-    const uint32_t gbase = ngs;
+#pragma unroll
+    for (int j = 0; j < BP_SLAB / WAVE; j++)  // u16: 0xFFFF = none
+      wv[lane + WAVE * j] = (sizeof(VT) == 2 && wl[j] == (VT)0xFFFFu) ? 0xFFFFFFFFu : wl[j];
+    if ((it & 63u) == 0) vg = first_groups(s + NW);
+    window(it);
+    entries(s + NW < s1 ? s + NW : s1 - 1u);
     const uint32_t wd[4] = {cur.x, cur.y, cur.z, cur.w};
-    const uint32_t *wt = cw.v;
-    uint32_t ent[BP_EPT];
-#pragma unroll
-    for (int q = 0; q < BP_EPT; q++) ent[q] = (q & 1) ? (wd[q >> 1] >> 16) : (wd[q >> 1] & 0xFFFFu);
-    uint32_t gq[BP_EPT];
-    uint32_t run = gbase - 1u;
-    uint64_t b0 = 0;
-#pragma unroll
-    for (int q = 0; q < BP_EPT; q++) {
-      const uint64_t bq = __ballot(ent[q] >> 15);
-      if (q == 0) b0 = bq;
-      gq[q] = run + lane_rank(bq) + (ent[q] >> 15);
-      run += (uint32_t)__popcll(bq);
-    }
-    const uint32_t w0 = (b0 & 1ull) ? gbase : gbase - 1u;
-    uint32_t wl[BP_SLAB / WAVE];
-#pragma unroll
-    for (int j = 0; j < BP_SLAB / WAVE; j++) {
-      const uint32_t x = val[w0 + lane + WAVE * j];
-      wl[j] = (sizeof(VT) == 2 && x == 0xFFFFu) ? 0xFFFFFFFFu : x;  // u16: 0xFFFF = none
-    }
-    {
-      const uint32_t sn = s + NW < s1 ? s + NW : s1 - 1u;
-      const uint64_t o = (uint64_t)sn * BP_SLAB + lane * BP_EPT;
-      nx = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(d2 + o));
-      nw.load(w2, o);
-      ngs = gs512[sn];
-    }
-#pragma unroll
-    for (int j = 0; j < BP_SLAB / WAVE; j++) wv[lane + WAVE * j] = wl[j];
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     uint32_t x[BP_EPT];
-#pragma unroll
-    for (int q = 0; q < BP_EPT; q++) x[q] = wv[gq[q] - w0];
+    window_values(wd, wv, x);
     const uint32_t sb = s * BP_SLAB;
     const bool whole = sb >= t.e0 && sb + BP_SLAB <= t.e1;  // wave-uniform
 #pragma unroll
     for (int q = 0; q < BP_EPT; q++) {
-      const uint64_t c = (uint64_t)x[q] + wt[q];
+      // saturating at "none", which every sum from "none" stays
+      const uint32_t c = __builtin_elementwise_add_sat(x[q], cw.weight(q));
       const uint32_t pe = sb + WAVE * q + lane;
       const bool mine = whole || (pe >= t.e0 && pe < t.e1);
-      if (mine && x[q] < INFINIT && c < INFINIT)
-        atomicMin(&acc[ent[q] & ((1u << MAXB) - 1u)], (uint32_t)c);
+      if (mine && c < INFINIT) atomicMin(&acc[entry_slot<MAXB>(wd, q)], c);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -820,11 +851,13 @@ __global__ __launch_bounds__(BP_BLOCK) void k_bp_min(const BpTask *tasks, const 
 #pragma unroll
     for (int r = 0; r < (1 << MAXB) / BP_BLOCK; r++) {
       const uint32_t i = threadIdx.x + BP_BLOCK * r;
-      if (i < nb && acc[i] != 0xFFFFFFFFu) atomicMin(&gmin[v0 + i], acc[i]);
+      if (i >= nb) continue;
+      const uint32_t best = acc[acc_slot(i)];
+      if (best != 0xFFFFFFFFu) atomicMin(&gmin[v0 + i], best);
     }
     return;
   }
-  finish_rows<MAXB>(v0, nb, [&](uint32_t i) { return acc[i]; }, a);
+  finish_rows<MAXB>(v0, nb, [&](uint32_t i) { return acc[acc_slot(i)]; }, a);
 }
 
 // rows of the bins split over several tasks, one workgroup per bin; resets
@@ -997,7 +1030,8 @@ __global__ void k_bp_chunks(const uint64_t *goff, const uint32_t *next, uint64_t
   *nch = n;
 }
 
-// phase-2 stream keys: CSR edge e -> (bin of its destination, entry)
+// phase-2 stream keys: CSR edge e -> (bin of its destination, entry: the
+// group-start flag and the destination's accumulator)
 __global__ void k_bp_d2_keys(const uint32_t *col, uint64_t E, int bits, const uint32_t *flag,
                              uint64_t *key, uint32_t *ent) {
   uint64_t e = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
@@ -1006,7 +1040,7 @@ __global__ void k_bp_d2_keys(const uint32_t *col, uint64_t E, int bits, const ui
   for (; e < E; e += stride) {
     const uint32_t v = col[e];
     key[e] = v >> bits;
-    ent[e] = (flag[e] << 15) | (v & mask);
+    ent[e] = (flag[e] << 15) | acc_slot(v & mask);
   }
 }
 
@@ -1037,11 +1071,11 @@ __global__ void k_bp_d2(const uint64_t *key, const uint32_t *ent, uint64_t E, ui
   }
 }
 
-// gs512[s] = groups that start before slab s
-__global__ void k_bp_gs512(const uint32_t *excl, uint64_t E, uint64_t ns, uint32_t *gs512) {
+// gs512[s]: the group that the first entry of slab s belongs to
+__global__ void k_bp_gs512(const uint32_t *excl, const uint32_t *f, uint64_t ns, uint32_t *gs512) {
   uint64_t k = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
   uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (; k < ns; k += stride) gs512[k] = excl[k * BP_SLAB < E ? k * BP_SLAB : E - 1];
+  for (; k < ns; k += stride) gs512[k] = excl[k * BP_SLAB] + f[k * BP_SLAB] - 1u;
 }
 
 // PageRank as a window reduction: sum of contrib[u] over the in-edges
@@ -1475,7 +1509,7 @@ bool build_binned(Graph &g, PrWork &w, int bits) {
     GRUS_LAUNCH_CHECK();
     scan_excl_u32(ctx, f, flag.as<uint32_t>(), E);  // flag now holds the exclusive scan
     pr::k_bp_gs512<<<grid_cap(ctx, nk, BLOCK), BLOCK, 0, ctx.stream>>>(
-        flag.as<uint32_t>(), E, nk, w.bp_gs512.as<uint32_t>());
+        flag.as<uint32_t>(), f, nk, w.bp_gs512.as<uint32_t>());
     GRUS_LAUNCH_CHECK();
     GRUS_HIP(hipMemcpyAsync(bstart.data(), bs.p, (nbins + 1) * 4, hipMemcpyDeviceToHost,
                             ctx.stream));
