@@ -1347,6 +1347,26 @@ uint64_t automatic_task_edges(uint64_t E, uint64_t most) {
 }
 constexpr uint64_t BP_TASK_PR = 1ull << 19, BP_TASK_SP = 1ull << 18;
 
+// Keys and values of a pair sort, and its second copies, in one allocation
+// (an allocation of some megabytes takes 0.3 ms unless the runtime still holds
+// a freed one of the size).  First SSSP call, with the layout built, one
+// allocation for each buffer / for each sort: 2 M edges 7.5 / 3.4 ms, RMAT
+// scale 18 8 / 4.9, scale 20 12 / 7.2.
+struct SortBufs {
+  Buf mem;
+  uint64_t *ka = nullptr, *kb = nullptr;
+  uint32_t *va = nullptr, *vb = nullptr;  // va: only if asked for
+  SortBufs(uint64_t n, bool with_va) {
+    const uint64_t keys = div_up(n * 8, 256) * 256, vals = div_up(n * 4, 256) * 256;
+    mem.alloc(2 * keys + (with_va ? 2 : 1) * vals);
+    char *p = mem.as<char>();
+    ka = reinterpret_cast<uint64_t *>(p);
+    kb = reinterpret_cast<uint64_t *>(p + keys);
+    vb = reinterpret_cast<uint32_t *>(p + 2 * keys);
+    if (with_va) va = reinterpret_cast<uint32_t *>(p + 2 * keys + vals);
+  }
+};
+
 bool build_binned(Graph &g, PrWork &w, int bits) {
   Context &ctx = *g.ctx;
   const CsrView out = g.csr();
@@ -1392,28 +1412,23 @@ bool build_binned(Graph &g, PrWork &w, int bits) {
     // (two chunks in a row that end for their groups hold more than
     // chunk_groups together)
     const uint64_t most = 2 * (G / chunk_groups) + V / pr::BP_SPAN + 4;
-    Buf goff, next, cu, ci, n;
-    goff.alloc((V + 1) * 8);
-    next.alloc((V + 1) * 4);
-    cu.alloc(most * 4);
-    ci.alloc(most * 4);
-    n.alloc(4);
+    Buf tmp;  // goff, then next, the chunks' first rows and groups, and their number
+    tmp.alloc((V + 1) * 12 + (2 * most + 1) * 4);
+    auto *goff = tmp.as<uint64_t>();
+    auto *next = reinterpret_cast<uint32_t *>(goff + V + 1), *cu = next + V + 1, *ci = cu + most;
     pr::k_pb_goff<<<grid_cap(ctx, V + 1, BLOCK), BLOCK, 0, ctx.stream>>>(
-        out.off, V, E, excl.as<uint32_t>(), G, goff.as<uint64_t>());
+        out.off, V, E, excl.as<uint32_t>(), G, goff);
     GRUS_LAUNCH_CHECK();
-    pr::k_bp_next<<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(
-        goff.as<uint64_t>(), V, chunk_groups, next.as<uint32_t>());
+    pr::k_bp_next<<<grid_cap(ctx, V, BLOCK), BLOCK, 0, ctx.stream>>>(goff, V, chunk_groups, next);
     GRUS_LAUNCH_CHECK();
-    pr::k_bp_chunks<<<1, 1, 0, ctx.stream>>>(goff.as<uint64_t>(), next.as<uint32_t>(), V, G,
-                                             (uint32_t)most, cu.as<uint32_t>(), ci.as<uint32_t>(),
-                                             n.as<uint32_t>());
+    pr::k_bp_chunks<<<1, 1, 0, ctx.stream>>>(goff, next, V, G, (uint32_t)most, cu, ci, ci + most);
     GRUS_LAUNCH_CHECK();
-    GRUS_HIP(hipMemcpyAsync(&nch, n.p, 4, hipMemcpyDeviceToHost, ctx.stream));
+    GRUS_HIP(hipMemcpyAsync(&nch, ci + most, 4, hipMemcpyDeviceToHost, ctx.stream));
     ctx.sync();
     w.bp_ch_u0.alloc((nch + 1) * 4);
     w.bp_ch_i0.alloc((nch + 1) * 4);
-    GRUS_HIP(hipMemcpyAsync(w.bp_ch_u0.p, cu.p, (nch + 1) * 4, hipMemcpyDeviceToDevice, ctx.stream));
-    GRUS_HIP(hipMemcpyAsync(w.bp_ch_i0.p, ci.p, (nch + 1) * 4, hipMemcpyDeviceToDevice, ctx.stream));
+    GRUS_HIP(hipMemcpyAsync(w.bp_ch_u0.p, cu, (nch + 1) * 4, hipMemcpyDeviceToDevice, ctx.stream));
+    GRUS_HIP(hipMemcpyAsync(w.bp_ch_i0.p, ci, (nch + 1) * 4, hipMemcpyDeviceToDevice, ctx.stream));
     ctx.sync();
   }
   // group keys (bin << 32 | source), by group id
@@ -1424,45 +1439,32 @@ bool build_binned(Graph &g, PrWork &w, int bits) {
                                                       gkey.as<uint64_t>());
   GRUS_LAUNCH_CHECK();
   slot.alloc(G * 4);
-  {  // slots: (bin, source) order
-    Buf ka, kb, va, vb;
-    ka.alloc(G * 8);
-    kb.alloc(G * 8);
-    va.alloc(G * 4);
-    vb.alloc(G * 4);
+  const uint64_t Gpad = div_up(G, pr::BP_SLAB) * pr::BP_SLAB;
+  const uint64_t nslab1 = Gpad / pr::BP_SLAB;
+  {
+    SortBufs b(G, true);
+    // slots: (bin, source) order
     pr::k_bp_bin_keys<<<grid_cap(ctx, G, BLOCK), BLOCK, 0, ctx.stream>>>(
-        gkey.as<uint64_t>(), G, ka.as<uint64_t>(), va.as<uint32_t>());
+        gkey.as<uint64_t>(), G, b.ka, b.va);
     GRUS_LAUNCH_CHECK();
     uint32_t *sorted = nullptr;
-    sort_pairs_u64_u32(ctx, ka.as<uint64_t>(), kb.as<uint64_t>(), va.as<uint32_t>(),
-                       vb.as<uint32_t>(), G, &sorted, std::max(1, bits_for(nbins - 1)));
+    sort_pairs_u64_u32(ctx, b.ka, b.kb, b.va, b.vb, G, &sorted,
+                       std::max(1, bits_for(nbins - 1)));
     pr::k_bp_slots<<<grid_cap(ctx, G, BLOCK), BLOCK, 0, ctx.stream>>>(sorted, G,
                                                                      slot.as<uint32_t>());
     GRUS_LAUNCH_CHECK();
-    ctx.sync();
-  }
-  const uint64_t Gpad = div_up(G, pr::BP_SLAB) * pr::BP_SLAB;
-  const uint64_t nslab1 = Gpad / pr::BP_SLAB;
-  w.bp_p1.alloc(Gpad * 2);
-  w.bp_rbase.alloc(nslab1 * 4);
-  w.bp_ch_r0.alloc((nch + 1) * 4);
-  {  // phase-1 stream: (chunk, bin, source) order
-    Buf ka, kb, va, vb;
-    ka.alloc(G * 8);
-    kb.alloc(G * 8);
-    va.alloc(G * 4);
-    vb.alloc(G * 4);
+    // phase-1 stream: (chunk, bin, source) order
+    w.bp_p1.alloc(Gpad * 2);
+    w.bp_rbase.alloc(nslab1 * 4);
+    w.bp_ch_r0.alloc((nch + 1) * 4);
     pr::k_bp_p1_keys<<<grid_cap(ctx, G, BLOCK), BLOCK, 0, ctx.stream>>>(
-        gkey.as<uint64_t>(), G, w.bp_ch_i0.as<uint32_t>(), nch, ka.as<uint64_t>(),
-        va.as<uint32_t>());
+        gkey.as<uint64_t>(), G, w.bp_ch_i0.as<uint32_t>(), nch, b.ka, b.va);
     GRUS_LAUNCH_CHECK();
-    uint32_t *sorted = nullptr;
-    sort_pairs_u64_u32(ctx, ka.as<uint64_t>(), kb.as<uint64_t>(), va.as<uint32_t>(),
-                       vb.as<uint32_t>(), G, &sorted, 16 + bits_for(nch));
+    sort_pairs_u64_u32(ctx, b.ka, b.kb, b.va, b.vb, G, &sorted, 16 + bits_for(nch));
     // run flags, offsets and their scan reuse buffers the sort is done with:
     // the other value buffer, and ka (2G u32)
-    uint32_t *rflag = sorted == va.as<uint32_t>() ? vb.as<uint32_t>() : va.as<uint32_t>();
-    uint32_t *rdel = ka.as<uint32_t>();
+    uint32_t *rflag = sorted == b.va ? b.vb : b.va;
+    uint32_t *rdel = reinterpret_cast<uint32_t *>(b.ka);
     uint32_t *rexcl = rdel + G;
     pr::k_bp_p1<<<grid_cap(ctx, Gpad, BLOCK), BLOCK, 0, ctx.stream>>>(
         sorted, gkey.as<uint64_t>(), slot.as<uint32_t>(), G, Gpad, w.bp_ch_u0.as<uint32_t>(),
@@ -1490,20 +1492,17 @@ bool build_binned(Graph &g, PrWork &w, int bits) {
   w.bp_d2.alloc(Epad * 2);
   w.bp_gs512.alloc(nk * 4);
   {
-    Buf ka, kb, vb, bs;
-    ka.alloc(E * 8);
-    kb.alloc(E * 8);
-    vb.alloc(E * 4);
+    SortBufs b(E, false);
+    Buf bs;
     bs.alloc((nbins + 1) * 4);
     pr::k_bp_d2_keys<<<edge_grid, BLOCK, 0, ctx.stream>>>(out.col, E, bits, flag.as<uint32_t>(),
-                                                         ka.as<uint64_t>(), excl.as<uint32_t>());
+                                                         b.ka, excl.as<uint32_t>());
     GRUS_LAUNCH_CHECK();
     uint32_t *ent = nullptr;
-    uint64_t *key = sort_pairs_u64_u32(ctx, ka.as<uint64_t>(), kb.as<uint64_t>(),
-                                       excl.as<uint32_t>(), vb.as<uint32_t>(), E, &ent,
+    uint64_t *key = sort_pairs_u64_u32(ctx, b.ka, b.kb, excl.as<uint32_t>(), b.vb, E, &ent,
                                        std::max(1, bits_for(nbins - 1)));
     // flags of the sorted stream go to whichever entry buffer is free
-    uint32_t *f = (ent == excl.as<uint32_t>()) ? vb.as<uint32_t>() : excl.as<uint32_t>();
+    uint32_t *f = ent == excl.as<uint32_t>() ? b.vb : excl.as<uint32_t>();
     pr::k_bp_d2<<<grid_cap(ctx, Epad, BLOCK), BLOCK, 0, ctx.stream>>>(
         key, ent, E, Epad, (uint32_t)nbins, w.bp_d2.as<uint16_t>(), f, bs.as<uint32_t>());
     GRUS_LAUNCH_CHECK();
@@ -1717,19 +1716,15 @@ bool build_binned_weights(Graph &g, PrWork &w) {
   if (free_b < 24 * E + 4 * Epad + (1ull << 30)) return false;
   w.bp_w2.release();
   {
-    Buf ka, kb, va, vb;
-    ka.alloc(E * 8);
-    kb.alloc(E * 8);
-    va.alloc(E * 4);
-    vb.alloc(E * 4);
+    SortBufs b(E, true);
     pr::k_bp_w2_keys<<<grid_cap(ctx, E, BLOCK), BLOCK, 0, ctx.stream>>>(
-        out.col, out.w, E, w.bp_bits, ka.as<uint64_t>(), va.as<uint32_t>());
+        out.col, out.w, E, w.bp_bits, b.ka, b.va);
     GRUS_LAUNCH_CHECK();
     // the stream is as narrow as the largest weight allows (RMAT inputs
     // with weights below 256 read one byte per edge instead of four)
-    uint32_t *wmax = kb.as<uint32_t>();
+    uint32_t *wmax = reinterpret_cast<uint32_t *>(b.kb);
     GRUS_HIP(hipMemsetAsync(wmax, 0, 4, ctx.stream));
-    pr::k_max_u32<<<grid_cap(ctx, E, BLOCK, 4), BLOCK, 0, ctx.stream>>>(va.as<uint32_t>(), E,
+    pr::k_max_u32<<<grid_cap(ctx, E, BLOCK, 4), BLOCK, 0, ctx.stream>>>(b.va, E,
                                                                        wmax);
     GRUS_LAUNCH_CHECK();
     uint32_t hmax = 0;
@@ -1737,8 +1732,8 @@ bool build_binned_weights(Graph &g, PrWork &w) {
     ctx.sync();
     w.bp_w2_bytes = hmax < 256u ? 1 : hmax < 65536u ? 2 : 4;
     uint32_t *wt = nullptr;
-    sort_pairs_u64_u32(ctx, ka.as<uint64_t>(), kb.as<uint64_t>(), va.as<uint32_t>(),
-                       vb.as<uint32_t>(), E, &wt, std::max(1, bits_for(w.bp_nbins - 1)));
+    sort_pairs_u64_u32(ctx, b.ka, b.kb, b.va,
+                       b.vb, E, &wt, std::max(1, bits_for(w.bp_nbins - 1)));
     w.bp_w2.alloc(Epad * (uint64_t)w.bp_w2_bytes);
     const unsigned grid = grid_cap(ctx, Epad, BLOCK);
     if (w.bp_w2_bytes == 1)
