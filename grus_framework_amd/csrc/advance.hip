@@ -103,12 +103,9 @@ __global__ void k_fill_u64(uint64_t *a, uint64_t n, uint64_t v) {
   for (; i < n; i += stride) a[i] = v;
 }
 
-// reached vertices and their out-edges; one atomic pair per workgroup (a
-// pair from every wave onto the same two addresses serialised at the L2:
-// 0.4 ms at V = 2^24)
+// reached vertices and their out-edges
 __global__ __launch_bounds__(BLOCK) void k_reached(const uint64_t *off, const uint32_t *val,
-                                                   uint64_t V, unsigned long long *acc) {
-  __shared__ unsigned long long s_n[BLOCK / WAVE], s_e[BLOCK / WAVE];
+                                                   uint64_t V, uint64_t *ctl) {
   uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
   uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   unsigned long long n = 0, e = 0;
@@ -118,22 +115,7 @@ __global__ __launch_bounds__(BLOCK) void k_reached(const uint64_t *off, const ui
       e += off[i + 1] - off[i];
     }
   }
-  n = wave_sum(n);
-  e = wave_sum(e);
-  const uint32_t wid = threadIdx.x / WAVE;
-  if (lane_id() == 0) {
-    s_n[wid] = n;
-    s_e[wid] = e;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (uint32_t w = 1; w < BLOCK / WAVE; w++) {
-      n += s_n[w];
-      e += s_e[w];
-    }
-    if (n) atomicAdd(&acc[0], n);
-    if (e) atomicAdd(&acc[1], e);
-  }
+  block_add_spread(n, e, ctl, CTL_REACHED);
 }
 
 }  // namespace
@@ -142,9 +124,9 @@ void reached_stats(Context &ctx, const uint64_t *off, const uint32_t *val, uint6
                    uint64_t *vr, uint64_t *er) {
   // words 40 and 41 of the control block are nobody else's: zero since the
   // context began, and again whenever they were published
-  auto *acc = reinterpret_cast<unsigned long long *>(ctx.d_ctl.p) + 40;
   if (V) {
-    k_reached<<<grid_cap(ctx, V, BLOCK, 8), BLOCK, 0, ctx.stream>>>(off, val, V, acc);
+    k_reached<<<grid_cap(ctx, V, BLOCK, 8), BLOCK, 0, ctx.stream>>>(off, val, V,
+                                                                  ctx.d_ctl.as<uint64_t>());
     GRUS_LAUNCH_CHECK();
   }
   ctx.publish_ctl(42);

@@ -181,7 +181,7 @@ __global__ __launch_bounds__(BLOCK) void k_stamp_commit(const uint8_t *stamp, ui
       }
     }
   }
-  block_add_counts(found, edges, &cnt->next_count, (unsigned long long *)&cnt->next_edges);
+  block_add_spread(found, edges, cnt, CTL_STEP);
 }
 
 __global__ void k_init(uint32_t *label, uint64_t V, uint64_t *visited, const uint64_t *unreachable,
@@ -329,8 +329,7 @@ __global__ __launch_bounds__(BLOCK) void k_pull(CsrView in, const uint64_t *out_
       }
     }
   }
-  block_add_counts(my_found, my_edges, &cnt->next_count,
-                   (unsigned long long *)&cnt->next_edges);
+  block_add_spread(my_found, my_edges, cnt, CTL_STEP);
 }
 
 // Bottom-up step over a candidate list instead of the whole bitmap, for
@@ -363,10 +362,12 @@ constexpr uint32_t SL_PER = 4;                   // edges per thread per level
 constexpr uint32_t SL_F = SL_T;                  // frontier vertices staged in LDS
 constexpr uint64_t SL_E = (uint64_t)SL_T * SL_PER;
 constexpr uint32_t SL_LEVELS = 64;               // levels per launch at most
+constexpr uint64_t SL_COUNT = ~0ull;             // mf0: not known on the host
 
 // what the launch leaves behind (in the control block, after the counters)
 struct SmallLevels {
   uint64_t mf, mu, v_add, e_add;  // frontier edges, unexplored edges, reached sums
+  uint64_t mf0;                   // the first frontier's edges
   uint32_t nf, levels, cur, prev_nf;
 };
 
@@ -385,6 +386,11 @@ __global__ __launch_bounds__(SL_T) void k_small_levels(CsrView g, const uint64_t
   const uint32_t t = threadIdx.x, lane = lane_id(), wid = t / WAVE;
   int cur = cur0;
   uint32_t nf = nf0, prev = 0, lv = 0;
+  if (mf0 == SL_COUNT) {  // the frontier is the source: its edges are counted here
+    const uint32_t u = q[cur0][0];
+    mf0 = g.off[u + 1] - g.off[u];
+    mu0 = mu0 >= mf0 ? mu0 - mf0 : 0;
+  }
   uint64_t mf = mf0, mu = mu0, vadd = 0, eadd = 0;
   // every thread holds the same nf / mf / mu / lv, so the loop is uniform.
   // The host chose push for the first level (its pull -> push switch does
@@ -453,6 +459,7 @@ __global__ __launch_bounds__(SL_T) void k_small_levels(CsrView g, const uint64_t
   }
   if (t == 0) {
     out->mf = mf;
+    out->mf0 = mf0;
     out->mu = mu;
     out->v_add = vadd;
     out->e_add = eadd;
@@ -523,8 +530,7 @@ __global__ __launch_bounds__(BLOCK) void k_pull_sparse(
       if (is_long) longq[slot] = v[j];
     }
   }
-  block_add_counts(my_found, my_edges, &cnt->next_count,
-                   (unsigned long long *)&cnt->next_edges);
+  block_add_spread(my_found, my_edges, cnt, CTL_STEP);
 }
 
 // workgroup-cooperative scan of the vertices whose first K in-edges held no parent
@@ -744,14 +750,20 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
   if (const unsigned blocks = dir == GRUS_DIR_AUTO && !thin ? all_grid(g) : 0) {
     if (run_bfs_all(g, w, src, in, first_in, unreach, alpha, beta, K, blocks, st)) return;
   }
+  // The source's degree, which a copy to the host took 40 us to tell, is left
+  // to the first launch (thin or small levels), unless a source could have so
+  // many edges that the first level is a bottom-up one.
   uint64_t src_deg = 0;
-  {
+  bool deg_known = dir == GRUS_DIR_PULL ||
+                   (dir == GRUS_DIR_AUTO && (double)g.max_deg > (double)(g.E - g.max_deg) / alpha);
+  if (deg_known) {
     uint64_t o[2];
-    GRUS_HIP(hipMemcpy(o, g.off.as<uint64_t>() + src, 16, hipMemcpyDeviceToHost));
+    GRUS_HIP(hipMemcpyAsync(o, g.off.as<uint64_t>() + src, 16, hipMemcpyDeviceToHost, ctx.stream));
+    ctx.sync();
     src_deg = o[1] - o[0];
   }
   uint64_t launches = 0;
-  GRUS_HIP(hipMemsetAsync(cnt, 0, sizeof(StepCounters), ctx.stream));
+  GRUS_HIP(hipMemsetAsync(ctx.d_ctl.p, 0, ctx.d_ctl.bytes, ctx.stream));
   GRUS_HIP(hipEventRecord(ctx.ev0, ctx.stream));
   bfs::k_init<<<grid_cap(ctx, std::max(V, W), BLOCK), BLOCK, 0, ctx.stream>>>(
       label, V, w.visited.as<uint64_t>(), unreach, W, src, w.q[0].as<uint32_t>());
@@ -879,7 +891,9 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
           t_level = now;
         }
         // the launch counted the out-edges of what it expanded, this
-        // frontier's among them, and those of the frontier it left
+        // frontier's among them (mf is 0 while those are not known), and
+        // those of the frontier it left
+        deg_known = true;
         const uint64_t e_new = r.e_add - mf + r.mf;
         level += r.levels;
         cur = (int)r.cur;
@@ -893,18 +907,19 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
         have_bitmap = false;
         continue;
       }
-      if (nf <= bfs::SL_F && mf <= bfs::SL_E) {
+      if (nf <= bfs::SL_F && (!deg_known || mf <= bfs::SL_E)) {
         // small levels: one workgroup runs them back to back on the device
         auto *sl = reinterpret_cast<bfs::SmallLevels *>(ctx.d_ctl.as<uint64_t>() + 8);
         bfs::k_small_levels<<<1, bfs::SL_T, 0, ctx.stream>>>(
-            out, out.off, w.q[0].as<uint32_t>(), w.q[1].as<uint32_t>(), cur, (uint32_t)nf, mf,
-            mu, dir == GRUS_DIR_AUTO ? alpha : 0.0, label, w.visited.as<uint64_t>(), level, sl);
+            out, out.off, w.q[0].as<uint32_t>(), w.q[1].as<uint32_t>(), cur, (uint32_t)nf,
+            deg_known ? mf : bfs::SL_COUNT, mu, dir == GRUS_DIR_AUTO ? alpha : 0.0, label,
+            w.visited.as<uint64_t>(), level, sl);
         GRUS_LAUNCH_CHECK();
         launches++;
         ctx.publish_ctl(8 + sizeof(bfs::SmallLevels) / 8);
         bfs::SmallLevels r;
         std::memcpy(&r, ctx.h_ctl + 8, sizeof r);
-        if (r.nf > V || r.levels == 0 || r.cur > 1)
+        if (r.nf > V || (r.levels == 0 && deg_known) || r.cur > 1)
           raise(GRUS_E_HIP, "bfs small levels reported an impossible state");
         if (trace) {
           auto now = std::chrono::steady_clock::now();
@@ -920,7 +935,8 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
         mf = r.mf;
         mu = r.mu;
         v_reached += r.v_add;
-        e_reached += r.e_add;
+        e_reached += r.e_add + (deg_known ? 0 : r.mf0);
+        deg_known = true;
         have_queue = true;  // the frontier is queue cur; no bitmap of it
         have_bitmap = false;
         continue;
@@ -1052,7 +1068,7 @@ void run_bfs_2s(Graph &g, uint32_t src, uint64_t stage_edges, grus_stats *st) {
     src_deg = o[1] - o[0];
   }
   uint64_t launches = 0;
-  GRUS_HIP(hipMemsetAsync(cnt, 0, sizeof(StepCounters), ctx.stream));
+  GRUS_HIP(hipMemsetAsync(ctx.d_ctl.p, 0, ctx.d_ctl.bytes, ctx.stream));
   GRUS_HIP(hipEventRecord(ctx.ev0, ctx.stream));
   bfs::k_init<<<grid_cap(ctx, std::max(V, W), BLOCK), BLOCK, 0, ctx.stream>>>(
       label, V, w.visited.as<uint64_t>(), nullptr, W, src, w.q[0].as<uint32_t>());

@@ -182,10 +182,26 @@ bool Context::launch_cooperative(const void *kernel, unsigned blocks, unsigned t
 }
 
 namespace {
-__global__ void k_publish_ctl(uint64_t *d, uint64_t *h, uint32_t n) {
+// h[0, n) <- d[0, n) with the sums spread over the lines behind, all cleared
+// (one wave; see block_add_spread)
+__global__ __launch_bounds__(WAVE) void k_publish_ctl(uint64_t *d, uint64_t *h, uint32_t n) {
   const uint32_t i = threadIdx.x;
+  uint64_t x = i < n ? d[i] : 0;
+  // lanes 0..31 read a field's first word in their line, lanes 32..63 its second
+  constexpr uint32_t fields[3] = {CTL_STEP, CTL_REACHED, CTL_DIGEST}, words[3] = {0, 40, 48};
+#pragma unroll
+  for (int f = 0; f < 3; f++) {
+    if (n <= words[f]) break;
+    uint64_t *p = d + CTL_SPREAD + 8 * (i % CTL_LINES) + fields[f] + i / CTL_LINES;
+    uint64_t y = *p;
+    if (y) *p = 0;
+    for (int o = 16; o > 0; o >>= 1) y += __shfl_xor(y, o);
+    const uint64_t a = __shfl(y, 0), b = __shfl(y, 32);
+    if (i == words[f]) x += a;
+    if (i == words[f] + 1) x += b;
+  }
   if (i < n) {
-    h[i] = d[i];
+    h[i] = x;
     d[i] = 0;
   }
 }

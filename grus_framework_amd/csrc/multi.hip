@@ -891,17 +891,34 @@ __device__ __forceinline__ void block_add2(unsigned long long h, unsigned long l
   }
 }
 
-__global__ __launch_bounds__(BLOCK) void k_digest(const uint32_t *row, uint64_t V,
-                                                  unsigned long long *out) {
+// A thread's share of a row's digest, 8 entries in flight: one at a time waits
+// a read's latency for each.
+__device__ __forceinline__ void digest_row(const uint32_t *row, uint64_t V, unsigned long long &h,
+                                           unsigned long long &n) {
+  constexpr int U = 8;
   uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-  uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  unsigned long long h = 0, n = 0;
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (; i + (U - 1) * stride < V; i += U * stride) {
+    uint32_t x[U];
+#pragma unroll
+    for (int q = 0; q < U; q++) x[q] = row[i + q * stride];
+#pragma unroll
+    for (int q = 0; q < U; q++) {
+      h += digest_term(i + q * stride, x[q]);
+      n += (x[q] != INFINIT);
+    }
+  }
   for (; i < V; i += stride) {
-    uint32_t x = row[i];
+    const uint32_t x = row[i];
     h += digest_term(i, x);
     n += (x != INFINIT);
   }
-  block_add2(h, n, out);
+}
+
+__global__ __launch_bounds__(BLOCK) void k_digest(const uint32_t *row, uint64_t V, uint64_t *ctl) {
+  unsigned long long h = 0, n = 0;
+  digest_row(row, V, h, n);
+  block_add_spread(h, n, ctl, CTL_DIGEST);
 }
 
 // digests of the finished BFS lanes (rows of the row-major [lanes][V]
@@ -912,15 +929,8 @@ __global__ __launch_bounds__(BLOCK) void k_digest_rows(const uint32_t *vals, uin
   for (uint32_t k = 0; k < blockIdx.y; k++) m &= m - 1;  // drop the lowest set bits
   if (!m) return;  // block-uniform
   const uint32_t lane = (uint32_t)(__ffsll((unsigned long long)m) - 1);
-  const uint32_t *row = vals + (uint64_t)lane * V;
-  uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   unsigned long long h = 0, n = 0;
-  for (; i < V; i += stride) {
-    const uint32_t x = row[i];
-    h += digest_term(i, x);
-    n += (x != INFINIT);
-  }
+  digest_row(vals + (uint64_t)lane * V, V, h, n);
   block_add2(h, n, out + 2 * lane);
 }
 
@@ -974,11 +984,12 @@ __global__ __launch_bounds__(BLOCK) void k_digest_cols(const T *vals, uint64_t V
 
 void row_digest(Context &ctx, const uint32_t *row, uint64_t V, uint64_t *reached,
                 uint64_t *checksum) {
-  auto *d = reinterpret_cast<unsigned long long *>(ctx.d_ctl.p) + 48;
-  GRUS_HIP(hipMemsetAsync(d, 0, 16, ctx.stream));
-  ms::k_digest<<<grid_cap(ctx, V, BLOCK, 4), BLOCK, 0, ctx.stream>>>(row, V, d);
+  // (the digest's words of the control block are nobody else's: zero since the
+  // context began, and again whenever they were published)
+  ms::k_digest<<<grid_cap(ctx, V, BLOCK, 4), BLOCK, 0, ctx.stream>>>(row, V,
+                                                                   ctx.d_ctl.as<uint64_t>());
   GRUS_LAUNCH_CHECK();
-  ctx.read_ctl(50);
+  ctx.publish_ctl(50);
   *checksum = ctx.h_ctl[48];
   *reached = ctx.h_ctl[49];
 }
