@@ -206,21 +206,67 @@ struct push_job_t {
   __device__ __forceinline__ uint64_t out_degree(vtx_t) const { return 0; }
 };
 
-// ---- BFS finalize: commit new bits, levels, queue, lane counts ----
-__global__ __launch_bounds__(BLOCK) void k_bfs_finalize(const uint64_t *off, uint64_t *visit,
-                                                        uint64_t *front, uint64_t *next,
-                                                        uint32_t *level, uint64_t V,
-                                                        uint64_t running, uint32_t t,
-                                                        LaneStart st, uint32_t *queue,
-                                                        MsCounters *cnt) {
+// The queue entries of a workgroup's span of `items` x FIN_T vertices (bit i of
+// `bits`: the thread's vertex `first` + i * FIN_T has a new frontier), in
+// slots reserved with one atomic, and the span's lanes and out-edges added to
+// the counters: their line is the serial point of these passes.
+template <uint32_t FIN_T>
+__device__ __forceinline__ void queue_span(uint32_t bits, uint64_t first, uint64_t lanes,
+                                           uint64_t edges, uint32_t *queue, MsCounters *cnt) {
   __shared__ unsigned long long s_alive;
-  __shared__ uint32_t s_app[BLOCK / WAVE + 1];
+  __shared__ uint32_t s_wpre[FIN_T / WAVE];
+  __shared__ uint32_t s_base;
   if (threadIdx.x == 0) s_alive = 0;
   __syncthreads();
-  uint64_t edges = 0;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t base = (uint64_t)blockIdx.x * blockDim.x; base < V; base += stride) {
-    uint64_t v = base + threadIdx.x;
+  const uint64_t wm = wave_or(lanes);
+  if (lane_id() == 0 && wm) atomicOr(&s_alive, (unsigned long long)wm);
+  // exclusive scan of the per-thread counts over the workgroup
+  const uint32_t c = __popc(bits);
+  uint32_t incl = c;
+#pragma unroll
+  for (int o = 1; o < WAVE; o <<= 1) {
+    const uint32_t y = __shfl_up(incl, o);
+    if (lane_id() >= (uint32_t)o) incl += y;
+  }
+  const uint32_t wid = threadIdx.x / WAVE;
+  if (lane_id() == WAVE - 1) s_wpre[wid] = incl;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t tot = 0;
+    for (uint32_t w = 0; w < FIN_T / WAVE; w++) {
+      const uint32_t x = s_wpre[w];
+      s_wpre[w] = tot;
+      tot += x;
+    }
+    s_base = tot ? atomicAdd(&cnt->qcount, tot) : 0u;
+    or_bits(&cnt->alive, s_alive);
+  }
+  __syncthreads();
+  uint32_t slot = s_base + s_wpre[wid] + incl - c;
+  for (uint32_t m = bits; m; m &= m - 1) {
+    const uint32_t i = (uint32_t)(__ffs(m) - 1);
+    queue[slot++] = (uint32_t)(first + (uint64_t)i * FIN_T);
+  }
+  block_add_u64(edges, (unsigned long long *)&cnt->front_edges);
+}
+
+// ---- BFS finalize: commit new bits, levels, queue, lane counts ----
+// A workgroup owns a contiguous span of `items` x FIN_T vertices (items <=
+// 32).  With a queue append per 256 vertices, and three atomics from each of
+// 2048 workgroups, the counters' line was what a step waited for (12 ns an
+// atomic).
+template <uint32_t FIN_T>
+__global__ __launch_bounds__(FIN_T) void k_bfs_finalize(const uint64_t *off, uint64_t *visit,
+                                                        uint64_t *front, uint64_t *next,
+                                                        uint32_t *level, uint64_t V,
+                                                        uint32_t items, uint64_t running,
+                                                        uint32_t t, LaneStart st, uint32_t *queue,
+                                                        MsCounters *cnt) {
+  const uint64_t first = (uint64_t)blockIdx.x * items * FIN_T + threadIdx.x;
+  uint32_t bits = 0;
+  uint64_t lanes = 0, edges = 0;
+  for (uint32_t k = 0; k < items; k++) {
+    const uint64_t v = first + (uint64_t)k * FIN_T;
     uint64_t nw = 0;
     if (v < V) {
       uint64_t nx = next[v];
@@ -233,21 +279,18 @@ __global__ __launch_bounds__(BLOCK) void k_bfs_finalize(const uint64_t *off, uin
       if (front[v] != nw) front[v] = nw;
     }
     uint64_t wm = wave_or(nw);
-    if (lane_id() == 0 && wm) atomicOr(&s_alive, (unsigned long long)wm);
     while (wm) {  // level rows: one coalesced 64-vertex store per lane present
       int i = __ffsll((unsigned long long)wm) - 1;
       wm &= wm - 1;
       if ((nw >> i) & 1ull) level[(uint64_t)i * V + v] = t + 1 - st.s[i];
     }
-    uint32_t slot = block_append(&cnt->qcount, nw != 0, s_app);
     if (nw) {
-      queue[slot] = (uint32_t)v;
+      bits |= 1u << k;
+      lanes |= nw;
       edges += off[v + 1] - off[v];
     }
   }
-  __syncthreads();
-  if (threadIdx.x == 0) or_bits(&cnt->alive, s_alive);
-  block_add_u64(edges, (unsigned long long *)&cnt->front_edges);
+  queue_span<FIN_T>(bits, first, lanes, edges, queue, cnt);
 }
 
 // ---- SSSP ----
@@ -735,26 +778,17 @@ __global__ __launch_bounds__(PULL_WAVES * WAVE) void k_sssp_pull(CsrView in, uin
   }
 }
 
-// A workgroup owns a contiguous span of `items` x BLOCK vertices (items <= 32,
-// one bit per item in `bits`): it commits the next bits of its span, counts
-// its new frontier vertices, reserves their queue slots with one atomic and
-// then writes them.  One queue atomic per workgroup instead of one per
-// workgroup-wide step of a grid-stride loop: the single counter address is
-// the serial point of the pass.
-__global__ __launch_bounds__(BLOCK) void k_sssp_finalize(const uint64_t *off, uint64_t *front,
+// Commits the next bits of the vertices; spans and queue as in k_bfs_finalize.
+template <uint32_t FIN_T>
+__global__ __launch_bounds__(FIN_T) void k_sssp_finalize(const uint64_t *off, uint64_t *front,
                                                          uint64_t *next, uint64_t V, uint32_t items,
                                                          uint64_t running, uint32_t *queue,
                                                          MsCounters *cnt) {
-  __shared__ unsigned long long s_alive;
-  __shared__ uint32_t s_wpre[BLOCK / WAVE];
-  __shared__ uint32_t s_base;
-  if (threadIdx.x == 0) s_alive = 0;
-  __syncthreads();
-  const uint64_t first = (uint64_t)blockIdx.x * items * BLOCK + threadIdx.x;
+  const uint64_t first = (uint64_t)blockIdx.x * items * FIN_T + threadIdx.x;
   uint32_t bits = 0;
   uint64_t alive = 0, edges = 0;
   for (uint32_t i = 0; i < items; i++) {
-    const uint64_t v = first + (uint64_t)i * BLOCK;
+    const uint64_t v = first + (uint64_t)i * FIN_T;
     if (v < V) {
       const uint64_t nx = next[v];
       if (nx) next[v] = 0;
@@ -767,36 +801,7 @@ __global__ __launch_bounds__(BLOCK) void k_sssp_finalize(const uint64_t *off, ui
       }
     }
   }
-  const uint64_t wm = wave_or(alive);
-  if (lane_id() == 0 && wm) atomicOr(&s_alive, (unsigned long long)wm);
-  // exclusive scan of the per-thread counts over the workgroup
-  const uint32_t c = __popc(bits);
-  uint32_t incl = c;
-#pragma unroll
-  for (int o = 1; o < WAVE; o <<= 1) {
-    const uint32_t y = __shfl_up(incl, o);
-    if (lane_id() >= (uint32_t)o) incl += y;
-  }
-  const uint32_t wid = threadIdx.x / WAVE;
-  if (lane_id() == WAVE - 1) s_wpre[wid] = incl;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t tot = 0;
-    for (uint32_t w = 0; w < BLOCK / WAVE; w++) {
-      const uint32_t x = s_wpre[w];
-      s_wpre[w] = tot;
-      tot += x;
-    }
-    s_base = tot ? atomicAdd(&cnt->qcount, tot) : 0u;
-    or_bits(&cnt->alive, s_alive);
-  }
-  __syncthreads();
-  uint32_t slot = s_base + s_wpre[wid] + incl - c;
-  for (uint32_t m = bits; m; m &= m - 1) {
-    const uint32_t i = (uint32_t)(__ffs(m) - 1);
-    queue[slot++] = (uint32_t)(first + (uint64_t)i * BLOCK);
-  }
-  block_add_u64(edges, (unsigned long long *)&cnt->front_edges);
+  queue_span<FIN_T>(bits, first, alive, edges, queue, cnt);
 }
 
 // the step's counters to the pinned host mirror, cleared for the next step
@@ -1231,6 +1236,17 @@ std::vector<int> MsEngine::step() {
   // are reported and leave the running set at once); their lanes
   const SlotMask running = busy_ & ~finished_;
   const uint64_t run_lanes = lanes_of(running);
+  // Finalize: spans of up to 32 items a thread, about two workgroups of 1024
+  // threads per CU; of 256 threads on graphs of at most 2^15 vertices, whose
+  // passes are a workgroup's latency.  ms per batch of 64 BFS / 128 SSSP
+  // queries with 2048 workgroups of 256 / 512 of 1024: RMAT s12 0.288, 0.80 /
+  // 0.306, 0.82; s16 0.444, 1.79 / 0.424, 1.73; s18 0.866, 4.14 / 0.653, 3.81;
+  // s20 2.75, 11.3 / 2.13, 10.6; s22 7.9, 37.5 / 7.2, 37.6.
+  const uint32_t fin_t = V <= (1u << 15) ? 256 : 1024;
+  const uint64_t cap_v = (uint64_t)grid_cap(ctx, V, fin_t, 2) * fin_t;
+  const uint32_t items =
+      (uint32_t)std::min<uint64_t>(32, std::max<uint64_t>(1, (V + cap_v - 1) / cap_v));
+  const unsigned fin_grid = (unsigned)std::max<uint64_t>(1, div_up(V, (uint64_t)items * fin_t));
   // the counters are zero here: cleared by the previous publish()
   if (kind_ == MsKind::BFS) {
     const CsrView in = g_.csc();
@@ -1255,9 +1271,10 @@ std::vector<int> MsEngine::step() {
     for (int i = 0; i < 64; i++) st.s[i] = start_[i];
     // (a pull step left long_count set; finalize uses the other counters,
     // which are still zero)
-    ms::k_bfs_finalize<<<grid_cap(ctx, V, BLOCK, 8), BLOCK, 0, ctx.stream>>>(
+    (fin_t == 256 ? ms::k_bfs_finalize<256> : ms::k_bfs_finalize<1024>)<<<fin_grid, fin_t, 0,
+                                                                       ctx.stream>>>(
         out.off, visit_.as<uint64_t>(), front_.as<uint64_t>(), next_.as<uint64_t>(),
-        vals_.as<uint32_t>(), V, run_lanes, (uint32_t)t_, st, queue_.as<uint32_t>(), cnt);
+        vals_.as<uint32_t>(), V, items, run_lanes, (uint32_t)t_, st, queue_.as<uint32_t>(), cnt);
     GRUS_LAUNCH_CHECK();
   } else {
     // A step pulls when the frontier's out-edges are over a third of all edges
@@ -1300,12 +1317,8 @@ std::vector<int> MsEngine::step() {
             next_.as<uint64_t>(), vals_.as<uint32_t>(), cnt);
       GRUS_LAUNCH_CHECK();
     }
-    // spans of up to 32 x BLOCK vertices, about 8 workgroups per CU
-    const uint64_t cap_v = (uint64_t)grid_cap(ctx, V, BLOCK, 8) * BLOCK;
-    const uint32_t items = (uint32_t)std::min<uint64_t>(32, std::max<uint64_t>(1, (V + cap_v - 1) / cap_v));
-    const uint64_t span = (uint64_t)items * BLOCK;
-    const unsigned fin_grid = (unsigned)std::max<uint64_t>(1, (V + span - 1) / span);
-    ms::k_sssp_finalize<<<fin_grid, BLOCK, 0, ctx.stream>>>(
+    (fin_t == 256 ? ms::k_sssp_finalize<256> : ms::k_sssp_finalize<1024>)<<<fin_grid, fin_t, 0,
+                                                                         ctx.stream>>>(
         out.off, front_.as<uint64_t>(), next_.as<uint64_t>(), V, items, run_lanes,
         queue_.as<uint32_t>(), cnt);
     GRUS_LAUNCH_CHECK();
