@@ -687,21 +687,44 @@ __device__ __forceinline__ void finish_rows(uint64_t v0, uint32_t nb, Best best_
   const uint32_t lane = lane_id(), wid = threadIdx.x / WAVE;
   uint32_t nearm = 0, farm = 0;
   uint64_t edges = 0;
+  // U rows at a time, each kind of read issued for all of them before any is
+  // used (one row after the other waited three latencies a row; with that and
+  // the reservations below awaited one by one, an SSSP run on RMAT scale 17
+  // took 0.402 ms instead of 0.392, on scale 20 0.743 instead of 0.731)
+  constexpr int U = BPR < 8 ? BPR : 8;
 #pragma unroll
-  for (int r = 0; r < BPR; r++) {
-    const uint32_t i = threadIdx.x + BP_BLOCK * r;
-    if (i >= nb) continue;
-    const uint32_t best = best_of(i);
-    const uint64_t v = v0 + i;
-    if (best < INFINIT && best < a.dist[v]) {
-      a.dist[v] = best;
-      if (best < a.T_thr) {
-        a.near_stamp[v] = a.near_id;
-        nearm |= 1u << r;
-        edges += a.out_off[v + 1] - a.out_off[v];
-      } else if (a.far_stamp[v] != a.far_id) {
-        a.far_stamp[v] = a.far_id;
-        farm |= 1u << r;
+  for (int rb = 0; rb < BPR; rb += U) {
+    uint32_t best[U], d[U], stamp[U];
+    uint64_t o0[U], o1[U];
+#pragma unroll
+    for (int q = 0; q < U; q++) {
+      const uint32_t i = threadIdx.x + BP_BLOCK * (rb + q);
+      best[q] = i < nb ? best_of(i) : 0xFFFFFFFFu;
+      d[q] = i < nb ? a.dist[v0 + i] : 0u;
+    }
+#pragma unroll
+    for (int q = 0; q < U; q++) {
+      const uint64_t v = v0 + threadIdx.x + BP_BLOCK * (rb + q);
+      o0[q] = o1[q] = 0;
+      stamp[q] = a.far_id;
+      if (best[q] < INFINIT && best[q] < d[q]) {
+        a.dist[v] = best[q];
+        if (best[q] < a.T_thr) {
+          a.near_stamp[v] = a.near_id;
+          nearm |= 1u << (rb + q);
+          o0[q] = a.out_off[v];
+          o1[q] = a.out_off[v + 1];
+        } else {
+          stamp[q] = a.far_stamp[v];
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < U; q++) {
+      edges += o1[q] - o0[q];
+      if (stamp[q] != a.far_id) {
+        a.far_stamp[v0 + threadIdx.x + BP_BLOCK * (rb + q)] = a.far_id;
+        farm |= 1u << (rb + q);
       }
     }
   }
@@ -726,11 +749,15 @@ __device__ __forceinline__ void finish_rows(uint64_t v0, uint32_t nb, Best best_
     total += s_w[w];
     etot += s_e[w];
   }
-  if (threadIdx.x == 0) {
-    s_base[0] = (total >> 16) ? atomicAdd(&a.cnt->next_count, total >> 16) : 0u;
+  // (a wave each: the two reservations are awaited together.  cnt is the
+  // context's control block, whose lines behind take the edges)
+  if (threadIdx.x == 0) s_base[0] = (total >> 16) ? atomicAdd(&a.cnt->next_count, total >> 16) : 0u;
+  if (threadIdx.x == WAVE)
     s_base[1] = (total & 0xFFFFu) ? atomicAdd(&a.cnt->far_count, total & 0xFFFFu) : 0u;
-    if (etot) atomicAdd((unsigned long long *)&a.cnt->next_edges, etot);
-  }
+  if (threadIdx.x == 2 * WAVE && etot)
+    atomicAdd(reinterpret_cast<unsigned long long *>(a.cnt) + CTL_SPREAD +
+                  8 * (blockIdx.x % CTL_LINES) + CTL_STEP + 1,
+              etot);
   __syncthreads();
   const uint32_t excl = before + inc - mine;
   uint32_t pn = s_base[0] + (excl >> 16), pf = s_base[1] + (excl & 0xFFFFu);

@@ -212,6 +212,7 @@ __global__ void k_init(uint32_t *dist, uint64_t V, uint32_t src, uint32_t *q0,
   uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
   uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   if (i == 0) *cnt = StepCounters{};
+  if (i < 8 * CTL_LINES) reinterpret_cast<uint64_t *>(cnt)[CTL_SPREAD + i] = 0;
   for (; i < V; i += stride) {
     dist[i] = (i == src) ? 0u : INFINIT;  // SSSPInit sssp.cu:21
     if (i == 0) {
