@@ -695,7 +695,6 @@ bool run_bfs_all(Graph &g, BfsWork &w, uint32_t src, const CsrView &in, const ui
     raise(GRUS_E_HIP, "bfs reported an impossible state");
   if (st) {
     float ms = 0;
-    GRUS_HIP(hipEventSynchronize(ctx.ev1));  // (reached; the runtime may not know yet)
     GRUS_HIP(hipEventElapsedTime(&ms, ctx.ev0, ctx.ev1));
     *st = grus_stats{};
     st->device_ms = ms;

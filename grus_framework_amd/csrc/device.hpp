@@ -136,14 +136,6 @@ __device__ __forceinline__ void block_add_spread(unsigned long long a, unsigned 
   }
 }
 
-// The end of a one-wave kernel that has stored its results to coherent pinned
-// memory: the host, which polls *at, sees them all once it reads seq there.
-constexpr uint32_t CTL_SEQ = 511;  // word of the host's mirror of the control block
-__device__ __forceinline__ void publish_done(uint64_t *at, uint64_t seq) {
-  __threadfence_system();
-  if (lane_id() == 0) __hip_atomic_store(at, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 // One 64-bit sum, to one address (skipped when zero).
 __device__ __forceinline__ void block_add_u64(unsigned long long sum, unsigned long long *out) {
   __shared__ unsigned long long s_s[1024 / WAVE];

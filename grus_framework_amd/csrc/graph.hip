@@ -7,7 +7,6 @@
 // reference's host-side serial loops (csr_tocsc, include/graph.cuh:273-303).
 #include <algorithm>
 #include <atomic>
-#include <chrono>
 #include <cstring>
 
 #include "device.hpp"
@@ -131,8 +130,7 @@ Context::Context(int dev) {
   GRUS_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
   GRUS_HIP(hipEventCreate(&ev0));
   GRUS_HIP(hipEventCreate(&ev1));
-  GRUS_HIP(hipHostMalloc((void **)&h_ctl, 4096, hipHostMallocCoherent));
-  std::memset(h_ctl, 0, 4096);
+  GRUS_HIP(hipHostMalloc((void **)&h_ctl, 4096, hipHostMallocDefault));
   d_ctl.alloc(4096);
   GRUS_HIP(hipMemsetAsync(d_ctl.p, 0, 4096, stream));
   GRUS_HIP(hipStreamSynchronize(stream));
@@ -186,8 +184,7 @@ bool Context::launch_cooperative(const void *kernel, unsigned blocks, unsigned t
 namespace {
 // h[0, n) <- d[0, n) with the sums spread over the lines behind, all cleared
 // (one wave; see block_add_spread)
-__global__ __launch_bounds__(WAVE) void k_publish_ctl(uint64_t *d, uint64_t *h, uint32_t n,
-                                                      uint64_t seq) {
+__global__ __launch_bounds__(WAVE) void k_publish_ctl(uint64_t *d, uint64_t *h, uint32_t n) {
   const uint32_t i = threadIdx.x;
   uint64_t x = i < n ? d[i] : 0;
   // lanes 0..31 read a field's first word in their line, lanes 32..63 its second
@@ -207,31 +204,14 @@ __global__ __launch_bounds__(WAVE) void k_publish_ctl(uint64_t *d, uint64_t *h, 
     h[i] = x;
     d[i] = 0;
   }
-  publish_done(h + CTL_SEQ, seq);
 }
 }  // namespace
 
 void Context::publish_ctl(size_t n) {
   if (n > 64) raise(GRUS_E_INVALID, "publish_ctl: at most 64 words");
-  k_publish_ctl<<<1, 64, 0, stream>>>(d_ctl.as<uint64_t>(), h_ctl, (uint32_t)n, ++seq);
+  k_publish_ctl<<<1, 64, 0, stream>>>(d_ctl.as<uint64_t>(), h_ctl, (uint32_t)n);
   GRUS_LAUNCH_CHECK();
-  wait_published(h_ctl + CTL_SEQ, seq);
-}
-
-void Context::wait_published(const uint64_t *at, uint64_t value) {
-  // the kernels before the publishing one have ended when it starts, and its
-  // words are there before the number: nothing else of the stream is awaited
-  const auto t0 = std::chrono::steady_clock::now();
-  for (uint32_t k = 1; __atomic_load_n(at, __ATOMIC_ACQUIRE) != value; k++) {
-    __builtin_ia32_pause();
-    if (k % 256 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(1)) {
-      // a long step, or a failed one: the runtime waits and says so
-      GRUS_HIP(hipStreamSynchronize(stream));
-      if (__atomic_load_n(at, __ATOMIC_ACQUIRE) != value)
-        raise(GRUS_E_HIP, "a step's counters were not published");
-      return;
-    }
-  }
+  GRUS_HIP(hipStreamSynchronize(stream));
 }
 
 void Context::read_ctl(size_t n) {

@@ -112,13 +112,6 @@ struct Context {
   // zeroes them on the device; then wait.  Replaces a copy and the next
   // step's memset (two launches) in per-level read-backs.
   void publish_ctl(size_t n);
-  // wait until a kernel of this stream has published `value` at a word of
-  // pinned memory (publish_done): read there, a step's result is known 6 us
-  // before the runtime reports the kernel's end (RMAT scale 20 SSSP, 15 steps:
-  // 911 us with the runtime's wait, 832 with this; BFS scale 24, 8 steps a
-  // source: 849 and 811).  Waits past 1 ms are the runtime's.
-  void wait_published(const uint64_t *at, uint64_t value);
-  uint64_t seq = 0;  // of publish_ctl
   // whether cooperative grids may be launched: under a CU mask or beside other
   // contexts' kernels a grid might not be resident
   bool cooperative() const { return !cu_masked && !shared_device && !coop_refused; }

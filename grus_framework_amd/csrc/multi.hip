@@ -805,15 +805,12 @@ __global__ __launch_bounds__(FIN_T) void k_sssp_finalize(const uint64_t *off, ui
 }
 
 // the step's counters to the pinned host mirror, cleared for the next step
-constexpr uint32_t MS_SEQ = 31;  // word of the mirror that numbers them
-__global__ __launch_bounds__(WAVE) void k_publish(uint64_t *d, uint64_t *h, uint32_t n,
-                                                  uint64_t seq) {
+__global__ void k_publish(uint64_t *d, uint64_t *h, uint32_t n) {
   const uint32_t i = threadIdx.x;
   if (i < n) {
     h[i] = d[i];
     d[i] = 0;
   }
-  publish_done(h + MS_SEQ, seq);
 }
 
 // ---- extraction ----
@@ -1039,7 +1036,6 @@ void MsEngine::init() {
   cnt_.alloc(sizeof(MsCounters));
   push_cnt_.alloc(sizeof(StepCounters));
   hmirror_.alloc(256, Mem::HostPinned);
-  memset(hmirror_.p, 0, 256);
   if (kind_ == MsKind::BFS) {
     vals_.alloc((uint64_t)lanes_ * V * 4 + 8);  // level[lane][v]
     fill_u64(ctx, visit_.as<uint64_t>(), V + 1, 0);
@@ -1211,9 +1207,9 @@ MsCounters MsEngine::publish() {
   Context &ctx = *ctx_;
   static_assert(sizeof(MsCounters) % 8 == 0 && sizeof(MsCounters) <= 128, "counter block");
   ms::k_publish<<<1, 64, 0, ctx.stream>>>(cnt_.as<uint64_t>(), hmirror_.as<uint64_t>(),
-                                          (uint32_t)(sizeof(MsCounters) / 8), ++seq_);
+                                          (uint32_t)(sizeof(MsCounters) / 8));
   GRUS_LAUNCH_CHECK();
-  ctx.wait_published(hmirror_.as<uint64_t>() + ms::MS_SEQ, seq_);
+  ctx.sync();
   MsCounters h;
   memcpy(&h, hmirror_.p, sizeof h);
   return h;

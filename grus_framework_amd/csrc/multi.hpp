@@ -102,7 +102,6 @@ class MsEngine {
   uint32_t src_[128] = {};  // each slot's source (a widened SSSP slot restarts from it)
   bool narrow_ = false;
   uint64_t t_ = 0;         // global step counter
-  uint64_t seq_ = 0;       // of publish()
   uint64_t qn_ = 0, front_edges_ = 0;
   uint32_t pull_per_ = 0;  // SSSP: in-edges per wave of a pull step; 0: steps only push
   Buf visit_, front_, next_, vals_, queue_, longq_, row_, rows_, digest_, srcs_dev_, cnt_, push_cnt_;
