@@ -211,7 +211,7 @@ def main():
                     help="comma list of extras to run: pagerank,cc,sssp (or sssp_rmat, "
                          "sssp_grid),cu,serving,capped; batched (the batched engines "
                          "alone, run only when named)")
-    ap.add_argument("--leg-limit", type=float, default=240.0,
+    ap.add_argument("--leg-limit", type=float, default=150.0,
                     help="seconds after which an extra leg with no result is abandoned "
                          "(0 = never)")
     ap.add_argument("--copy-calibration", action="store_true",
