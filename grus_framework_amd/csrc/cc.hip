@@ -13,7 +13,9 @@
 //   CAS, so parent[x] <= x holds throughout and every root is the minimum of
 //   its tree.  Rows of generated graphs ascend, so the first neighbour is the
 //   lowest: on RMAT s20 the hooks alone put 93% of the vertices with edges
-//   into the giant component, and the rest hold 0.3% of the edges.
+//   into the giant component, and the rest hold 0.3% of the edges.  Where the
+//   sample finds too many edges outside, every vertex's first two neighbours
+//   are linked before the rest.
 // method 1 -- the reference's min-label propagation through the push
 //   operator (advance.hpp), frontier deduplicated by round stamps.
 #include <algorithm>
@@ -90,29 +92,42 @@ __device__ __forceinline__ uint32_t climb(uint32_t v, uint32_t *parent, uint32_t
   return p;
 }
 
+// What the sampled edges tell, in the scratch.
+struct Giant {
+  uint32_t root;  // the most frequent root
+  uint32_t more;  // too many edges lie outside it
+};
+
 // A full climb by every vertex at once is slow on long chains (each starts
 // before those above it have shortened theirs), so the first pass stops
 // after FIRST_HOPS and k_link_rest climbs the rest: 4096 x 4096 grid 1.19 ->
 // 0.44 ms in all; RMAT s22, where FIRST_HOPS reach every root, 0.13 either way.
 constexpr uint32_t FIRST_HOPS = 8;
-__global__ __launch_bounds__(BLOCK) void k_compress(uint32_t *parent, uint64_t V, uint32_t hops) {
+__global__ __launch_bounds__(BLOCK) void k_compress(uint32_t *parent, uint64_t V, uint32_t hops,
+                                                    const Giant *if_more) {
+  if (if_more && !if_more->more) return;
   uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
   uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (; v < V; v += stride) climb((uint32_t)v, parent, GRUS_NO_VERTEX, hops);
 }
 
-// The most frequent root among kSample pseudo-random vertices (ties: the
-// smaller root) to *giant, in one workgroup with a vertex per thread: each
-// thread counts the samples equal to its own, so the mode needs no sort and
-// no trip to the host.
-constexpr uint32_t kSample = 1024;
-__global__ __launch_bounds__(kSample) void k_sample_mode(uint32_t *parent, uint64_t V,
-                                                         uint64_t seed, uint32_t *giant) {
+// The most frequent root among the heads of kSample pseudo-random edges
+// (ties: the smaller root) to *out, in one workgroup with an edge per thread:
+// each thread counts the samples equal to its own, so the mode needs no sort
+// and no trip to the host (256 of them 5 us, 1024 in 16 waves 22).  Edges and
+// not vertices, because what is left to do is the edges outside: more of them
+// than half the vertices, and the links of k_link_two cost less than theirs.
+// `again`: only if `more` was found before.
+constexpr uint32_t kSample = 256;
+__global__ __launch_bounds__(kSample) void k_sample_mode(CsrView g, uint32_t *parent,
+                                                         uint64_t seed, bool again, Giant *out) {
   __shared__ uint4 s_root[kSample / 4];
   __shared__ unsigned long long s_best[kSample / WAVE];
+  if (again && !out->more) return;
   const uint32_t t = threadIdx.x;
-  const uint32_t mine =
-      climb((uint32_t)(mix64(seed + t) % V), parent, GRUS_NO_VERTEX, 0xFFFFFFFFu);
+  uint32_t mine = GRUS_NO_VERTEX;
+  if (g.E)
+    mine = climb(edge_col(g, mix64(seed + t) % g.E), parent, GRUS_NO_VERTEX, 0xFFFFFFFFu);
   reinterpret_cast<uint32_t *>(s_root)[t] = mine;
   __syncthreads();
   uint32_t n = 0;
@@ -130,7 +145,28 @@ __global__ __launch_bounds__(kSample) void k_sample_mode(uint32_t *parent, uint6
   __syncthreads();
   if (t == 0) {
     for (uint32_t w = 1; w < kSample / WAVE; w++) best = s_best[w] > best ? s_best[w] : best;
-    *giant = 0xFFFFFFFFu - (uint32_t)best;
+    const uint32_t outside = kSample - (uint32_t)(best >> 32);
+    *out = {0xFFFFFFFFu - (uint32_t)best, (double)outside * g.E > (double)kSample / 2 * g.V};
+  }
+}
+
+// The hooks alone join few vertices where first neighbours are not often the
+// smallest of a neighbourhood (numberings without order, rows in any order):
+// half of the edges and more are then outside the giant component, and to link
+// them all takes longer than everything else.  There the edges to every
+// vertex's first two neighbours are linked too, as Afforest does.  ms per call
+// without / with them: uniform edges, V = 2^16, 8 a vertex 0.134 / 0.080; V =
+// 2^20, 16 a vertex 1.76 / 0.25; RMAT s20 with its rows in random order 19.3 /
+// 0.19.  Where the hooks do (RMAT s22) the three idle launches take 13 us.
+__global__ __launch_bounds__(BLOCK) void k_link_two(CsrView g, const Giant *giant,
+                                                    uint32_t *parent) {
+  if (!giant->more) return;
+  uint64_t u = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (; u < g.V; u += stride) {
+    const uint64_t beg = g.off[u], end = g.off[u + 1];
+    for (uint64_t e = beg; e < end && e < beg + 2; e++)
+      link((uint32_t)u, edge_col(g, e), parent);
   }
 }
 
@@ -140,9 +176,9 @@ __global__ __launch_bounds__(kSample) void k_sample_mode(uint32_t *parent, uint6
 // coalesced read of the parents: RMAT s22 spent 325 of 503 us here with a
 // wave per vertex; the whole call now takes 126 us on the device.
 constexpr uint64_t REST_LANE = 16;
-__global__ __launch_bounds__(BLOCK) void k_link_rest(CsrView g, const uint32_t *giant_p,
+__global__ __launch_bounds__(BLOCK) void k_link_rest(CsrView g, const Giant *giant_p,
                                                      uint32_t *parent) {
-  const uint32_t giant = *giant_p;
+  const uint32_t giant = giant_p->root;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   const uint64_t first = blockIdx.x * (uint64_t)blockDim.x + (threadIdx.x & ~(uint32_t)(WAVE - 1));
   for (uint64_t base = first; base < g.V; base += stride) {  // wave-uniform
@@ -198,7 +234,7 @@ struct job_t {
 
 // The device buffers of one CC run beyond the graph and the labels.
 struct CcSpace {
-  uint32_t *giant = nullptr;            // method 0: root of the giant component
+  cc::Giant *giant = nullptr;           // method 0: what the sampled edges tell
   uint32_t *q[2] = {nullptr, nullptr};  // method 1: frontier queues, V + 1 each
   uint32_t *stamp = nullptr;            // method 1: round stamps, V + 1
   uint32_t *stamp_id = nullptr;         // method 1: last stamp handed out (host)
@@ -220,15 +256,21 @@ void cc_core(Graph &g, int method, uint32_t *label, CcSpace &sp, grus_stats *st)
     if (V) {
       cc::k_hook_first<<<grid, BLOCK, 0, ctx.stream>>>(gr, label);
       GRUS_LAUNCH_CHECK();
-      cc::k_compress<<<grid, BLOCK, 0, ctx.stream>>>(label, V, cc::FIRST_HOPS);
+      cc::k_compress<<<grid, BLOCK, 0, ctx.stream>>>(label, V, cc::FIRST_HOPS, nullptr);
       GRUS_LAUNCH_CHECK();
-      cc::k_sample_mode<<<1, cc::kSample, 0, ctx.stream>>>(label, V, 0x5EEDull, sp.giant);
+      cc::k_sample_mode<<<1, cc::kSample, 0, ctx.stream>>>(gr, label, 0x5EEDull, false, sp.giant);
+      GRUS_LAUNCH_CHECK();
+      cc::k_link_two<<<grid, BLOCK, 0, ctx.stream>>>(gr, sp.giant, label);
+      GRUS_LAUNCH_CHECK();
+      cc::k_compress<<<grid, BLOCK, 0, ctx.stream>>>(label, V, cc::FIRST_HOPS, sp.giant);
+      GRUS_LAUNCH_CHECK();
+      cc::k_sample_mode<<<1, cc::kSample, 0, ctx.stream>>>(gr, label, 0x5EEDull, true, sp.giant);
       GRUS_LAUNCH_CHECK();
       cc::k_link_rest<<<grid, BLOCK, 0, ctx.stream>>>(gr, sp.giant, label);
       GRUS_LAUNCH_CHECK();
-      cc::k_compress<<<grid, BLOCK, 0, ctx.stream>>>(label, V, 0xFFFFFFFFu);
+      cc::k_compress<<<grid, BLOCK, 0, ctx.stream>>>(label, V, 0xFFFFFFFFu, nullptr);
       GRUS_LAUNCH_CHECK();
-      launches += 5;
+      launches += 8;
     }
     iterations = 2;  // the hooks, then the rest
   } else {
@@ -293,7 +335,7 @@ void run_cc(Graph &g, int method, grus_stats *st) {
   CcSpace sp;
   if (method == 0) {
     w.giant.ensure(kGiantBytes);
-    sp.giant = w.giant.as<uint32_t>();
+    sp.giant = w.giant.as<cc::Giant>();
   } else {
     if (w.cap_v < V) {
       w.q[0].alloc((V + 1) * 4);
@@ -338,7 +380,7 @@ void run_cc_in(Graph &g, int method, uint32_t *label, void *scratch, uint64_t sc
   PushWork push;  // borrowed buffers only: its own Bufs stay empty
   uint32_t stamp_id = 0;
   if (method == 0) {
-    sp.giant = reinterpret_cast<uint32_t *>(base);
+    sp.giant = reinterpret_cast<cc::Giant *>(base);
   } else {
     uint64_t at = 0;
     auto take = [&](uint64_t bytes) {
