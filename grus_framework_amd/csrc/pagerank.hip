@@ -108,6 +108,8 @@ struct PrWork {
     uint64_t ntask = 0, nmulti = 0;
     uint64_t edges = 0;  // task size it was cut with (0: not cut)
   } bp_pr, bp_sp;
+  double peak = 0;  // dest_peak(), of the out-edges whose offsets are peak_for
+  const void *peak_for = nullptr;
   uint64_t bp_G = 0, bp_nch = 0;
   uint32_t bp_nbins = 0;
   int bp_bits = 0;
@@ -928,6 +930,30 @@ __global__ void k_bp_w2(const uint32_t *wt, uint64_t E, uint64_t Epad, WT *w2) {
   }
 }
 
+// *most = sampled edges whose destination lies in the fullest of PEAK_RANGES
+// equal ranges of the vertices (one workgroup; E > 0)
+constexpr uint32_t PEAK_T = 1024, PEAK_RANGES = 256, PEAK_SAMPLES = 65536;
+__global__ __launch_bounds__(PEAK_T) void k_dest_peak(CsrView g, uint32_t *most) {
+  __shared__ uint32_t s_n[PEAK_RANGES], s_most;
+  const uint32_t t = threadIdx.x;
+  if (t < PEAK_RANGES) s_n[t] = 0;
+  if (t == 0) s_most = 0;
+  __syncthreads();
+  constexpr int U = 16;
+  for (uint32_t i0 = t; i0 < PEAK_SAMPLES; i0 += U * PEAK_T) {
+    uint32_t c[U];
+#pragma unroll
+    for (int q = 0; q < U; q++)
+      c[q] = edge_col(g, (uint64_t)(i0 + q * PEAK_T) * g.E / PEAK_SAMPLES);
+#pragma unroll
+    for (int q = 0; q < U; q++) atomicAdd(&s_n[(uint64_t)c[q] * PEAK_RANGES / g.V], 1u);
+  }
+  __syncthreads();
+  if (t < PEAK_RANGES) atomicMax(&s_most, s_n[t]);
+  __syncthreads();
+  if (t == 0) *most = s_most;
+}
+
 __global__ void k_max_u32(const uint32_t *a, uint64_t n, uint32_t *out) {
   uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
   uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -1353,26 +1379,70 @@ constexpr uint32_t BP_CHUNK_GROUPS = 32768;
 
 // Automatic bin width and task sizes.  2^14-vertex bins leave a graph of V
 // vertices V / 2^14 bins to spread over 256 CUs; narrower bins make more and
-// smaller accumulators but more groups to write and read.  Tasks of E / 512
-// edges give every CU two, down to 2^14 edges (E / 128 below that), where a
-// task's own clearing and finishing shows, and up to a size of each use: the
-// bins of the largest graphs are split as little as fills the chip, because
-// every piece adds its whole bin to memory.  Measured on RMAT, ms per SSSP
-// run / us per PageRank iteration:
-//   s16  2^14 bins, 2^18 edges 0.95 / 65   2^11 and E/128 0.49 / 23
-//   s18  1.01 / 69                          2^11, 2^14 edges 0.63 / 42
-//   s20  1.14 / 84                          2^12 and E/512 0.92 / 78
-//   s21  - / 152                            2^12 and E/512 1.17 / 121
-//   s22  2.15 / 250                         2^13 and E/512 1.96 / 227
-//   s24  SSSP 2^14, 2^18 edges 6.28, 2^19 6.52; PageRank 1035, 2^19 956
-int automatic_bin_bits(uint64_t V) {
-  return V <= (1ull << 19) ? 11 : V <= (1ull << 21) ? 12 : V <= (1ull << 22) ? 13 : PB_BITS;
+// smaller accumulators, but shorter runs of group values to write and read.
+// What is best depends on how evenly the destinations spread over the bins
+// (dest_peak): the densest of 256 equal ranges of vertices holds 1.05 to 1.2
+// times its share of the edges of uniform graphs, small worlds and the like,
+// 1.4 to 1.8 times under hubs numbered without order, 30 times on RMAT.
+//
+// Width: two workgroups of the narrowest bins fit a CU, and about 256 bins
+// fill the chip; where a few ranges hold most of the edges, narrower bins
+// share them out and the rest are short anyway.  us per PageRank iteration
+// with 2^12 / 2^13 / 2^14-vertex bins, tasks as below:
+//   RMAT s20 64 / 74 / 92, s21 100 / 113 / 130, s22 215 / 198 / 211
+//   shuffled s20 72 / 79 / 97, s21 142 / 126 / 141, s22 334 / 255 / 223
+//   uniform V = 2^20, 16 edges a vertex 45 / 50 / 69, 100 edges 277 / 187 / 150
+//   V = 2^21, 4 edges 36 / 34 / 38, 40 edges 231 / 222 / 192
+//   V = 2^22, 4 edges 64 / 61 / 57, 40 edges 577 / 460 / 497
+// and at 2^16 and 2^18 vertices 2^11 was best on all of them.
+//
+// Tasks of an even graph: whole bins, or equal pieces of them once they are
+// larger than `most`.  Cut at E / 512, half of the bins were a little larger
+// and cut in two (V = 2^22, 4 edges: 61 -> 85 us; V = 2^20, 8: 30 -> 46).
+// Otherwise E / 512 edges, two tasks a CU, down to 2^14 edges (E / 128 below
+// that), where a task's own clearing and finishing shows, and up to a size of
+// each use: the bins of the largest graphs are split as little as fills the
+// chip, because every piece adds its whole bin to memory.  RMAT, ms per SSSP
+// run / us per PageRank iteration, 2^14-vertex bins and 2^18 edges a task
+// against these rules:
+//   s16 0.95 / 65 and 0.49 / 15, s18 1.01 / 69 and 0.51 / 29
+//   s20 1.14 / 84 and 0.73 / 64, s22 2.15 / 250 and 1.46 / 198
+//   s24 SSSP 2^18 6.28, 2^19 6.52; PageRank 1035 and 956
+constexpr double EVEN_PEAK = 1.35, SKEW_PEAK = 4;
+constexpr uint64_t BP_TASK_PR = 1ull << 19, BP_TASK_SP = 1ull << 18;
+
+int automatic_bin_bits(uint64_t V, uint64_t E, double peak) {
+  if (V <= (1ull << 19)) return 11;
+  if (peak >= SKEW_PEAK) return V <= (1ull << 21) ? 12 : V <= (1ull << 22) ? 13 : PB_BITS;
+  if (E > (1ull << 26)) return PB_BITS;
+  return V <= (1ull << 20) ? 12 : V <= (1ull << 21) ? 13 : PB_BITS;
 }
-uint64_t automatic_task_edges(uint64_t E, uint64_t most) {
+uint64_t automatic_task_edges(uint64_t E, uint32_t nbins, double peak, uint64_t most) {
+  const uint64_t bin = div_up(E, nbins), parts = div_up(bin, most);
+  if (peak < EVEN_PEAK && nbins * parts >= 128) {
+    const uint64_t piece = div_up(bin, parts);
+    return std::max<uint64_t>(256, piece + piece / 4);
+  }
   const uint64_t fill = std::max(E / 512, std::min<uint64_t>(E / 128, 1ull << 14));
   return std::max<uint64_t>(256, std::min(fill, most));
 }
-constexpr uint64_t BP_TASK_PR = 1ull << 19, BP_TASK_SP = 1ull << 18;
+
+// the densest of PEAK_RANGES equal ranges of destinations, in multiples of its
+// share, by PEAK_SAMPLES edges at equal distances; found out once
+double dest_peak(Graph &g, PrWork &w) {
+  const CsrView out = g.csr();
+  if (out.E == 0) return 1;
+  if (w.peak_for != out.off) {
+    Context &ctx = *g.ctx;
+    pr::k_dest_peak<<<1, pr::PEAK_T, 0, ctx.stream>>>(
+        out, reinterpret_cast<uint32_t *>(ctx.d_ctl.as<uint64_t>() + 33));
+    GRUS_LAUNCH_CHECK();
+    ctx.read_ctl(34);
+    w.peak = (double)(uint32_t)ctx.h_ctl[33] * pr::PEAK_RANGES / pr::PEAK_SAMPLES;
+    w.peak_for = out.off;
+  }
+  return w.peak;
+}
 
 // Keys and values of a pair sort, and its second copies, in one allocation
 // (an allocation of some megabytes takes 0.3 ms unless the runtime still holds
@@ -1786,9 +1856,10 @@ bool sssp_binned_ready(Graph &g) {
   PrWork &w = *g.pr;
   if (w.bp_unusable_for == out.off) return false;
   if (w.bp_for != out.off) {  // a layout PageRank already built is used as it is
-    const int bits = std::min(
-        ctx.tuning.pr_bin_bits ? (int)ctx.tuning.pr_bin_bits : automatic_bin_bits(g.V),
-        pr::BP_MAX_BITS);
+    const int bits = std::min(ctx.tuning.pr_bin_bits
+                                  ? (int)ctx.tuning.pr_bin_bits
+                                  : automatic_bin_bits(g.V, g.E, dest_peak(g, w)),
+                              pr::BP_MAX_BITS);
     if (!build_binned(g, w, bits)) {
       w.bp_unusable_for = out.off;
       return false;
@@ -1796,8 +1867,9 @@ bool sssp_binned_ready(Graph &g) {
   }
   if (w.bp_sp.edges == 0)
     build_binned_tasks(g, w, w.bp_sp,
-                       ctx.tuning.pr_task_edges ? ctx.tuning.pr_task_edges
-                                                : automatic_task_edges(g.E, BP_TASK_SP));
+                       ctx.tuning.pr_task_edges
+                           ? ctx.tuning.pr_task_edges
+                           : automatic_task_edges(g.E, w.bp_nbins, dest_peak(g, w), BP_TASK_SP));
   if (w.bp_w2_for != out.off && !build_binned_weights(g, w)) {
     w.bp_unusable_for = out.off;
     return false;
@@ -1887,13 +1959,16 @@ void run_pagerank(Graph &g, float alpha, int iters, grus_stats *st) {
   // binned push (automatic choice on HBM graphs that fit it; bins of at
   // most 2^14 destinations, the LDS accumulators)
   if ((layout == 0 || layout == 4) && g.placement == GRUS_PLACE_HBM) {
-    const int bb = std::min(ctx.tuning.pr_bin_bits ? bits : automatic_bin_bits(V), pr::BP_MAX_BITS);
+    const double peak = dest_peak(g, w);
+    const int bb = std::min(ctx.tuning.pr_bin_bits ? bits : automatic_bin_bits(V, g.E, peak),
+                            pr::BP_MAX_BITS);
     bool binned = true;
     if (w.bp_for != out.off || w.bp_bits != bb) binned = build_binned(g, w, bb);
-    const uint64_t te = ctx.tuning.pr_task_edges ? ctx.tuning.pr_task_edges
-                                                 : automatic_task_edges(g.E, BP_TASK_PR);
-    if (binned && w.bp_pr.edges != te) build_binned_tasks(g, w, w.bp_pr, te);
     if (binned) {
+      const uint64_t te = ctx.tuning.pr_task_edges
+                              ? ctx.tuning.pr_task_edges
+                              : automatic_task_edges(g.E, w.bp_nbins, peak, BP_TASK_PR);
+      if (w.bp_pr.edges != te) build_binned_tasks(g, w, w.bp_pr, te);
       run_binned(g, w, alpha, iters, st);
       return;
     }

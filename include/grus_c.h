@@ -125,8 +125,9 @@ typedef struct grus_tuning {
                              (same ranks up to float rounding).  Every layout
                              is bit-identical run to run. */
   uint32_t pr_bin_bits;   /* blocked / binned layout bin width, log2 (0 =
-                             automatic: 14; layout 4: 11 to 14 by the number
-                             of vertices, at most 14) */
+                             automatic: 14; layout 4: 11 to 14 by the numbers
+                             of vertices and edges and by how evenly the
+                             edges' heads spread, at most 14) */
   uint32_t sssp_pull_div; /* SSSP: a round pulls (each unsettled vertex takes
                              the min over its in-neighbours in the frontier)
                              when the frontier's out-edges exceed
@@ -140,8 +141,10 @@ typedef struct grus_tuning {
                              round); 0 = automatic (256), at most 256 */
   uint32_t pr_task_edges; /* binned PageRank layout: edges per accumulation
                              task; a bin with more edges is split over several
-                             tasks (0 = automatic: about E / 512, at most
-                             2^19; 2^18 for SSSP pull rounds) */
+                             tasks (0 = automatic: about E / 512, or equal
+                             pieces of the bins where the edges' heads spread
+                             evenly; at most 5/4 of 2^19, of 2^18 for SSSP
+                             pull rounds) */
   uint32_t sssp_pull_layout; /* SSSP pull rounds: 0 automatic (= 2 where it
                              applies, else 1); 1 window reduction over the
                              in-edges; 2 binned push over PageRank's binned

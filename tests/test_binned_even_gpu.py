@@ -1,0 +1,77 @@
+"""Bin widths and task sizes of the binned layout by how evenly the destinations
+spread: uniform graphs, hubs numbered without order and RMAT's hubs at low ids
+choose different ones, none of which may change a rank or a distance; and a
+uniform graph takes no longer than with the widest bins asked for."""
+import numpy as np
+import pytest
+
+import grus_framework_amd as grus
+
+pytestmark = pytest.mark.gpu
+
+
+def uniform(V, degree, weights=False):
+    rng = np.random.default_rng(V + degree)
+    key = np.unique(rng.integers(0, V, V * degree) * V + rng.integers(0, V, V * degree))
+    off = np.zeros(V + 1, np.uint64)
+    off[1:] = np.cumsum(np.bincount(key // V, minlength=V))
+    w = rng.integers(1, 100, len(key)).astype(np.uint32) if weights else None
+    return off, (key % V).astype(np.uint32), w
+
+
+def tuned(bits, task_edges):
+    c = grus.Context(0)
+    t = c.tuning
+    t.pr_layout, t.pr_bin_bits, t.pr_task_edges = 4, bits, task_edges
+    c.tuning = t
+    return c
+
+
+# sizes around the changes of width; 1 edge a vertex leaves many rows empty
+@pytest.mark.parametrize("V,degree", [((1 << 19) + 1, 5), (1 << 20, 3), ((1 << 20) + 77, 4),
+                                      ((1 << 21) + 1, 2), (1200000, 1)])
+def test_ranks_do_not_depend_on_the_cut(ctx, V, degree):
+    csr = uniform(V, degree)
+    with grus.Graph.from_csr(ctx, *csr) as g:
+        want = grus.pagerank(g, iters=4)[0].view(np.uint32)
+    with tuned(14, 1 << 18) as c, grus.Graph.from_csr(c, *csr) as g:
+        assert (grus.pagerank(g, iters=4)[0].view(np.uint32) == want).all()
+
+
+@pytest.mark.parametrize("V,degree", [(5000, 20), (700001, 6), ((1 << 20) + 3, 6)])
+def test_distances(ctx, oracle, V, degree):
+    csr = uniform(V, degree, weights=True)
+    with grus.Graph.from_csr(ctx, *csr) as g:
+        got, st = grus.sssp(g, 1)
+        assert (got == oracle.sssp(oracle.CSR(*csr), 1)).all()
+
+
+def test_shuffled_hubs(ctx):
+    with grus.Graph.rmat(ctx, 21, edge_factor=4) as g:
+        off, col, _ = g.csr()
+    V = len(off) - 1
+    p = np.random.default_rng(2).permutation(V)
+    u = p[np.repeat(np.arange(V), np.diff(off).astype(np.int64))]
+    order = np.argsort(u, kind="stable")
+    off2 = np.zeros(V + 1, np.uint64)
+    off2[1:] = np.cumsum(np.bincount(u, minlength=V))
+    csr = off2, p[col.astype(np.int64)][order].astype(np.uint32), None
+    with grus.Graph.from_csr(ctx, *csr, symmetric=True) as g:
+        want = grus.pagerank(g, iters=3)[0].view(np.uint32)
+    with tuned(11, 1 << 15) as c, grus.Graph.from_csr(c, *csr, symmetric=True) as g:
+        assert (grus.pagerank(g, iters=3)[0].view(np.uint32) == want).all()
+
+
+def device_ms(c, csr):
+    with grus.Graph.from_csr(c, *csr) as g:
+        grus.pagerank(g, copy=False)
+        return min(grus.pagerank(g, copy=False)[1].device_ms for _ in range(5))
+
+
+@pytest.mark.parametrize("V", [1 << 21, 1 << 22])
+def test_uniform_no_slower_than_widest_bins(ctx, V):
+    csr = uniform(V, 4)
+    with tuned(14, 1 << 18) as c:
+        widest = device_ms(c, csr)
+    # two runs of one setting differ by a few percent
+    assert device_ms(ctx, csr) < 1.2 * widest
