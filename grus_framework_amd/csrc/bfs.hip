@@ -637,11 +637,19 @@ unsigned all_grid(const Graph &g) {
   return div_up(W, ctx.cu_count) > bfs::ALL_OWN ? 0 : std::min(want, (unsigned)ctx.cu_count);
 }
 
-// a whole traversal in one launch (bfs_all.hpp); false when the runtime
-// refuses the launch
+// what a traversal has come to between launches
+struct Progress {
+  uint32_t level = 0, pulls = 0;
+  uint64_t nf = 1, mf = 0, mu = 0, prev_nf = 0, v_reached = 0, e_reached = 0;
+};
+
+// a whole traversal in one launch (bfs_all.hpp), or the rest of one (t.level >
+// 0: its frontier in w.front[0]).  t.nf afterwards: 0, or the frontier of the
+// thin levels it was left at, in queue 0.  False when the runtime refuses the
+// launch.
 bool run_bfs_all(Graph &g, BfsWork &w, uint32_t src, const CsrView &in, const uint32_t *first_in,
                  const uint64_t *unreach, double alpha, double beta, uint32_t K, unsigned blocks,
-                 grus_stats *st) {
+                 Progress *t) {
   Context &ctx = *g.ctx;
   const uint64_t W = g.words();
   w.front2.ensure((W + 1) * 8);
@@ -658,9 +666,9 @@ bool run_bfs_all(Graph &g, BfsWork &w, uint32_t src, const CsrView &in, const ui
   p.first_in = first_in;
   p.unreachable = unreach;
   p.visited = w.visited.as<uint64_t>();
-  p.front[0] = w.front[0].as<uint64_t>();
-  p.front[1] = w.front[1].as<uint64_t>();
-  p.front[2] = w.front2.as<uint64_t>();
+  p.front[t->level % 3] = w.front[0].as<uint64_t>();
+  p.front[(t->level + 1) % 3] = w.front[1].as<uint64_t>();
+  p.front[(t->level + 2) % 3] = w.front2.as<uint64_t>();
   p.huge[0] = w.q[0].as<uint32_t>();
   p.huge[1] = w.q[1].as<uint32_t>();
   p.label = g.result.as<uint32_t>();
@@ -668,6 +676,14 @@ bool run_bfs_all(Graph &g, BfsWork &w, uint32_t src, const CsrView &in, const ui
   p.K = K;
   p.W = (uint32_t)W;
   p.own = (uint32_t)div_up(W, blocks);
+  p.level = t->level;
+  p.nf = (uint32_t)t->nf;
+  p.prev_nf = (uint32_t)t->prev_nf;
+  p.mf = t->mf;
+  p.mu = t->mu;
+  p.thin_nf = bfs::SL_F;
+  p.thin_mf = bfs::SL_E;
+  p.queue = w.q[0].as<uint32_t>();
   p.alpha = alpha;
   p.beta = beta;
   p.flags = w.all_flags.as<unsigned long long>();
@@ -675,7 +691,7 @@ bool run_bfs_all(Graph &g, BfsWork &w, uint32_t src, const CsrView &in, const ui
   p.ctl = reinterpret_cast<bfs::AllCtl *>(ctx.d_ctl.as<uint64_t>() + 8);
   p.timeout = ctx.wall_ticks_per_ms() * 20000;  // 20 s per barrier wait
   const size_t lds = (W + 2 * p.own) * 8;
-  GRUS_HIP(hipEventRecord(ctx.ev0, ctx.stream));
+  if (t->level == 0) GRUS_HIP(hipEventRecord(ctx.ev0, ctx.stream));
   if (blocks == 1) {
     bfs::k_bfs_all<<<1, bfs::ALL_T, lds, ctx.stream>>>(p);
     GRUS_LAUNCH_CHECK();
@@ -691,19 +707,17 @@ bool run_bfs_all(Graph &g, BfsWork &w, uint32_t src, const CsrView &in, const ui
   std::memcpy(&r, ctx.h_ctl + 8, sizeof r);
   w.all_tag += std::min<uint32_t>(r.levels, (uint32_t)bfs::ALL_MAX_V) + 2;
   if (r.status) raise(GRUS_E_TIMEOUT, "bfs aborted (barrier timeout)");
-  if (r.levels == 0 || r.levels > g.V + 1 || r.v_reached > g.V)
+  if (r.levels == 0 || r.levels > g.V + 1 || r.v_reached > g.V || r.nf != r.queued ||
+      r.nf > bfs::SL_F)
     raise(GRUS_E_HIP, "bfs reported an impossible state");
-  if (st) {
-    float ms = 0;
-    GRUS_HIP(hipEventElapsedTime(&ms, ctx.ev0, ctx.ev1));
-    *st = grus_stats{};
-    st->device_ms = ms;
-    st->iterations = r.levels;
-    st->pull_iterations = r.pulls;
-    st->vertices_reached = r.v_reached;
-    st->edges_reached = r.e_reached;
-    st->kernel_launches = 1;
-  }
+  t->level += r.levels;
+  t->pulls += r.pulls;
+  t->nf = r.nf;
+  t->mf = r.mf;
+  t->mu = r.mu;
+  t->prev_nf = r.prev_nf;
+  t->v_reached += r.v_reached;
+  t->e_reached += r.e_reached;
   return true;
 }
 }  // namespace
@@ -747,28 +761,30 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
   const uint32_t K = ctx.tuning.bu_thread_edges ? ctx.tuning.bu_thread_edges : 32;
 
   const uint4 *thin = dir == GRUS_DIR_PULL ? nullptr : thin_rows(g, w);
-  if (const unsigned blocks = dir == GRUS_DIR_AUTO && !thin ? all_grid(g) : 0) {
-    if (run_bfs_all(g, w, src, in, first_in, unreach, alpha, beta, K, blocks, st)) return;
-  }
+  Progress all;
+  unsigned all_blocks = dir == GRUS_DIR_AUTO && !thin ? all_grid(g) : 0;
+  if (all_blocks && !run_bfs_all(g, w, src, in, first_in, unreach, alpha, beta, K, all_blocks, &all))
+    all_blocks = 0;
   // The source's degree, which a copy to the host took 40 us to tell, is left
   // to the first launch (thin or small levels), unless a source could have so
   // many edges that the first level is a bottom-up one.
   uint64_t src_deg = 0;
-  bool deg_known = dir == GRUS_DIR_PULL ||
+  bool deg_known = all_blocks || dir == GRUS_DIR_PULL ||
                    (dir == GRUS_DIR_AUTO && (double)g.max_deg > (double)(g.E - g.max_deg) / alpha);
-  if (deg_known) {
+  if (deg_known && !all_blocks) {
     uint64_t o[2];
     GRUS_HIP(hipMemcpyAsync(o, g.off.as<uint64_t>() + src, 16, hipMemcpyDeviceToHost, ctx.stream));
     ctx.sync();
     src_deg = o[1] - o[0];
   }
-  uint64_t launches = 0;
-  GRUS_HIP(hipMemsetAsync(ctx.d_ctl.p, 0, ctx.d_ctl.bytes, ctx.stream));
-  GRUS_HIP(hipEventRecord(ctx.ev0, ctx.stream));
-  bfs::k_init<<<grid_cap(ctx, std::max(V, W), BLOCK), BLOCK, 0, ctx.stream>>>(
-      label, V, w.visited.as<uint64_t>(), unreach, W, src, w.q[0].as<uint32_t>());
-  GRUS_LAUNCH_CHECK();
-  launches++;
+  uint64_t launches = 1;
+  if (!all_blocks) {
+    GRUS_HIP(hipMemsetAsync(ctx.d_ctl.p, 0, ctx.d_ctl.bytes, ctx.stream));
+    GRUS_HIP(hipEventRecord(ctx.ev0, ctx.stream));
+    bfs::k_init<<<grid_cap(ctx, std::max(V, W), BLOCK), BLOCK, 0, ctx.stream>>>(
+        label, V, w.visited.as<uint64_t>(), unreach, W, src, w.q[0].as<uint32_t>());
+    GRUS_LAUNCH_CHECK();
+  }
 
   int cur = 0;               // index of the current queue / bitmap
   bool have_queue = true;    // current frontier available as a queue
@@ -778,6 +794,22 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
   uint64_t mu = g.E >= src_deg ? g.E - src_deg : 0;
   uint64_t v_reached = 1, e_reached = src_deg;
   uint32_t level = 0, pull_levels = 0;
+  bool timed = false;  // the last launch has been recorded as the end
+  auto take = [&] {    // what the launches of bfs_all.hpp have come to
+    cur = 0;
+    have_queue = true;
+    have_bitmap = pull = false;
+    level = all.level;
+    pull_levels = all.pulls;
+    nf = all.nf;
+    mf = all.mf;
+    mu = all.mu;
+    prev_nf = all.prev_nf;
+    v_reached = all.v_reached;
+    e_reached = all.e_reached;
+    timed = nf == 0;
+  };
+  if (all_blocks) take();
   // a bottom-up step with few unvisited vertices left scans a list of them
   // instead of every bitmap word; the host knows how many are left from
   // the vertices reached so far and the in-degree-0 count
@@ -789,6 +821,18 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
   while (nf) {
     // every level discovers at least one new vertex, so V levels is a bound
     if (level > V) raise(GRUS_E_HIP, "bfs did not converge within V levels");
+    // (a traversal that left bfs_all.hpp is here with the queue that thin
+    // levels left, and pushes)
+    if (all_blocks && (nf > bfs::SL_F || mf > bfs::SL_E || (double)mf > (double)mu / alpha)) {
+      all = {level, pull_levels, nf, mf, mu, prev_nf, v_reached, e_reached};
+      queue_to_bitmap(ctx, w.q[cur].as<uint32_t>(), (uint32_t)nf, w.front[0].as<uint64_t>(), W);
+      if (run_bfs_all(g, w, src, in, first_in, unreach, alpha, beta, K, all_blocks, &all)) {
+        launches += 3;
+        take();
+        continue;
+      }
+      all_blocks = 0;
+    }
     if (dir == GRUS_DIR_AUTO) {
       if (!pull && (double)mf > (double)mu / alpha) pull = true;
       else if (pull && (double)nf < (double)V / beta && nf < prev_nf) pull = false;
@@ -1002,11 +1046,13 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
     cur ^= 1;
     level++;
   }
-  GRUS_HIP(hipEventRecord(ctx.ev1, ctx.stream));
-  GRUS_HIP(hipEventSynchronize(ctx.ev1));
-  float ms = 0;
-  GRUS_HIP(hipEventElapsedTime(&ms, ctx.ev0, ctx.ev1));
+  if (!timed) {
+    GRUS_HIP(hipEventRecord(ctx.ev1, ctx.stream));
+    GRUS_HIP(hipEventSynchronize(ctx.ev1));
+  }
   if (st) {
+    float ms = 0;
+    GRUS_HIP(hipEventElapsedTime(&ms, ctx.ev0, ctx.ev1));
     *st = grus_stats{};
     st->device_ms = ms;
     st->iterations = level;

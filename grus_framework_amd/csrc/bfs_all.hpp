@@ -45,10 +45,24 @@ constexpr int ALL_TAG = 40;               // flags: tag | huge rows | vertices, 
 constexpr int ALL_NF = 20;
 static_assert(ALL_MAX_V < (1ull << ALL_NF), "a frontier's size fits its field");
 
+// A launch ends early after ALL_THIN thin levels in a row, pushes of at most
+// thin_nf vertices and thin_mf out-edges: k_small_levels runs those at 2.7 us
+// each, and here every one costs the whole grid a bitmap's reads and a barrier
+// (4.5 us in one workgroup, 5.7 to 9 in a grid).  What k_small_levels leaves
+// comes back here.  Chains, grids and rings with a hub, ms without / with the
+// hand-over: 20000 levels 114 / 55, 599 levels 4.9 / 2.8, 10001 levels 96 / 40.
+// RMAT never has so many thin levels in a row.
+constexpr uint32_t ALL_THIN = 8;
+
 struct AllCtl {
-  uint32_t status, levels, pulls, abort;
+  uint32_t status, levels, pulls, abort;  // levels: of this launch; status 1: aborted
   unsigned long long v_reached, e_reached;
   uint32_t huge[4];  // huge rows listed for the frontier of level L, in slot L % 3
+  // left at a thin frontier: its vertices (in the queue, `queued` of them
+  // counted there), their out-edges, the unexplored edges, the level before
+  uint32_t nf, queued;
+  unsigned long long mf, mu;
+  uint32_t prev_nf, pad;
 };
 
 struct AllParams {
@@ -59,6 +73,13 @@ struct AllParams {
   uint32_t *huge[2];  // huge rows of the frontier of level L, in list L % 2
   uint32_t *label;
   uint32_t src, K, W, own;  // own = words per workgroup at most
+  // a traversal that goes on: level > 0, its frontier in front[level % 3],
+  // visited and levels in place, and the counts as AllCtl has them
+  uint32_t level, nf, prev_nf;
+  uint64_t mf, mu;
+  uint32_t thin_nf;
+  uint64_t thin_mf;
+  uint32_t *queue;  // of the frontier left (may be huge[0]: a thin frontier lists none)
   double alpha, beta;
   unsigned long long *flags;  // [2 parities][2 counts][ALL_MAX_G]
   uint32_t tag;               // of the first barrier; never used before
@@ -170,31 +191,54 @@ __global__ __launch_bounds__(ALL_T) void k_bfs_all(AllParams p) {
     s_n = s_e = 0;
     s_abort = 0;
   }
+  uint32_t level = p.level, pulls = 0, streak = 0;
+  const bool fresh = level == 0;
+  uint64_t found = 0;  // huge rows of a frontier that goes on
   for (uint32_t k = wid; k < mine; k += NW) {
     const uint32_t w = k * G + b;
-    const uint64_t at = w == (p.src >> 6) ? 1ull << (p.src & 63) : 0ull;
-    const uint64_t vis = p.unreachable[w] | at;
     const uint64_t v = (uint64_t)w * 64 + lane;
-    if (v < V) p.label[v] = v == p.src ? 0u : INFINIT;
+    uint64_t at = w == (p.src >> 6) ? 1ull << (p.src & 63) : 0ull, vis;
+    if (fresh) {
+      vis = p.unreachable[w] | at;
+      if (v < V) p.label[v] = v == p.src ? 0u : INFINIT;
+    } else {
+      vis = p.visited[w];
+      at = p.front[level % 3][w];
+      if (((at >> lane) & 1ull) && p.out.off[v + 1] - p.out.off[v] > ALL_HUGE) {
+        found += 1ull << ALL_NF;
+        st_agent(&p.huge[level & 1][atomicAdd(&p.ctl->huge[level % 3], 1u)], (uint32_t)v);
+      }
+    }
     if (lane == 0) {
       s_vis[k] = vis;
       s_cur[k] = at;
-      st_agent64(&p.visited[w], vis);
-      st_agent64(&p.front[0][w], at);
-      st_agent64(&p.front[1][w], 0);
+      if (fresh) {
+        st_agent64(&p.visited[w], vis);
+        st_agent64(&p.front[0][w], at);
+      }
+      st_agent64(&p.front[(level + 1) % 3][w], 0);
     }
   }
-  uint64_t nf = 1, mf = p.out.off[p.src + 1] - p.out.off[p.src], prev_nf = 0, x, y;
-  uint64_t mu = p.out.E >= mf ? p.out.E - mf : 0, v_reached = 1, e_reached = mf;
-  uint32_t nhuge = mf > ALL_HUGE ? 1u : 0u;
-  if (b == 0 && t == 0) st_agent(&p.huge[0][0], p.src);
-  uint32_t level = 0, pulls = 0;
+  uint64_t nf = p.nf, mf = p.mf, mu = p.mu, prev_nf = p.prev_nf, x, y;
+  if (fresh) {
+    nf = 1;
+    mf = p.out.off[p.src + 1] - p.out.off[p.src];
+    mu = p.out.E >= mf ? p.out.E - mf : 0;
+    if (mf > ALL_HUGE && b == 0 && t == 0) {
+      found = 1ull << ALL_NF;
+      st_agent(&p.huge[0][0], p.src);
+    }
+  }
+  uint64_t v_reached = fresh ? 1 : 0, e_reached = fresh ? mf : 0;
   bool pull = false, pushed = false;  // pushed: own frontier words await their owner
   __syncthreads();
-  bool ok = barrier(0, 0, &x, &y);
+  bool ok = barrier(found, 0, &x, &y);
+  uint32_t nhuge = (uint32_t)(x >> ALL_NF);
   while (ok && nf) {
     if (!pull && (double)mf > (double)mu / p.alpha) pull = true;
     else if (pull && (double)nf < (double)V / p.beta && nf < prev_nf) pull = false;
+    streak = !pull && nf <= p.thin_nf && mf <= p.thin_mf ? streak + 1 : 0;
+    if (streak > ALL_THIN) break;
     const uint64_t *cur = p.front[level % 3];
     uint64_t *next = p.front[(level + 1) % 3], *clear = p.front[(level + 2) % 3];
     uint64_t n = 0;  // new vertices, and huge rows among them from bit ALL_NF on
@@ -399,9 +443,26 @@ __global__ __launch_bounds__(ALL_T) void k_bfs_all(AllParams p) {
     e_reached += mf;
     level++;
   }
+  if (ok && nf) {  // left at a thin frontier: its levels, if they await their owner, and the queue
+    for (uint32_t k = wid; k < mine; k += NW) {
+      const uint64_t m = ld_agent64(&p.front[level % 3][k * G + b]);
+      const uint32_t v = (k * G + b) * 64 + lane;
+      uint32_t at = 0;
+      if (lane == 0 && m) at = atomicAdd(&p.ctl->queued, (uint32_t)__popcll(m));
+      at = __shfl(at, 0);
+      if ((m >> lane) & 1ull) {
+        p.label[v] = level;
+        p.queue[at + lane_rank(m)] = v;
+      }
+    }
+  }
   if (b == 0 && t == 0) {
+    p.ctl->nf = ok ? (uint32_t)nf : 0u;
+    p.ctl->mf = mf;
+    p.ctl->mu = mu;
+    p.ctl->prev_nf = (uint32_t)prev_nf;
     p.ctl->status = ok ? 0u : 1u;
-    p.ctl->levels = level;
+    p.ctl->levels = level - p.level;
     p.ctl->pulls = pulls;
     p.ctl->v_reached = v_reached;
     p.ctl->e_reached = e_reached;
