@@ -17,8 +17,11 @@
 // step per level whatever it holds.  Load is light while the engines of a
 // kind, each serving one query at a time, would empty the queue within the
 // time of one batch (running means of both times, per kind; until a batch
-// has run, 16 waiting queries start one, so that its time is known), or while at most solo_max queries wait when
-// the caller sets it.  Measured on RMAT scale 22 at 1100 queries/s (50/50
+// has run, 16 waiting queries, 32 above 2^20 vertices, start one, so that its
+// time is known), or while at most solo_max queries wait when the caller sets
+// it.  A burst still arrives when its first queries start a batch; the rest
+// joins that one, and no engine beside it takes a few (bursts of 64 SSSP
+// queries at RMAT s24: mean of 24 of them 190 -> 151 ms).  Measured on RMAT scale 22 at 1100 queries/s (50/50
 // BFS/SSSP): p50 5 ms when every query is served alone, 99-120 ms when a
 // queue of 8 already starts a batch (which then slows the single queries
 // beside it).
@@ -68,8 +71,23 @@ double now_us() {
 // them on RMAT scale 22, as two or three at scale 16, where a single query is
 // mostly launches.  Taken to cost 32 until one had run, 128 queries at scale
 // 16 were all served alone and no batch ever ran (256 mixed queries 23-35 ms;
-// 8.4 ms with the first batch started at 16).
-constexpr size_t kLearnBatch = 16;
+// 8.4 ms with the first batch started at 16).  24 queries of a kind, one batch
+// of most of them / all alone, BFS and SSSP: RMAT s16 0.75 / 1.7 and 2.6 / 3.4
+// ms, s20 1.4 / 2.4 and 10.1 / 8.6, s22 5.8 / 4.1 and 33 / 30, s24 14.9 / 10.4
+// and 137 / 111; 32 of them at s24 13.5 / 15.6 and 134 / 156.
+size_t learn_batch(uint64_t V) { return V <= (1ull << 20) ? 16 : 32; }
+
+// Running mean: plain up to 8 values, then weight 1/8 to the newest.  (The
+// first query of a worker makes its workspace: with 1/8 from the second value
+// on, its time stood for the others' for dozens of queries.)  0: none yet.
+struct Mean {
+  double ms = 0;
+  int n = 0;
+  void add(double x) {
+    n = std::min(n + 1, 8);
+    ms += (x - ms) / n;
+  }
+};
 
 struct Query {
   uint64_t id;
@@ -296,7 +314,7 @@ class ServerImpl : public Server {
           auto room = [&] { return refused_at != mem_epoch_; };
           auto ready = [&] {
             if (stop_ || (eng && eng->active())) return true;
-            if (pending_[kind].empty()) return false;
+            if (pending_[kind].size() <= (young_[kind].ei == ei ? 0 : young_[kind].free)) return false;
             return eng != nullptr || room();
           };
           if (eng && !eng->active() && !first && release_ms_ >= 0 && !stop_) {
@@ -342,6 +360,18 @@ class ServerImpl : public Server {
               take.push_back(pending_[kind].front());
               pending_[kind].pop_front();
             }
+            // what still arrives joins a batch that has just begun
+            const bool opens = eng && !solo && !stop_ && window_ > 0 &&
+                               (eng->active() ? eng->steps() - cohort_start < (uint64_t)window_
+                                              : !take.empty());
+            Young &y = young_[kind];
+            if (opens && (y.free == 0 || y.ei == ei)) {
+              y.ei = ei;
+              y.free = (size_t)std::max(0, eng->free_slots() - (int)take.size());
+            } else if (!opens && y.ei == ei && y.free) {
+              y.free = 0;
+              cv_work_.notify_all();
+            }
           }
         }
         if (release) {
@@ -370,6 +400,9 @@ class ServerImpl : public Server {
           if (!eng->active()) {
             cohort_start = eng->steps();
             batch_t0 = now_us();
+            std::lock_guard<std::mutex> lk(mu_);
+            batches_running_++;
+            batches_begun_++;
           }
           std::vector<uint32_t> srcs;
           for (auto &q : take) srcs.push_back(q.src);
@@ -402,7 +435,9 @@ class ServerImpl : public Server {
           finish(q, GRUS_OK, reached[sl], checksum[sl]);
         }
         if (!eng->active()) {
-          note_time(batch_ms_[kind], (now_us() - batch_t0) / 1e3);
+          std::lock_guard<std::mutex> lk(mu_);
+          batches_running_--;
+          batch_[kind].add((now_us() - batch_t0) / 1e3);
           idle_since = now_us();
         }
       }
@@ -436,6 +471,13 @@ class ServerImpl : public Server {
     Context &ctx = *v.ctx;
     q.start_us = now_us();
     const double t0 = q.start_us;
+    uint64_t begun;
+    bool by_itself;  // no batch beside it
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      begun = batches_begun_;
+      by_itself = batches_running_ == 0;
+    }
     try {
       if (q.kind == GRUS_Q_BFS) run_bfs(v, q.src, GRUS_DIR_AUTO, nullptr);
       else run_sssp(v, q.src, nullptr);
@@ -449,7 +491,18 @@ class ServerImpl : public Server {
       GRUS_HIP(hipMemcpyAsync(q.out, v.result.p, v.V * 4, hipMemcpyDeviceToHost, ctx.stream));
       ctx.sync();
     }
-    note_time(solo_ms_[q.kind], (now_us() - t0) / 1e3);
+    const double ms = (now_us() - t0) / 1e3;
+    {
+      // A query beside a batch takes as long as the batch: means of such
+      // times made batches of 6 queries look worth starting, several side by
+      // side (32 SSSP queries at RMAT s24: 264 ms instead of 134 in one).
+      // They count only until a query has run without one.
+      std::lock_guard<std::mutex> lk(mu_);
+      by_itself = by_itself && begun == batches_begun_;
+      if (by_itself && !solo_known_[q.kind]) solo_[q.kind] = Mean();
+      if (by_itself || !solo_known_[q.kind]) solo_[q.kind].add(ms);
+      solo_known_[q.kind] |= by_itself;
+    }
     finish(q, GRUS_OK, reached, checksum);
     return true;
   }
@@ -459,15 +512,9 @@ class ServerImpl : public Server {
   bool short_queue(int kind) const {
     const size_t n = pending_[kind].size();
     if (n == 0) return false;
-    if (opts_.solo_max > 0 || solo_ms_[kind] <= 0) return (int)n <= solo_max_;
-    if (batch_ms_[kind] <= 0) return n < kLearnBatch;
-    return (double)n * solo_ms_[kind] <= opts_.max_inflight_batches * batch_ms_[kind];
-  }
-
-  // running mean (weight 1/8 to the newest), 0 = nothing measured yet
-  void note_time(double &mean, double ms) {
-    std::lock_guard<std::mutex> lk(mu_);
-    mean = mean > 0 ? mean + (ms - mean) / 8 : ms;
+    if (opts_.solo_max > 0 || !solo_[kind].n) return (int)n <= solo_max_;
+    if (!batch_[kind].n) return n < learn_batch(g_.V);
+    return (double)n * solo_[kind].ms <= opts_.max_inflight_batches * batch_[kind].ms;
   }
 
   void fail(int code, const std::string &msg) {
@@ -496,7 +543,15 @@ class ServerImpl : public Server {
   int window_ = 2;  // steps after an idle start during which a batch admits
   int lanes_ = 64;  // lanes per engine
   int solo_max_ = 8;  // queue length up to which idle engines serve queries alone
-  double solo_ms_[2] = {0, 0}, batch_ms_[2] = {0, 0};  // running means per kind
+  // an engine that still admits to the batch it has begun, and its free slots:
+  // the other engines of the kind leave it that many queries
+  struct Young {
+    size_t ei = 0, free = 0;
+  } young_[2];
+  Mean solo_[2], batch_[2];              // times per kind
+  bool solo_known_[2] = {false, false};  // solo_ holds queries with no batch beside them only
+  int batches_running_ = 0;              // engines with active slots
+  uint64_t batches_begun_ = 0;
   int per_kind_ = 4;        // workers (engines) per kind
   double release_ms_ = -1;  // idle time after which state is given back (< 0: never)
   uint64_t est_[2] = {0, 0};  // state bytes of an engine of each kind

@@ -387,9 +387,9 @@ typedef struct grus_server_opts {
                                  0 = default: while the engines of the kind,
                                  one query each at a time, would empty the
                                  queue within one batch's time (running
-                                 means of both; fewer than 16 waiting until
-                                 a batch has run, at most 8 until a single
-                                 query has run);
+                                 means of both; fewer than 16 waiting, 32
+                                 above 2^20 vertices, until a batch has run,
+                                 at most 8 until a single query has run);
                                  negative = never */
   int idle_release_ms;        /* an engine other than the first of its kind
                                  that has run no query for this long gives
