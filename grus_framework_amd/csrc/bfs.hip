@@ -46,9 +46,6 @@ struct BfsWork {
   Buf cand;  // sparse bottom-up step: the unvisited vertices
   Buf first_in;                     // first in-neighbour of every vertex (GRUS_NO_VERTEX if none)
   const void *first_for = nullptr;  // in-edge columns first_in was built from
-  Buf pad;                          // thin levels: padded rows of a low-degree graph
-  uint32_t pad_deg = 0;             // columns per padded row
-  const void *pad_for = nullptr;    // out-edge columns they were built from
   Buf front2, all_flags;            // whole traversals: third bitmap, barrier flags
   uint32_t all_tag = 0;             // their barrier tags handed out so far
   Buf thin_flags;                   // thin levels: their grid barrier's flags
@@ -594,27 +591,40 @@ constexpr int THIN_T = 256, SOLO_T = 1024;
 constexpr unsigned THIN_BLOCKS = 32;
 constexpr uint64_t THIN_DEG = 16;  // largest maximum degree whose rows are padded
 
-// the padded rows of g, built on first use; null where thin levels do not
-// apply (long rows, edges outside HBM, or a device budget, which the
-// workspace reserve does not count them in)
-const uint4 *thin_rows(Graph &g, BfsWork &w) {
+}  // namespace
+
+// Null where thin levels do not apply (long rows, edges outside HBM, or a
+// device budget, which the workspace reserve does not count the rows in) and
+// where the device lacks the memory: a gigabyte is left for the traversal.
+const void *thin_rows(Graph &g) {
   Context &ctx = *g.ctx;
   if (g.max_deg == 0 || g.max_deg > THIN_DEG || g.placement != GRUS_PLACE_HBM ||
       devmem_budget(ctx.device))
     return nullptr;
-  const CsrView out = g.csr();
-  if (w.pad_for != out.col) {
+  if (!g.pad_tried) {
+    g.pad_tried = true;
     const uint32_t D = g.max_deg <= 4 ? 4 : g.max_deg <= 8 ? 8 : 16;
-    w.pad.alloc(g.V * D * 4);
-    bfs::k_pad_cols<<<grid_cap(ctx, g.V * D, BLOCK), BLOCK, 0, ctx.stream>>>(out, D,
-                                                                           w.pad.as<uint32_t>());
+    size_t free_b = 0, total_b = 0;
+    GRUS_HIP(hipMemGetInfo(&free_b, &total_b));
+    if (free_b < g.V * D * 4 + (1ull << 30)) return nullptr;
+    auto pad = std::make_shared<Buf>();
+    try {
+      pad->alloc(g.V * D * 4);
+    } catch (const Error &e) {
+      if (e.code != GRUS_E_NOMEM && e.code != GRUS_E_BUDGET) throw;
+      return nullptr;
+    }
+    bfs::k_pad_cols<<<grid_cap(ctx, g.V * D, BLOCK), BLOCK, 0, ctx.stream>>>(g.csr(), D,
+                                                                           pad->as<uint32_t>());
     GRUS_LAUNCH_CHECK();
-    w.pad_deg = D;
-    w.pad_for = out.col;
+    ctx.sync();  // (views run on other streams)
+    g.pad = std::move(pad);
+    g.pad_deg = D;
   }
-  return w.pad.as<const uint4>();
+  return g.pad ? g.pad->p : nullptr;
 }
 
+namespace {
 // workgroups of the cooperative thin kernel (0: it may not run here: under a
 // CU mask or beside other contexts its grid might not be resident)
 unsigned thin_grid(const Context &ctx) {
@@ -760,7 +770,8 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
   const double beta = ctx.tuning.bfs_beta > 0 ? ctx.tuning.bfs_beta : 64.0;
   const uint32_t K = ctx.tuning.bu_thread_edges ? ctx.tuning.bu_thread_edges : 32;
 
-  const uint4 *thin = dir == GRUS_DIR_PULL ? nullptr : thin_rows(g, w);
+  const auto *thin =
+      dir == GRUS_DIR_PULL ? nullptr : static_cast<const uint4 *>(thin_rows(g));
   Progress all;
   unsigned all_blocks = dir == GRUS_DIR_AUTO && !thin ? all_grid(g) : 0;
   if (all_blocks && !run_bfs_all(g, w, src, in, first_in, unreach, alpha, beta, K, all_blocks, &all))
@@ -887,7 +898,7 @@ void run_bfs(Graph &g, uint32_t src, int dir, grus_stats *st) {
         auto *tc = reinterpret_cast<bfs::ThinCtl *>(ctx.d_ctl.as<uint64_t>() + 8);
         bfs::ThinParams p{};
         p.pad = thin;
-        p.pad_q = w.pad_deg / 4;
+        p.pad_q = g.pad_deg / 4;
         p.off = out.off;
         p.q0 = w.q[0].as<uint32_t>();
         p.q1 = w.q[1].as<uint32_t>();

@@ -225,6 +225,8 @@ Graph::Graph(Context *c) : ctx(c) {}
 void Graph::make_room(App keep) {
   if (!devmem_budget(ctx->device)) return;  // unbudgeted: keep every cache
   GRUS_HIP(hipStreamSynchronize(ctx->stream));
+  pad.reset();  // (not used under a budget)
+  pad_tried = false;
   if (keep != App::BFS) bfs.reset();
   if (keep != App::SSSP) sssp.reset();
   // SSSP's binned pull rounds run on PageRank's layout (HBM graphs): kept
@@ -555,6 +557,7 @@ std::unique_ptr<Graph> graph_view(Graph &g, Context *ctx) {
   g.csc();          // directed graphs: the in-edges, built once on g
   g.unreachable();  // the in-degree-0 bitmap
   if (g.symmetric && g.placement == GRUS_PLACE_HBM) g.weights_mirror();
+  thin_rows(g);
   auto v = std::make_unique<Graph>(ctx);
   v->V = g.V;
   v->E = g.E;
@@ -583,6 +586,9 @@ std::unique_ptr<Graph> graph_view(Graph &g, Context *ctx) {
   borrow(v->in_col, g.in_col);
   borrow(v->in_w, g.in_w);
   v->csc_ready = g.csc_ready;
+  v->pad = g.pad;
+  v->pad_deg = g.pad_deg;
+  v->pad_tried = g.pad_tried;
   borrow(v->unreachable_bm, g.unreachable_bm);
   v->unreachable_ready = true;
   v->unreachable_count = g.unreachable_count;

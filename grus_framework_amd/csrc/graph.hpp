@@ -167,6 +167,11 @@ struct Graph {
   int mirror = -1;  // weights_mirror(), once it has been found out
   uint64_t unreachable_count = 0;  // vertices with in-degree 0 (set by unreachable())
   uint64_t host_bytes = 0;
+  // padded rows of a low-degree graph (thin_rows(): optional, shared with the
+  // graph's views)
+  std::shared_ptr<Buf> pad;
+  uint32_t pad_deg = 0;    // columns per padded row
+  bool pad_tried = false;  // built, or found not to fit
   // workspaces and last result
   Buf result;
   std::shared_ptr<BfsWork> bfs;
@@ -209,10 +214,13 @@ void csr_from_sorted_keys(Context &ctx, const uint64_t *keys, uint64_t m, uint64
 // (re)place a device-built CSR per the placement request
 void graph_apply_placement(Graph &g, const grus_place *place);
 // A graph that borrows g's arrays (CSR, CSC, first neighbours, in-degree-0
-// bitmap, all built on g first) and runs on ctx with workspaces of its own:
+// bitmap, padded rows, all built on g first) and runs on ctx with workspaces of its own:
 // single-source apps of several threads on one graph, one view each.  g must
 // outlive the view.
 std::unique_ptr<Graph> graph_view(Graph &g, Context *ctx);
+// The padded rows of g (csrc/bfs_thin.hpp), built on first use; null where thin
+// levels do not apply or the rows do not fit.
+const void *thin_rows(Graph &g);
 // Upper bound of the device bytes one app (BFS, SSSP, PageRank pull, CC) on
 // a capped graph of V vertices and E edges allocates beside the graph: its
 // workspace, the result array, control blocks and scan temporaries.
