@@ -608,12 +608,7 @@ const void *thin_rows(Graph &g) {
     GRUS_HIP(hipMemGetInfo(&free_b, &total_b));
     if (free_b < g.V * D * 4 + (1ull << 30)) return nullptr;
     auto pad = std::make_shared<Buf>();
-    try {
-      pad->alloc(g.V * D * 4);
-    } catch (const Error &e) {
-      if (e.code != GRUS_E_NOMEM && e.code != GRUS_E_BUDGET) throw;
-      return nullptr;
-    }
+    if (!pad->try_ensure(g.V * D * 4)) return nullptr;
     bfs::k_pad_cols<<<grid_cap(ctx, g.V * D, BLOCK), BLOCK, 0, ctx.stream>>>(g.csr(), D,
                                                                            pad->as<uint32_t>());
     GRUS_LAUNCH_CHECK();
@@ -656,17 +651,17 @@ struct Progress {
 // a whole traversal in one launch (bfs_all.hpp), or the rest of one (t.level >
 // 0: its frontier in w.front[0]).  t.nf afterwards: 0, or the frontier of the
 // thin levels it was left at, in queue 0.  False when the runtime refuses the
-// launch.
+// launch, or the device's budget the 40 KB that only this needs.
 bool run_bfs_all(Graph &g, BfsWork &w, uint32_t src, const CsrView &in, const uint32_t *first_in,
                  const uint64_t *unreach, double alpha, double beta, uint32_t K, unsigned blocks,
                  Progress *t) {
   Context &ctx = *g.ctx;
   const uint64_t W = g.words();
-  w.front2.ensure((W + 1) * 8);
   constexpr uint64_t NF = 2 * 2 * bfs::ALL_MAX_G;
+  const bool fresh_flags = !w.all_flags.p;
+  if (!w.front2.try_ensure((W + 1) * 8) || !w.all_flags.try_ensure(NF * 8)) return false;
   // a traversal takes at most V + 2 barriers
-  if (!w.all_flags.p || w.all_tag > (1u << 24) - 2 * bfs::ALL_MAX_V) {
-    w.all_flags.ensure(NF * 8);
+  if (fresh_flags || w.all_tag > (1u << 24) - 2 * bfs::ALL_MAX_V) {
     fill_u64(ctx, w.all_flags.as<uint64_t>(), NF, 0);
     w.all_tag = 0;
   }

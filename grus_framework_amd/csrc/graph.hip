@@ -110,6 +110,16 @@ void Buf::alloc(size_t nbytes, Mem k) {
   kind = k;
 }
 
+bool Buf::try_ensure(size_t nbytes) {
+  try {
+    ensure(nbytes);
+    return true;
+  } catch (const Error &e) {
+    if (e.code != GRUS_E_NOMEM && e.code != GRUS_E_BUDGET) throw;
+    return false;
+  }
+}
+
 // ------------------------------------------------------------------ Context
 Context::Context(int dev) {
   int n = 0;

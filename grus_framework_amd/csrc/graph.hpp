@@ -61,6 +61,9 @@ struct Buf {
   void ensure(size_t nbytes, Mem k = Mem::Device) {
     if (nbytes > bytes || kind != k) alloc(nbytes, k);
   }
+  // the same for device memory that the caller can do without: false, and
+  // empty, where the device or its budget has no room
+  bool try_ensure(size_t nbytes);
   void release();
   template <class T>
   T *as() const {

@@ -1411,16 +1411,14 @@ void MsEngine::copy_out(int slot0, int n, uint32_t *host_out) {
     return;
   }
   // as many rows at a time as ROWS_OUT bytes hold, from a buffer kept with
-  // the engine; under a device budget, which has no room for it, one at a time
+  // the engine; one at a time where the device, or a budget, has no room for it
   constexpr uint64_t ROWS_OUT = 64ull << 20;
   uint64_t rows = 1;
   uint32_t *stage = row_.as<uint32_t>();
   if (!devmem_budget(ctx.device) && V) {
     rows = std::min<uint64_t>((uint64_t)n, std::max<uint64_t>(1, ROWS_OUT / (V * 4)));
-    if (rows > 1) {
-      rows_.ensure(rows * V * 4);
-      stage = rows_.as<uint32_t>();
-    }
+    if (rows > 1 && rows_.try_ensure(rows * V * 4)) stage = rows_.as<uint32_t>();
+    else rows = 1;
   }
   for (uint64_t at = 0; at < (uint64_t)n; at += rows) {
     const uint32_t m = (uint32_t)std::min<uint64_t>(rows, (uint64_t)n - at);

@@ -17,7 +17,7 @@ class Ballast:
 
     def __init__(self, leave):
         self.hip, self.held = C.CDLL("libamdhip64.so"), []
-        for size in (64 * GB, 16 * GB, 4 * GB, GB, GB // 4):
+        for size in (64 * GB, 16 * GB, 4 * GB, GB, GB // 4, GB // 16, GB // 64):
             while self.free() > leave + size:
                 p = C.c_void_p()
                 if self.hip.hipMalloc(C.byref(p), C.c_size_t(size)) != 0:

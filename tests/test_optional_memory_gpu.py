@@ -1,0 +1,54 @@
+"""Calls whose workspace is there already run without the buffers that only a
+faster path wants: the third bitmap and the flags of a whole traversal in one
+launch under a device budget, and the staged rows of a batch's results."""
+import numpy as np
+import pytest
+
+import grus_framework_amd as grus
+from test_bfs_rows_memory_gpu import GB, Ballast
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("scale", [9, 14])  # one workgroup and a grid
+def test_whole_traversal_under_a_full_budget(oracle, scale):
+    c = grus.Context(0)
+    try:
+        with grus.Graph.rmat(c, scale) as g:
+            off, col, _ = g.csr()
+            src = g.info.max_degree_vertex
+            want = oracle.bfs(oracle.CSR(off, col, None), src)
+            grus.bfs(g, src, direction="pull")  # the workspace
+            c.set_device_budget(c.device_memory()[0])
+            try:
+                for _ in range(2):
+                    assert (grus.bfs(g, src)[0] == want).all()
+            finally:
+                c.set_device_budget(0)
+            got, st = grus.bfs(g, src)
+            assert (got == want).all() and st.kernel_launches == 1
+    finally:
+        c.close()
+
+
+@pytest.mark.parametrize("wmax", [200, 1 << 20])
+def test_batch_results_without_room_for_staged_rows(oracle, wmax):
+    c = grus.Context(0)
+    try:
+        with grus.Graph.rmat(c, 17, 4, weights=(1, wmax), wseed=2) as g:
+            off, col, w = g.csr()
+            srcs = np.random.default_rng(1).integers(0, g.V, 128)
+            grus.sssp_multi(g, srcs, copy=False)  # the engine
+            ballast = Ballast(GB // 128)
+            try:
+                assert ballast.free() < 4 * g.V * 128
+                got, _ = grus.sssp_multi(g, srcs)
+            finally:
+                ballast.release()
+            again, _ = grus.sssp_multi(g, srcs)
+            assert (got == again).all()
+            h = oracle.CSR(off, col, w)
+            for i in (0, 31, 32, 127):
+                assert (got[i] == oracle.sssp(h, int(srcs[i]))).all()
+    finally:
+        c.close()
