@@ -622,7 +622,7 @@ const void *thin_rows(Graph &g) {
 namespace {
 // workgroups of the cooperative thin kernel (0: it may not run here: under a
 // CU mask or beside other contexts its grid might not be resident)
-unsigned thin_grid(const Context &ctx) {
+unsigned thin_grid(Context &ctx) {
   if (!ctx.cooperative()) return 0;
   int per_cu = 0;
   GRUS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
@@ -632,7 +632,7 @@ unsigned thin_grid(const Context &ctx) {
 }
 // workgroups of a whole traversal in one launch (0: it does not apply)
 unsigned all_grid(const Graph &g) {
-  const Context &ctx = *g.ctx;
+  Context &ctx = *g.ctx;
   const uint64_t W = g.words();
   if (g.V > bfs::ALL_MAX_V || g.placement != GRUS_PLACE_HBM) return 0;
   if (W <= bfs::ALL_OWN) return 1;  // one workgroup needs no grid barrier

@@ -7,6 +7,7 @@
 // reference's host-side serial loops (csr_tocsc, include/graph.cuh:273-303).
 #include <algorithm>
 #include <atomic>
+#include <cstdlib>
 #include <cstring>
 
 #include "device.hpp"
@@ -183,11 +184,14 @@ void Context::set_cu_mask(const uint32_t *mask, uint32_t words) {
 
 bool Context::launch_cooperative(const void *kernel, unsigned blocks, unsigned threads,
                                  void **args, size_t lds) {
-  if (hipLaunchCooperativeKernel(kernel, dim3(blocks), dim3(threads), args, (unsigned)lds,
-                                 stream) == hipSuccess)
-    return true;
+  const hipError_t e =
+      hipLaunchCooperativeKernel(kernel, dim3(blocks), dim3(threads), args, (unsigned)lds, stream);
+  if (e == hipSuccess) return true;
+  if (!coop.refused(e)) GRUS_HIP(e);
   (void)hipGetLastError();
-  coop_refused = true;
+  // GRUS_TRACE=1 prints one line per refusal
+  static const bool trace = getenv("GRUS_TRACE") != nullptr;
+  if (trace) fprintf(stderr, "cooperative launch refused: %s\n", hipGetErrorString(e));
   return false;
 }
 

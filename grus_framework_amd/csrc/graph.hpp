@@ -87,6 +87,28 @@ struct PushWork {
   uint64_t *scan_ptr() const { return scan_ext ? scan_ext : scan.as<uint64_t>(); }
 };
 
+// Whether to ask for cooperative launches.  The runtime refuses them while
+// another process holds the device's one cooperative queue; the traversals
+// have another path, and ask again after some more of them.
+struct CoopGate {
+  static constexpr int WAIT = 64;  // traversals
+  int wait = 0;
+  // once a traversal that could launch one
+  bool open() {
+    if (wait == 0) return true;
+    wait--;
+    return false;
+  }
+  // e, from a launch, says that none are to be had (else it is an error)
+  bool refused(hipError_t e) {
+    if (e != hipErrorIllegalState && e != hipErrorNotSupported &&
+        e != hipErrorCooperativeLaunchTooLarge)
+      return false;
+    wait = WAIT;
+    return true;
+  }
+};
+
 struct Context {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -97,9 +119,7 @@ struct Context {
   // other contexts run kernels on the device at the same time (server
   // workers): no cooperative persistent launches, whose grid must be resident
   bool shared_device = false;
-  // set once the runtime has refused a cooperative launch (another process
-  // may hold the device's one cooperative queue): not asked again
-  bool coop_refused = false;
+  CoopGate coop;
   int wall_khz = 100000;  // device wall clock rate (wall_clock64 ticks per ms)
   grus_tuning tuning{};
   uint64_t *h_ctl = nullptr;  // pinned host mirror of the control block
@@ -115,11 +135,11 @@ struct Context {
   // zeroes them on the device; then wait.  Replaces a copy and the next
   // step's memset (two launches) in per-level read-backs.
   void publish_ctl(size_t n);
-  // whether cooperative grids may be launched: under a CU mask or beside other
-  // contexts' kernels a grid might not be resident
-  bool cooperative() const { return !cu_masked && !shared_device && !coop_refused; }
+  // whether this traversal may launch cooperative grids: under a CU mask or
+  // beside other contexts' kernels a grid might not be resident
+  bool cooperative() { return !cu_masked && !shared_device && coop.open(); }
   // launches a cooperative grid on the stream; false when the runtime refuses
-  // (the caller then takes its other path)
+  // (the caller then takes its other path); any other error is raised
   bool launch_cooperative(const void *kernel, unsigned blocks, unsigned threads, void **args,
                           size_t lds);
   // replace the stream by one restricted to the CUs set in mask (words == 0:
