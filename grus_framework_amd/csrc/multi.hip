@@ -1061,18 +1061,22 @@ void MsEngine::init() {
   push_.tmp = scan_tmp_.p;
   push_.tmp_bytes = tb;
   dirty_ = all_slots();  // state starts uninitialised
-  // SSSP steps that pull need the in-edges and their weights in HBM (a
-  // directed graph's are not built for this alone)
-  if (kind_ == MsKind::SSSP && g.placement == GRUS_PLACE_HBM && g.E &&
-      (g.symmetric ? g.weights_mirror() : g.csc_ready)) {
-    pull_per_ = ms::PULL_EDGES;
-    while (div_up(g.E, (uint64_t)pull_per_) > V) pull_per_ *= 2;  // (longq_ holds the first rows)
-    const uint64_t n = div_up(g.E, (uint64_t)pull_per_);
-    ms::k_pull_first<<<grid_cap(ctx, n, BLOCK), BLOCK, 0, ctx.stream>>>(
-        g.csc().off, V, pull_per_, n, longq_.as<uint32_t>());
-    GRUS_LAUNCH_CHECK();
-  }
+  look_for_in_edges();
   ctx.sync();
+}
+
+void MsEngine::look_for_in_edges() {
+  Graph &g = g_;
+  if (pull_per_ || kind_ != MsKind::SSSP || g.placement != GRUS_PLACE_HBM || !g.E ||
+      !(g.symmetric ? g.weights_mirror() : g.csc_ready))
+    return;
+  ctx_->activate();
+  pull_per_ = ms::PULL_EDGES;
+  while (div_up(g.E, (uint64_t)pull_per_) > g.V) pull_per_ *= 2;  // (longq_ holds the first rows)
+  const uint64_t n = div_up(g.E, (uint64_t)pull_per_);
+  ms::k_pull_first<<<grid_cap(*ctx_, n, BLOCK), BLOCK, 0, ctx_->stream>>>(
+      g.csc().off, g.V, pull_per_, n, longq_.as<uint32_t>());
+  GRUS_LAUNCH_CHECK();
 }
 
 MsEngine::~MsEngine() {
@@ -1252,6 +1256,7 @@ std::vector<int> MsEngine::step() {
     const CsrView in = g_.csc();
     const bool pull = (double)front_edges_ > (double)g_.E / 24.0;
     if (pull) {
+      pulls_++;
       ms::k_bfs_pull<<<grid_cap(ctx, V, BLOCK, 8), BLOCK, 0, ctx.stream>>>(
           in, visit_.as<uint64_t>(), front_.as<uint64_t>(), next_.as<uint64_t>(), run_lanes,
           longq_.as<uint32_t>(), cnt);
@@ -1284,6 +1289,7 @@ std::vector<int> MsEngine::step() {
     // By queries at scale 18, push against pull: 8 (4 lanes) 2.55 and 2.80 ms,
     // 16 3.73 and 2.92, 32 6.29 and 3.04.
     if (pull_per_ && qn_ && front_edges_ > g_.E / 3 && __builtin_popcountll(run_lanes) >= 8) {
+      pulls_++;
       const CsrView in = g_.csc();
       const unsigned grid = (unsigned)div_up(in.E, (uint64_t)pull_per_ * ms::PULL_WAVES);
       const uint32_t *first = longq_.as<uint32_t>();
@@ -1454,6 +1460,8 @@ void run_multi(Graph &g, MsKind kind, const uint32_t *srcs, int k, uint32_t *out
   if (!g.ms || g.ms->kind() != kind) g.ms = std::make_shared<MsEngine>(g, kind, 64, false);
   MsEngine &e = *g.ms;
   Context &ctx = e.ctx();
+  e.look_for_in_edges();
+  const uint64_t pulls = e.pulls();
   for (SlotMask m = e.busy_mask(); m; m &= m - 1) e.release(slot_lowest(m));
   GRUS_HIP(hipEventRecord(ctx.ev0, ctx.stream));
   std::vector<int> slots = e.admit(srcs, k);
@@ -1485,6 +1493,7 @@ void run_multi(Graph &g, MsKind kind, const uint32_t *srcs, int k, uint32_t *out
     *st = grus_stats{};
     st->device_ms = ms;
     st->iterations = (uint32_t)steps;
+    st->pull_iterations = (uint32_t)(e.pulls() - pulls);
     st->vertices_reached = vr;
   }
 }

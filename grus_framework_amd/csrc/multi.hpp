@@ -84,8 +84,13 @@ class MsEngine {
   // the engine's stream, done once the caller has synchronised it
   void copy_out(int slot0, int n, uint32_t *host_out);
   void release(int slot);  // slot becomes free (reset lazily at next admit)
+  // SSSP steps may pull from now on if the graph's in-edges and their weights
+  // are in HBM (a directed graph's are not built for this alone, and another
+  // traversal may have built them since the engine was made)
+  void look_for_in_edges();
   Context &ctx() { return *ctx_; }
   uint64_t steps() const { return t_; }
+  uint64_t pulls() const { return pulls_; }  // of them, the steps over the in-edges
   uint64_t state_bytes() const;
   bool narrow() const { return narrow_; }  // SSSP rows of 16-bit entries
 
@@ -102,6 +107,7 @@ class MsEngine {
   uint32_t src_[128] = {};  // each slot's source (a widened SSSP slot restarts from it)
   bool narrow_ = false;
   uint64_t t_ = 0;         // global step counter
+  uint64_t pulls_ = 0;
   uint64_t qn_ = 0, front_edges_ = 0;
   uint32_t pull_per_ = 0;  // SSSP: in-edges per wave of a pull step; 0: steps only push
   Buf visit_, front_, next_, vals_, queue_, longq_, row_, rows_, digest_, srcs_dev_, cnt_, push_cnt_;
