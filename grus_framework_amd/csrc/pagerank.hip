@@ -1865,11 +1865,10 @@ bool sssp_binned_ready(Graph &g) {
       return false;
     }
   }
-  if (w.bp_sp.edges == 0)
-    build_binned_tasks(g, w, w.bp_sp,
-                       ctx.tuning.pr_task_edges
-                           ? ctx.tuning.pr_task_edges
-                           : automatic_task_edges(g.E, w.bp_nbins, dest_peak(g, w), BP_TASK_SP));
+  const uint64_t te = ctx.tuning.pr_task_edges
+                          ? ctx.tuning.pr_task_edges
+                          : automatic_task_edges(g.E, w.bp_nbins, dest_peak(g, w), BP_TASK_SP);
+  if (w.bp_sp.edges != te) build_binned_tasks(g, w, w.bp_sp, te);
   if (w.bp_w2_for != out.off && !build_binned_weights(g, w)) {
     w.bp_unusable_for = out.off;
     return false;
