@@ -86,7 +86,8 @@ __device__ __forceinline__ void chunk_owners(const uint64_t *S, uint32_t F, uint
                                              uint64_t c1, uint32_t *own) {
   const uint32_t wid = threadIdx.x / WAVE;
   if (wid < 2) {
-    const uint32_t i = wave_upper_bound_u64(S, 0, F + 1, wid ? c1 - 1 : c0) - 1;
+    const uint32_t i =
+        (uint32_t)wave_upper_bound_u64(S, 0, (uint64_t)F + 1, wid ? c1 - 1 : c0) - 1;
     if (lane_id() == 0) own[wid] = i;
   }
   __syncthreads();

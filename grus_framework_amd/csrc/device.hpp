@@ -177,20 +177,38 @@ __device__ __forceinline__ uint64_t readlane_u64(uint64_t x, uint32_t i) {
   return ((uint64_t)hi << 32) | lo;
 }
 
+// One search step of a wave over the indexes [lo, hi): WAVE probes at equal
+// distances.  In 64 bits: a graph may have 2^32 - 1 vertices, and one offset
+// more.
+struct WaveSearch {
+  uint64_t lo, hi;
+  __host__ __device__ uint64_t step() const { return (hi - lo + WAVE - 1) / WAVE; }
+  __host__ __device__ uint64_t probe(uint32_t lane) const { return lo + lane * step(); }
+  // c: the probes below hi that hold at most the key, which are the first ones;
+  // true when lo is the result
+  __host__ __device__ bool advance(uint32_t c) {
+    const uint64_t s = step();
+    if (s <= 1 || c == 0) {
+      lo += c;
+      return true;
+    }
+    const uint64_t end = lo + c * s;
+    lo += (c - 1) * s + 1;
+    if (end < hi) hi = end;
+    return false;
+  }
+};
+
 // First index in [lo, hi) whose entry is above key, or hi, by a whole wave
-// (every lane calls it with the same arguments): 64 probes a step, so a queue of 4096 takes two dependent
-// loads and one of 2^24 four, where one thread's binary search took 12 and 24.
-__device__ __forceinline__ uint32_t wave_upper_bound_u64(const uint64_t *a, uint32_t lo,
-                                                         uint32_t hi, uint64_t key) {
+// (every lane calls it with the same arguments; a is non-decreasing): a queue
+// of 4096 takes two dependent loads and one of 2^24 four, where one thread's
+// binary search took 12 and 24.
+__device__ __forceinline__ uint64_t wave_upper_bound_u64(const uint64_t *a, uint64_t lo,
+                                                         uint64_t hi, uint64_t key) {
+  WaveSearch w{lo, hi};
   for (;;) {
-    const uint32_t step = (hi - lo + WAVE - 1) / WAVE;
-    const uint64_t idx = (uint64_t)lo + (uint64_t)lane_id() * step;
-    // a is non-decreasing, so the probes at most key are the first c lanes
-    const uint32_t c = (uint32_t)__popcll(__ballot(idx < hi && a[idx] <= key));
-    if (step <= 1 || c == 0) return lo + c;
-    const uint64_t end = (uint64_t)lo + (uint64_t)c * step;
-    lo += (c - 1) * step + 1;
-    if (end < hi) hi = (uint32_t)end;
+    const uint64_t i = w.probe(lane_id());
+    if (w.advance((uint32_t)__popcll(__ballot(i < w.hi && a[i] <= key)))) return w.lo;
   }
 }
 
@@ -206,7 +224,7 @@ __device__ __forceinline__ void wave_edge_rows(const uint64_t *off, uint64_t V, 
                                                uint64_t e1, F &&f) {
   if (e0 >= e1) return;
   const uint32_t lane = lane_id();
-  uint64_t r = wave_upper_bound_u64(off, 0, (uint32_t)V + 1, e0) - 1, rb = r;
+  uint64_t r = wave_upper_bound_u64(off, 0, V + 1, e0) - 1, rb = r;
   uint64_t ends = off[rb + 1 + lane < V ? rb + 1 + lane : V];  // of rows rb .. rb + 63
   uint64_t row_beg = off[r];
   for (uint64_t base = e0; base < e1; base += WAVE) {

@@ -373,7 +373,7 @@ __global__ __launch_bounds__(BLOCK) void k_sssp_relax(CsrView g, const uint32_t 
   const uint64_t c0 = wave * per;
   const uint64_t c1 = c0 + per < chunks ? c0 + per : chunks;
   if (c0 < c1) {
-    uint32_t jb = wave_upper_bound_u64(CS, 0, F + 1, c0) - 1;  // owner of c0
+    uint32_t jb = (uint32_t)wave_upper_bound_u64(CS, 0, (uint64_t)F + 1, c0) - 1;  // owner of c0
     uint64_t w_cs = 0, w_off = 0, w_end = 0, w_fm = 0, wend = 0;
     uint32_t w_u = 0;
     auto load_window = [&]() {  // queue entries jb .. jb+63
