@@ -930,28 +930,19 @@ __global__ void k_bp_w2(const uint32_t *wt, uint64_t E, uint64_t Epad, WT *w2) {
   }
 }
 
-// *most = sampled edges whose destination lies in the fullest of PEAK_RANGES
-// equal ranges of the vertices (one workgroup; E > 0)
+// count[r] += sampled edges whose destination lies in the r-th of PEAK_RANGES
+// equal ranges of the vertices (E > 0; PEAK_SAMPLES / PEAK_T workgroups: one
+// alone waits 0.1 ms for its reads)
 constexpr uint32_t PEAK_T = 1024, PEAK_RANGES = 256, PEAK_SAMPLES = 65536;
-__global__ __launch_bounds__(PEAK_T) void k_dest_peak(CsrView g, uint32_t *most) {
-  __shared__ uint32_t s_n[PEAK_RANGES], s_most;
+__global__ __launch_bounds__(PEAK_T) void k_dest_ranges(CsrView g, uint32_t *count) {
+  __shared__ uint32_t s_n[PEAK_RANGES];
   const uint32_t t = threadIdx.x;
   if (t < PEAK_RANGES) s_n[t] = 0;
-  if (t == 0) s_most = 0;
   __syncthreads();
-  constexpr int U = 16;
-  for (uint32_t i0 = t; i0 < PEAK_SAMPLES; i0 += U * PEAK_T) {
-    uint32_t c[U];
-#pragma unroll
-    for (int q = 0; q < U; q++)
-      c[q] = edge_col(g, (uint64_t)(i0 + q * PEAK_T) * g.E / PEAK_SAMPLES);
-#pragma unroll
-    for (int q = 0; q < U; q++) atomicAdd(&s_n[(uint64_t)c[q] * PEAK_RANGES / g.V], 1u);
-  }
+  const uint64_t i = (uint64_t)blockIdx.x * PEAK_T + t;
+  atomicAdd(&s_n[(uint64_t)edge_col(g, i * g.E / PEAK_SAMPLES) * PEAK_RANGES / g.V], 1u);
   __syncthreads();
-  if (t < PEAK_RANGES) atomicMax(&s_most, s_n[t]);
-  __syncthreads();
-  if (t == 0) *most = s_most;
+  if (t < PEAK_RANGES && s_n[t]) atomicAdd(&count[t], s_n[t]);
 }
 
 __global__ void k_max_u32(const uint32_t *a, uint64_t n, uint32_t *out) {
@@ -1434,11 +1425,15 @@ double dest_peak(Graph &g, PrWork &w) {
   if (out.E == 0) return 1;
   if (w.peak_for != out.off) {
     Context &ctx = *g.ctx;
-    pr::k_dest_peak<<<1, pr::PEAK_T, 0, ctx.stream>>>(
-        out, reinterpret_cast<uint32_t *>(ctx.d_ctl.as<uint64_t>() + 33));
+    constexpr uint32_t at = 384;  // the last words of the control block
+    static_assert(at * 8 + pr::PEAK_RANGES * 4 <= 4096, "the counts fit it");
+    auto *count = reinterpret_cast<uint32_t *>(ctx.d_ctl.as<uint64_t>() + at);
+    fill_u32(ctx, count, pr::PEAK_RANGES, 0);
+    pr::k_dest_ranges<<<pr::PEAK_SAMPLES / pr::PEAK_T, pr::PEAK_T, 0, ctx.stream>>>(out, count);
     GRUS_LAUNCH_CHECK();
-    ctx.read_ctl(34);
-    w.peak = (double)(uint32_t)ctx.h_ctl[33] * pr::PEAK_RANGES / pr::PEAK_SAMPLES;
+    ctx.read_ctl(512);
+    const auto *h = reinterpret_cast<const uint32_t *>(ctx.h_ctl + at);
+    w.peak = (double)*std::max_element(h, h + pr::PEAK_RANGES) * pr::PEAK_RANGES / pr::PEAK_SAMPLES;
     w.peak_for = out.off;
   }
   return w.peak;
