@@ -930,9 +930,10 @@ __global__ void k_bp_w2(const uint32_t *wt, uint64_t E, uint64_t Epad, WT *w2) {
   }
 }
 
-// count[r] += sampled edges whose destination lies in the r-th of PEAK_RANGES
-// equal ranges of the vertices (E > 0; PEAK_SAMPLES / PEAK_T workgroups: one
-// alone waits 0.1 ms for its reads)
+// count[r] += pseudo-random edges whose destination lies in the r-th of
+// PEAK_RANGES equal ranges of the vertices (E > 0; PEAK_SAMPLES / PEAK_T
+// workgroups: one alone waits 0.1 ms for its reads).  At equal distances the
+// samples of a regular graph were all first edges of rows, which ascend.
 constexpr uint32_t PEAK_T = 1024, PEAK_RANGES = 256, PEAK_SAMPLES = 65536;
 __global__ __launch_bounds__(PEAK_T) void k_dest_ranges(CsrView g, uint32_t *count) {
   __shared__ uint32_t s_n[PEAK_RANGES];
@@ -940,7 +941,7 @@ __global__ __launch_bounds__(PEAK_T) void k_dest_ranges(CsrView g, uint32_t *cou
   if (t < PEAK_RANGES) s_n[t] = 0;
   __syncthreads();
   const uint64_t i = (uint64_t)blockIdx.x * PEAK_T + t;
-  atomicAdd(&s_n[(uint64_t)edge_col(g, i * g.E / PEAK_SAMPLES) * PEAK_RANGES / g.V], 1u);
+  atomicAdd(&s_n[(uint64_t)edge_col(g, mix64(i) % g.E) * PEAK_RANGES / g.V], 1u);
   __syncthreads();
   if (t < PEAK_RANGES && s_n[t]) atomicAdd(&count[t], s_n[t]);
 }
@@ -1419,7 +1420,7 @@ uint64_t automatic_task_edges(uint64_t E, uint32_t nbins, double peak, uint64_t 
 }
 
 // the densest of PEAK_RANGES equal ranges of destinations, in multiples of its
-// share, by PEAK_SAMPLES edges at equal distances; found out once
+// share, by PEAK_SAMPLES edges; found out once
 double dest_peak(Graph &g, PrWork &w) {
   const CsrView out = g.csr();
   if (out.E == 0) return 1;
