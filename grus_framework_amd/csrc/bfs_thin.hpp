@@ -13,7 +13,7 @@
 // vertex a thread expands next is requested before the barrier (grid 1300 x
 // 1700: 3.9 -> 3.1 us a level, with the barrier polled by a wave of its own).
 // Per call, launched level by level / thin: grid 64 x 64 1.1 / 0.2 ms, 300 x
-// 300 3.2 / 1.1 ms, 1300 x 1700 51 / 9 ms, 4096 x 4096 268 / 28 ms.  A workgroup keeps
+// 300 3.2 / 1.1 ms, 1300 x 1700 51 / 7.5 ms, 4096 x 4096 268 / 28 ms.  A workgroup keeps
 // the vertices it discovers in LDS and expands them itself in the next level;
 // what exceeds its share goes to the global queue, which the next level deals
 // round-robin over all workgroups.

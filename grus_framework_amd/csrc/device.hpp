@@ -104,13 +104,13 @@ __device__ __forceinline__ T wave_sum(T x) {
 // Adds every thread's two numbers up, with one atomic pair per workgroup
 // (skipped where zero).  Every thread of the workgroup must call it, at the
 // end of the kernel; blockDim.x <= 1024.  The sums go into the context's
-// control block, to 32 cache lines by turns, and publish_ctl puts them
-// together: atomics on one line run one after the other, 12 ns each, and the
-// workgroups of a launch end together (RMAT scale 20, digest of 1 M entries: 2048 workgroups 52 us, 256 of
-// them 9).  `field` is the first of two words of a line: CTL_STEP for
-// StepCounters' next_count and next_edges, CTL_REACHED for words 40 and 41,
-// CTL_DIGEST for words 48 and 49.
-constexpr uint32_t CTL_SPREAD = 128;  // first word; 8 words a line
+// control block, to 32 slots of 64 bytes by turns (16 cache lines), and
+// publish_ctl puts them together: atomics on one line run one after the other,
+// 12 ns each, and the workgroups of a launch end together (RMAT scale 20,
+// digest of 1 M entries: 2048 workgroups 52 us, 256 of them 9).  `field` is
+// the first of two words of a slot: CTL_STEP for StepCounters' next_count and
+// next_edges, CTL_REACHED for words 40 and 41, CTL_DIGEST for words 48 and 49.
+constexpr uint32_t CTL_SPREAD = 128;  // first word; 8 words a slot
 constexpr uint32_t CTL_LINES = 32;
 constexpr uint32_t CTL_STEP = 0, CTL_REACHED = 2, CTL_DIGEST = 4;
 __device__ __forceinline__ void block_add_spread(unsigned long long a, unsigned long long b,
