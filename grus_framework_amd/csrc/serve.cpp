@@ -297,7 +297,7 @@ class ServerImpl : public Server {
     const bool first = (int)ei % per_kind_ == 0;  // holds its state throughout
     std::vector<Query> slot_q(128);
     uint64_t cohort_start = 0;  // engine step at which the running batch started
-    double batch_t0 = 0;        // and its clock
+    double batch_us = 0;        // the longest of its queries
     double idle_since = now_us();
     uint64_t refused_at = ~0ull;  // memory epoch of the last refusal
     try {
@@ -399,7 +399,7 @@ class ServerImpl : public Server {
         if (!take.empty()) {
           if (!eng->active()) {
             cohort_start = eng->steps();
-            batch_t0 = now_us();
+            batch_us = 0;
             std::lock_guard<std::mutex> lk(mu_);
             batches_running_++;
             batches_begun_++;
@@ -431,13 +431,18 @@ class ServerImpl : public Server {
         for (SlotMask m = done; m; m &= m - 1) {
           const int sl = slot_lowest(m);
           const Query &q = slot_q[sl];
+          batch_us = std::max(batch_us, now_us() - q.start_us);
           eng->release(sl);
           finish(q, GRUS_OK, reached[sl], checksum[sl]);
         }
         if (!eng->active()) {
           std::lock_guard<std::mutex> lk(mu_);
           batches_running_--;
-          batch_[kind].add((now_us() - batch_t0) / 1e3);
+          // (not the batch's own length: one that keeps admitting may never
+          // end, and next to it every queue looked short enough to serve
+          // alone: s21, a window of 1000 steps, 600 SSSP queries with 128
+          // outstanding 374 ms alone, 179 in batches)
+          batch_[kind].add(batch_us / 1e3);
           idle_since = now_us();
         }
       }
