@@ -55,6 +55,7 @@
 #include "apps.hpp"
 #include "multi.hpp"
 #include "serve.hpp"
+#include "serve_time.hpp"
 
 namespace mgg {
 
@@ -76,18 +77,6 @@ double now_us() {
 // ms, s20 1.4 / 2.4 and 10.1 / 8.6, s22 5.8 / 4.1 and 33 / 30, s24 14.9 / 10.4
 // and 137 / 111; 32 of them at s24 13.5 / 15.6 and 134 / 156.
 size_t learn_batch(uint64_t V) { return V <= (1ull << 20) ? 16 : 32; }
-
-// Running mean: plain up to 8 values, then weight 1/8 to the newest.  (The
-// first query of a worker makes its workspace: with 1/8 from the second value
-// on, its time stood for the others' for dozens of queries.)  0: none yet.
-struct Mean {
-  double ms = 0;
-  int n = 0;
-  void add(double x) {
-    n = std::min(n + 1, 8);
-    ms += (x - ms) / n;
-  }
-};
 
 struct Query {
   uint64_t id;
@@ -156,6 +145,7 @@ class ServerImpl : public Server {
     }
     engines_.resize(n);
     state_.assign(n, 0);
+    served_.assign(n, 0);
     // the first engine of each kind holds its state from the start; with
     // memory uncapped every engine does (nothing to admit by, and no
     // allocation in a worker thread while the others launch)
@@ -255,6 +245,7 @@ class ServerImpl : public Server {
         return false;
       }
       reserved_ += est;
+      slow_.begin();
     }
     std::unique_ptr<MsEngine> e;
     try {
@@ -262,12 +253,14 @@ class ServerImpl : public Server {
     } catch (const Error &x) {
       std::lock_guard<std::mutex> lk(mu_);
       reserved_ -= est;
+      slow_.end();
       if (x.code != GRUS_E_BUDGET && x.code != GRUS_E_NOMEM) throw;
       memory_waits_++;
       return false;
     }
     std::lock_guard<std::mutex> lk(mu_);
     reserved_ -= est;
+    slow_.end();
     state_[i] = e->state_bytes();
     if (!est_[kind]) est_[kind] = state_[i];
     engines_[i] = std::move(e);
@@ -401,8 +394,7 @@ class ServerImpl : public Server {
             cohort_start = eng->steps();
             batch_us = 0;
             std::lock_guard<std::mutex> lk(mu_);
-            batches_running_++;
-            batches_begun_++;
+            slow_.begin();
           }
           std::vector<uint32_t> srcs;
           for (auto &q : take) srcs.push_back(q.src);
@@ -437,7 +429,7 @@ class ServerImpl : public Server {
         }
         if (!eng->active()) {
           std::lock_guard<std::mutex> lk(mu_);
-          batches_running_--;
+          slow_.end();
           // (not the batch's own length: one that keeps admitting may never
           // end, and next to it every queue looked short enough to serve
           // alone: s21, a window of 1000 steps, 600 SSSP queries with 128
@@ -476,37 +468,42 @@ class ServerImpl : public Server {
     Context &ctx = *v.ctx;
     q.start_us = now_us();
     const double t0 = q.start_us;
-    uint64_t begun;
-    bool by_itself;  // no batch beside it
+    // the worker's first query makes its workspace, which may take hundreds of
+    // milliseconds and holds up the others' launches: of it, the device time
+    const bool first = !served_[ei];
+    uint64_t mark;
     {
       std::lock_guard<std::mutex> lk(mu_);
-      begun = batches_begun_;
-      by_itself = batches_running_ == 0;
+      if (first) slow_.begin();
+      mark = slow_.mark();
     }
+    auto settled = [&] {
+      std::lock_guard<std::mutex> lk(mu_);
+      if (first) slow_.end();
+    };
+    grus_stats st{};
     try {
-      if (q.kind == GRUS_Q_BFS) run_bfs(v, q.src, GRUS_DIR_AUTO, nullptr);
-      else run_sssp(v, q.src, nullptr);
+      if (q.kind == GRUS_Q_BFS) run_bfs(v, q.src, GRUS_DIR_AUTO, first ? &st : nullptr);
+      else run_sssp(v, q.src, first ? &st : nullptr);
     } catch (const Error &e) {
+      settled();
       if (e.code != GRUS_E_BUDGET && e.code != GRUS_E_NOMEM) throw;
       return false;
     }
+    served_[ei] = 1;
+    settled();
+    const double ran = now_us();
     uint64_t reached = 0, checksum = 0;
     row_digest(ctx, v.result.as<uint32_t>(), v.V, &reached, &checksum);
     if (opts_.copy_results && q.out) {
       GRUS_HIP(hipMemcpyAsync(q.out, v.result.p, v.V * 4, hipMemcpyDeviceToHost, ctx.stream));
       ctx.sync();
     }
-    const double ms = (now_us() - t0) / 1e3;
+    const double end = now_us();
     {
-      // A query beside a batch takes as long as the batch: means of such
-      // times made batches of 6 queries look worth starting, several side by
-      // side (32 SSSP queries at RMAT s24: 264 ms instead of 134 in one).
-      // They count only until a query has run without one.
       std::lock_guard<std::mutex> lk(mu_);
-      by_itself = by_itself && begun == batches_begun_;
-      if (by_itself && !solo_known_[q.kind]) solo_[q.kind] = Mean();
-      if (by_itself || !solo_known_[q.kind]) solo_[q.kind].add(ms);
-      solo_known_[q.kind] |= by_itself;
+      solo_[q.kind].add(first ? st.device_ms + (end - ran) / 1e3 : (end - t0) / 1e3,
+                        !slow_.quiet_since(mark));
     }
     finish(q, GRUS_OK, reached, checksum);
     return true;
@@ -517,9 +514,9 @@ class ServerImpl : public Server {
   bool short_queue(int kind) const {
     const size_t n = pending_[kind].size();
     if (n == 0) return false;
-    if (opts_.solo_max > 0 || !solo_[kind].n) return (int)n <= solo_max_;
+    if (opts_.solo_max > 0 || !solo_[kind].mean.n) return (int)n <= solo_max_;
     if (!batch_[kind].n) return n < learn_batch(g_.V);
-    return (double)n * solo_[kind].ms <= opts_.max_inflight_batches * batch_[kind].ms;
+    return (double)n * solo_[kind].mean.ms <= opts_.max_inflight_batches * batch_[kind].ms;
   }
 
   void fail(int code, const std::string &msg) {
@@ -553,10 +550,10 @@ class ServerImpl : public Server {
   struct Young {
     size_t ei = 0, free = 0;
   } young_[2];
-  Mean solo_[2], batch_[2];              // times per kind
-  bool solo_known_[2] = {false, false};  // solo_ holds queries with no batch beside them only
-  int batches_running_ = 0;              // engines with active slots
-  uint64_t batches_begun_ = 0;
+  SoloTime solo_[2];  // times per kind
+  Mean batch_[2];
+  Slow slow_;  // batches, engines being made, workers' first queries
+  std::vector<char> served_;  // per worker: whether it has served a query alone (its own)
   int per_kind_ = 4;        // workers (engines) per kind
   double release_ms_ = -1;  // idle time after which state is given back (< 0: never)
   uint64_t est_[2] = {0, 0};  // state bytes of an engine of each kind
