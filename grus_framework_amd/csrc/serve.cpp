@@ -16,15 +16,15 @@
 // the single-source kernels on its own view of the graph: a batch costs a
 // step per level whatever it holds.  Load is light while the engines of a
 // kind, each serving one query at a time, would empty the queue within the
-// time of one batch (running means of both times, per kind; until a batch
-// has run, 16 waiting queries, 32 above 2^20 vertices, start one, so that its
-// time is known), or while at most solo_max queries wait when the caller sets
-// it.  A burst still arrives when its first queries start a batch; the rest
-// joins that one, and no engine beside it takes a few (bursts of 64 SSSP
-// queries at RMAT s24: mean of 24 of them 190 -> 151 ms).  Measured on RMAT scale 22 at 1100 queries/s (50/50
-// BFS/SSSP): p50 5 ms when every query is served alone, 99-120 ms when a
-// queue of 8 already starts a batch (which then slows the single queries
-// beside it).
+// time of one batch (running means of both times, per kind, see
+// serve_time.hpp; until a batch has run, 16 waiting queries, 32 above 2^20
+// vertices, start one, so that its time is known), or while at most solo_max
+// queries wait when the caller sets it.  A burst still arrives when its first
+// queries start a batch; the rest joins that one, and no engine beside it
+// takes a few (bursts of 64 SSSP queries at RMAT s24: mean of 24 of them 190
+// -> 151 ms).  Measured on RMAT scale 22 at 1100 queries/s (50/50 BFS/SSSP):
+// p50 5 ms when every query is served alone, 99-120 ms when a queue of 8
+// already starts a batch (which then slows the single queries beside it).
 //
 // Memory.  Each worker owns a context (stream).  When memory is capped
 // (state_budget_bytes or a device budget), its engine's device state (the
